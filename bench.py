@@ -869,7 +869,7 @@ def main():
     roofline = {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                 "frac": achieved / PEAK_FP32_TFLOPS,
                 "traffic": (tpf * fits_per_launch) if tpf is not None else None,
-                "kernel": "fit_1e_kernel<GS2D,7>", "flop_per_launch": FLOP_PER_FIT_7X7 * fits_per_launch,
+                "kernel": "fit_split_kernel<GS2D,7,1>", "flop_per_launch": FLOP_PER_FIT_7X7 * fits_per_launch,
                 "avg_launch_ms": fit_avg_ms}
 
     n_last = fits // max(args.steps, 1)

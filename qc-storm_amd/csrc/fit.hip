@@ -1,78 +1,12 @@
-// fit.hip -- BFGS Poisson-MLE Gaussian fitting and CRLB kernels for gfx950.
+// fit.hip -- host side of the reference-schedule fits (dispatch by ROI size and count, the
+// multi-emitter cascade) and the CRLB kernel for gfx950.  The fitting kernels are in fit_split.h.
 //
-// One ROI per lane of a wave64.  The ROI's photo-electron pixels q and log q live in VGPRs for the
-// whole fit; the Gaussian model is evaluated separably (one exp per ROI row and column), so a
-// pixel evaluation of the loss costs one FMA for the model, one log and three FMAs for the
-// weighted Poisson deviance.  The reference's fixed schedule (gradient, 2 + 10 line-search
-// evaluations, gradient, BFGS update; DLL/bfgsMLE_Loc_LD/bfgsMLE_GS2D_core.h:313-426) is run as a
-// uniform state machine over its loss evaluations, so the loss body is emitted once and every
-// lane of the wave executes the same instruction stream (no divergence: the schedule does not
-// depend on the data; the line-search side each lane updates is a per-lane select).
-//
-// Reference kernels (DLL = MLEbfgs/bfgs_MLE_dll x64/bfgsMLE_dll/bfgsMLE_dll):
-//   bfgsMLELoc_Gauss2D   DLL/bfgsMLE_Loc_LD/bfgsMLE_GS2D_core.h:56-310
-//   bfgsMLELoc_AS3D      DLL/bfgsMLE_Loc_LD/bfgsMLE_AS3D_core.h:57-337
+// Reference (DLL = MLEbfgs/bfgs_MLE_dll x64/bfgsMLE_dll/bfgsMLE_dll):
 //   GaussianCRLB_Calc_top DLL/bfgsMLE_Loc_top/LocPrecCalc_GaussianCRLB.h:64-243
-#include "qcs_internal.h"
-#include "qcs_devmath.h"
+//   BFGS_MLELocalization  DLL/bfgsMLE_Loc_top/bfgs_top.cu:26-204
+#include "fit_dev.h"
 
 namespace qcs {
-
-enum { MODEL_GS2D = 0, MODEL_AS3D = 1, MODEL_2E = 2, MODEL_3E = 3, MODEL_AS3D2E = 4 };
-
-// Parameter layout of each model: amplitude / x / y / sigma_x / sigma_y index of emitter k,
-// background index, iteration count, loss clamp, WLE weighting.
-template <int MODEL> struct Traits;
-template <> struct Traits<MODEL_GS2D> {   // bfgsMLE_GS2D_core.h:25-37
-    static constexpr int P = 5, ITERS = 8, K = 1, IB = 4;
-    static constexpr bool WEIGHTED = true;
-    static constexpr float CLAMP = 0.0f;
-    __device__ static constexpr int ia(int) { return 0; }
-    __device__ static constexpr int ix(int) { return 1; }
-    __device__ static constexpr int iy(int) { return 2; }
-    __device__ static constexpr int isx(int) { return 3; }
-    __device__ static constexpr int isy(int) { return 3; }
-};
-template <> struct Traits<MODEL_AS3D> {   // bfgsMLE_AS3D_core.h:25-38, loss clamp :501-505
-    static constexpr int P = 6, ITERS = 11, K = 1, IB = 5;
-    static constexpr bool WEIGHTED = true;
-    static constexpr float CLAMP = 0.01f;
-    __device__ static constexpr int ia(int) { return 0; }
-    __device__ static constexpr int ix(int) { return 1; }
-    __device__ static constexpr int iy(int) { return 2; }
-    __device__ static constexpr int isx(int) { return 3; }
-    __device__ static constexpr int isy(int) { return 4; }
-};
-template <> struct Traits<MODEL_2E> {     // bfgsMLE_GS2D_2Emitter_core.h:24-51
-    static constexpr int P = 8, ITERS = 13, K = 2, IB = 7;
-    static constexpr bool WEIGHTED = true;
-    static constexpr float CLAMP = 0.0f;
-    __device__ static constexpr int ia(int k) { return 3 * k; }
-    __device__ static constexpr int ix(int k) { return 3 * k + 1; }
-    __device__ static constexpr int iy(int k) { return 3 * k + 2; }
-    __device__ static constexpr int isx(int) { return 6; }
-    __device__ static constexpr int isy(int) { return 6; }
-};
-template <> struct Traits<MODEL_3E> {     // bfgsMLE_GS2D_3Emitter_core.h:24-54 (unweighted)
-    static constexpr int P = 11, ITERS = 16, K = 3, IB = 10;
-    static constexpr bool WEIGHTED = false;
-    static constexpr float CLAMP = 0.0f;
-    __device__ static constexpr int ia(int k) { return 3 * k; }
-    __device__ static constexpr int ix(int k) { return 3 * k + 1; }
-    __device__ static constexpr int iy(int k) { return 3 * k + 2; }
-    __device__ static constexpr int isx(int) { return 9; }
-    __device__ static constexpr int isy(int) { return 9; }
-};
-template <> struct Traits<MODEL_AS3D2E> { // bfgsMLE_AS3D_2Emitter_core.h:24-54 (unweighted), clamp :590-594
-    static constexpr int P = 11, ITERS = 16, K = 2, IB = 10;
-    static constexpr bool WEIGHTED = false;
-    static constexpr float CLAMP = 0.01f;
-    __device__ static constexpr int ia(int k) { return 5 * k; }
-    __device__ static constexpr int ix(int k) { return 5 * k + 1; }
-    __device__ static constexpr int iy(int k) { return 5 * k + 2; }
-    __device__ static constexpr int isx(int k) { return 5 * k + 3; }
-    __device__ static constexpr int isy(int k) { return 5 * k + 4; }
-};
 
 FitConst make_fit_const(const qcs_params &p)
 {
@@ -83,474 +17,6 @@ FitConst make_fit_const(const qcs_params &p)
     c.pL[0] = p.p4_XLY; c.pL[1] = p.p3_XLY; c.pL[2] = p.p2_XLY; c.pL[3] = p.p1_XLY; c.pL[4] = p.p0_XLY;
     return c;
 }
-
-// ---------------------------------------------------------------------------------------------
-// Weighted Poisson deviance, model I = sum_k A_k exp(-(sx_k dx^2 + sy_k dy^2)) + B evaluated
-// separably (one exp per emitter and ROI row / column).  Clamps p in place as the reference's
-// loss does with its argument array.  The pixel term is w (I - q - q (log I - log q)), formed as
-// fma(-q, log I + c, I) with c = 1 - log q precomputed per ROI and the log fused with c
-// (logtab_u); the weighted sum runs as sum_r wy[r] sum_c wx[c] t(r, c).
-//
-// The range check bounds every model value before the pixel loop: with positions below 2^60 in
-// magnitude and finite widths each exp term lies in [0, 1], so I lies in [B, sum of the
-// amplitudes + B].  Multi-emitter models need B in [2^-126, 2^124] and amplitudes at most 2^124
-// (I a positive normal float); the one-emitter models use the binade table log and need B and A
-// within [2^-10.5, 2^18.5] so that I stays inside the table.  A lane that fails it (a line-search
-// probe gone far out, a background at zero) takes the _any form of the log, whose range and
-// special-value handling gives the value the CPU oracle computes.
-template <int MODEL, int R, bool FAST, bool SAFE>
-__device__ __forceinline__ float pixel_sum(const float (&q)[R * R], const float (&c1)[R * R], const float (&wx)[R],
-                                           const float (&wy)[R], const float (&ex)[Traits<MODEL>::K][R],
-                                           const float (&ay)[Traits<MODEL>::K][R], float b, const float2 *lt)
-{
-    using T = Traits<MODEL>;
-    constexpr int K = T::K;
-    float total = 0.0f;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int c = 0; c < R; c++) {
-            float I;
-            if (K == 1) {
-                I = __builtin_fmaf(ay[0][r], ex[0][c], b);
-            } else {
-                I = ay[0][r] * ex[0][c];
-#pragma unroll
-                for (int k = 1; k < K; k++) I = __builtin_fmaf(ay[k][r], ex[k][c], I);
-                I = I + b;
-            }
-            const float cc = c1[r * R + c];
-            float u;
-            if (FAST) u = flogf(I) + cc;
-            else if (K == 1) u = SAFE ? logtabb_u_any(I, cc, lt) : logtabb_u(I, cc, lt);
-            else u = SAFE ? logtab_u_any(I, cc, lt) : logtab_u(I, cc, lt);
-            const float t = __builtin_fmaf(-q[r * R + c], u, I);
-            acc = T::WEIGHTED ? __builtin_fmaf(wx[c], t, acc) : acc + t;
-        }
-        total = T::WEIGHTED ? __builtin_fmaf(wy[r], acc, total) : total + acc;
-    }
-    return total;
-}
-
-template <int MODEL, int R, bool FAST>
-__device__ __forceinline__ float loss_eval(const float (&q)[R * R], const float (&c1)[R * R], const float (&wx)[R],
-                                          const float (&wy)[R], float (&p)[Traits<MODEL>::P], const float2 *lt)
-{
-    using T = Traits<MODEL>;
-    constexpr int P = T::P, K = T::K;
-#pragma unroll
-    for (int i = 0; i < P; i++) p[i] = (p[i] < T::CLAMP) ? T::CLAMP : p[i];
-    const float b = p[T::IB] * 64.0f;
-    // one-emitter models: every model value inside the binade table, I in [b, a + b]
-    constexpr float BLO = (K == 1) ? kLogTabBLo : 1.17549435082228751e-38f;
-    constexpr float AHI = (K == 1) ? kLogTabBHi * 0.125f : 0x1p124f;
-    bool inrange = (b >= BLO) && (b <= AHI);
-    float ex[K][R], ay[K][R];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const float a = p[T::ia(k)] * 128.0f;
-        const float sx = p[T::isx(k)] * 0.1f;
-        const float sy = p[T::isy(k)] * 0.1f;
-        inrange = inrange && (a <= AHI) && (sx <= 0x1p124f) && (sy <= 0x1p124f) &&
-                  (__builtin_fabsf(p[T::ix(k)]) <= 0x1p60f) && (__builtin_fabsf(p[T::iy(k)]) <= 0x1p60f);
-#pragma unroll
-        for (int c = 0; c < R; c++) {
-            const float dx = ((float)c + 0.5f) - p[T::ix(k)];
-            ex[k][c] = vexp_nonpos<FAST>((-(dx * dx)) * sx);
-        }
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const float dy = ((float)r + 0.5f) - p[T::iy(k)];
-            ay[k][r] = a * vexp_nonpos<FAST>((-(dy * dy)) * sy);
-        }
-    }
-    if (FAST || inrange) return pixel_sum<MODEL, R, FAST, false>(q, c1, wx, wy, ex, ay, b, lt);
-    return pixel_sum<MODEL, R, FAST, true>(q, c1, wx, wy, ex, ay, b, lt);
-}
-
-// ConstructD0 (bfgsMLE_core.h:87-182).  D is the lane's inverse-Hessian approximation, stored in
-// LDS with element k at D[k * 64] (lane-interleaved: conflict-free, off the VGPR budget).
-template <int P>
-__device__ __forceinline__ void bfgs_update(float *D, const float (&s)[P], const float (&y)[P])
-{
-    float sy = 0.0f;
-#pragma unroll
-    for (int k = 0; k < P; k++) sy = __builtin_fmaf(s[k], y[k], sy);
-    sy = 1.0f / sy;
-    float ty[P], ts[P];
-#pragma unroll
-    for (int k = 0; k < P; k++) { ty[k] = y[k] * sy; ts[k] = s[k] * sy; }
-    float A[P * P], T[P * P];
-#pragma unroll
-    for (int r = 0; r < P; r++)
-#pragma unroll
-        for (int c = 0; c < P; c++) A[r * P + c] = __builtin_fmaf(-s[r], ty[c], (r == c) ? 1.0f : 0.0f);
-#pragma unroll
-    for (int c = 0; c < P; c++) {
-        float Dc[P];
-#pragma unroll
-        for (int k = 0; k < P; k++) Dc[k] = D[(k * P + c) * 64];
-#pragma unroll
-        for (int r = 0; r < P; r++) {
-            float acc = 0.0f;
-#pragma unroll
-            for (int k = 0; k < P; k++) acc = __builtin_fmaf(A[r * P + k], Dc[k], acc);
-            T[r * P + c] = acc;
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < P; r++)
-#pragma unroll
-        for (int c = 0; c < P; c++) {
-            float acc = 0.0f;
-#pragma unroll
-            for (int k = 0; k < P; k++) acc = __builtin_fmaf(T[r * P + k], A[c * P + k], acc);
-            D[(r * P + c) * 64] = acc + s[r] * ts[c];
-        }
-}
-
-template <int P>
-__device__ __forceinline__ void normalize_dir(float (&d)[P])
-{
-    float tot = 0.0f;
-#pragma unroll
-    for (int k = 0; k < P; k++) tot = tot + __builtin_fabsf(d[k]);
-    tot = (float)P / tot;
-#pragma unroll
-    for (int k = 0; k < P; k++) d[k] = d[k] * tot;
-}
-
-enum { PH_G0 = 0, PH_G1 = 1, PH_L0 = 2, PH_L1 = 3, PH_BS = 4 };
-
-// Fixed-schedule BFGS (MLELocalization_GS2D, bfgsMLE_GS2D_core.h:313-426, with the gradient of
-// NumericalGradient_GS2D :429-454).  x holds the initial vector on entry, the result on exit.
-// Schedule: gradient (2P evaluations); per iteration: probes at 1e-4 and 1, ten bisection
-// evaluations (eleven halvings of [1e-5, 1]), step, clamp >= 0.01, and -- except after the
-// last iteration -- gradient, BFGS update and new direction.
-template <int MODEL, int R, bool FAST>
-__device__ __forceinline__ void bfgs_fit(const float (&q)[R * R], const float (&c1)[R * R], const float (&wx)[R],
-                                            const float (&wy)[R], float (&x)[Traits<MODEL>::P], float *cold,
-                                            const float2 *lt)
-{
-    constexpr int P = Traits<MODEL>::P, IT = Traits<MODEL>::ITERS;
-    constexpr int NEVAL = 2 * P + IT * 12 + (IT - 1) * 2 * P;
-    // cold state in LDS (element k at cold[k * 64]): D (P*P), previous gradient (P), step (P)
-    float *D = cold, *gprev_l = cold + P * P * 64, *s_l = cold + (P * P + P) * 64;
-    float g[P], d[P], t[P];
-#pragma unroll
-    for (int r = 0; r < P; r++)
-#pragma unroll
-        for (int c = 0; c < P; c++) D[(r * P + c) * 64] = (r == c) ? 1.0f : 0.0f;
-#pragma unroll
-    for (int k = 0; k < P; k++) { t[k] = x[k]; g[k] = 0.0f; d[k] = 0.0f; }
-    float L0 = 0.0f, L1 = 0.0f, lo = 0.0f, hi = 0.0f, ln = 0.0f;
-    bool sel = false;
-    int phase = PH_G0, gi = 0, bsn = 0;
-    bool first = true;
-
-    for (int e = 0; e < NEVAL; e++) {
-        float pr[P];
-        if (phase <= PH_G1) {
-            const float delta = (phase == PH_G0) ? -0.002f : 0.004f;
-#pragma unroll
-            for (int k = 0; k < P; k++) {
-                if (k == gi) t[k] = t[k] + delta;
-                pr[k] = t[k];
-            }
-        } else {
-            float step = (phase == PH_L0) ? 0.0001f : 1.0f;
-            if (phase == PH_BS) step = sel ? hi : lo;
-#pragma unroll
-            for (int k = 0; k < P; k++) pr[k] = __builtin_fmaf(d[k], step, x[k]);
-        }
-
-        const float L = loss_eval<MODEL, R, FAST>(q, c1, wx, wy, pr, lt);
-
-        if (phase == PH_G0) {
-#pragma unroll
-            for (int k = 0; k < P; k++) t[k] = pr[k];
-            ln = L;
-            phase = PH_G1;
-        } else if (phase == PH_G1) {
-#pragma unroll
-            for (int k = 0; k < P; k++) {
-                t[k] = pr[k];
-                if (k == gi) {
-                    g[k] = (L - ln) * 250.0f;
-                    t[k] = t[k] - 0.002f;
-                }
-            }
-            gi++;
-            phase = PH_G0;
-            if (gi == P) {
-                if (first) {
-                    first = false;
-#pragma unroll
-                    for (int k = 0; k < P; k++) d[k] = -g[k];
-                } else {
-                    float y[P], s[P];
-#pragma unroll
-                    for (int k = 0; k < P; k++) { y[k] = g[k] - gprev_l[k * 64]; s[k] = s_l[k * 64]; }
-                    bfgs_update<P>(D, s, y);
-#pragma unroll
-                    for (int r = 0; r < P; r++) {     // MatMulVector (bfgsMLE_core.h:184-204)
-                        float acc = 0.0f;
-#pragma unroll
-                        for (int c = 0; c < P; c++) acc = __builtin_fmaf(-D[(r * P + c) * 64], g[c], acc);
-                        d[r] = acc;
-                    }
-                }
-                normalize_dir<P>(d);
-                lo = 0.00001f;
-                hi = 1.0f;
-                phase = PH_L0;
-            }
-        } else if (phase == PH_L0) {
-            L0 = L;
-            phase = PH_L1;
-        } else {
-            if (phase == PH_L1) {
-                L1 = L;
-                bsn = 0;
-            } else {
-                if (sel) L1 = L; else L0 = L;
-                bsn++;
-            }
-            sel = (L0 < L1);
-            const float mid = (lo + hi) * 0.5f;
-            if (sel) hi = mid; else lo = mid;
-            phase = PH_BS;
-            if (bsn == 10) {
-                const float scale = (lo + hi) * 0.5f;
-#pragma unroll
-                for (int k = 0; k < P; k++) {
-                    const float sk = d[k] * scale;
-                    s_l[k * 64] = sk;
-                    x[k] = x[k] + sk;
-                }
-#pragma unroll
-                for (int k = 0; k < P; k++) {
-                    x[k] = (x[k] < 0.01f) ? 0.01f : x[k];   // IninfConstrain (bfgsMLE_core.h:76-85)
-                    gprev_l[k * 64] = g[k];
-                    t[k] = x[k];
-                }
-                gi = 0;
-                phase = PH_G0;
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Per-ROI setup shared by the fitting kernels: photo-electrons q, the loss's data term
-// c1 = 1 - log q, header.
-template <int R>
-__device__ __forceinline__ void load_roi(const uint16_t *__restrict__ rec, const FitConst &fc, float (&q)[R * R],
-                                         float (&c1)[R * R], int &xo, int &yo, int &fr)
-{
-    // the record is R*(R+1) 16-bit words; read it as 32-bit words (R*(R+1) is even)
-    constexpr int NW = R * (R + 1) / 2;
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(rec);
-    uint32_t v[NW];
-#pragma unroll
-    for (int k = 0; k < NW; k++) v[k] = __builtin_nontemporal_load(w + k);
-#pragma unroll
-    for (int i = 0; i < R * R; i++) {
-        const uint32_t word = v[i >> 1];
-        const float adu = (float)((i & 1) ? (word >> 16) : (word & 0xffffu));
-        const float e = (adu - fc.Offset) * fc.KAdc;     // bfgsMLE_GS2D_core.h:144
-        q[i] = (e > 1.0f) ? e : 1.0f;
-        c1[i] = 1.0f - qlogf_normal(q[i]);   // q >= 1
-    }
-    auto word_at = [&](int idx) -> int {
-        const uint32_t word = v[idx >> 1];
-        return (int)((idx & 1) ? (word >> 16) : (word & 0xffffu));
-    };
-    xo = word_at(R * R + 0);
-    yo = word_at(R * R + 1);
-    fr = word_at(R * R + 2) + 65536 * word_at(R * R + 3);
-}
-
-// WLEWeightsCalc (bfgsMLE_core.h:206-238), separable form: w(r, c) = wy[r] * wx[c]
-template <int R>
-__device__ __forceinline__ void wle_weights(float sgx, float sgy, bool mlefit, float (&wx)[R], float (&wy)[R])
-{
-    const float ctr = (float)R / 2.0f;
-    const float sx1 = 1.0f / ((2.0f * sgx) * sgx);
-    const float sy1 = 1.0f / ((2.0f * sgy) * sgy);
-#pragma unroll
-    for (int c = 0; c < R; c++) {
-        const float d = ((float)c + 0.5f) - ctr;
-        wx[c] = mlefit ? 1.0f : qexpf(-((d * d) * sx1));
-        wy[c] = mlefit ? 1.0f : qexpf(-((d * d) * sy1));
-    }
-}
-
-// Border sums of the ROI (PreEstimation_GS2D, bfgsMLE_GS2D_core.h:529-546).
-template <int R>
-__device__ __forceinline__ float border_bkg(const float (&q)[R * R])
-{
-    float m1 = 0.0f, m2 = 0.0f, m3 = 0.0f, m4 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-        m1 = m1 + q[k * R + 0];
-        m2 = m2 + q[k * R + R - 1];
-        m3 = m3 + q[0 * R + k];
-        m4 = m4 + q[(R - 1) * R + k];
-    }
-    m1 = m1 < m2 ? m1 : m2;
-    m3 = m3 < m4 ? m3 : m4;
-    return ((m1 + m3) / 2.0f) / (float)R;
-}
-
-__device__ __forceinline__ float zpoly(const float (&pc)[5], float d, float corr)
-{
-    // bfgsMLE_AS3D_core.h:266-279 with d^k formed by multiplication
-    const float d2 = d * d, d3 = d2 * d, d4 = d2 * d2;
-    float z = pc[0] * d4;
-    z = __builtin_fmaf(pc[1], d3, z);
-    z = __builtin_fmaf(pc[2], d2, z);
-    z = __builtin_fmaf(pc[3], d, z);
-    z = z + pc[4];
-    return z * corr;
-}
-
-// One-emitter fitting kernel.  Lane i fits ROI idx[i] (or i when idx is null) and writes its
-// 12-float row; flag[roi] (if non-null) is set to 1 when a rejected fit qualifies for the
-// two-emitter stage (valid background and SNR > 6, bfgsMLE_GS2D_core.h:279-297).
-// Up to 9x9 the register budget is held to two waves per SIMD (256 VGPRs).  The 7x7 exact-math
-// kernel fits without spills; at 9x9 the kernel spills 30 (2D) or 65 (elliptical) registers outside
-// its loss loop and still runs 1.5-1.6x faster than at its natural one wave.
-// Waves per work-group: they share the 32 KB log table in LDS.  With each wave's BFGS state
-// (9 KB for the 2D model, 12 KB elliptical) a CU holds two groups of four 2D waves, or one group
-// of eight elliptical ones, i.e. two waves per SIMD up to 9x9.
-template <int MODEL, int R> constexpr int fit_wg_waves() { return (MODEL == MODEL_AS3D && R <= 9) ? 8 : 4; }
-
-template <int MODEL, int R, bool FAST>
-__global__ void __launch_bounds__((64 * fit_wg_waves<MODEL, R>()))
-__attribute__((amdgpu_waves_per_eu(R <= 9 ? 2 : 1, R <= 9 ? 2 : 10)))
-fit_1e_kernel(const uint16_t *__restrict__ rois, const float *__restrict__ wle,
-                                                    const int *__restrict__ idx, int n, const int *__restrict__ n_dev,
-                                                    float *__restrict__ loc, int *__restrict__ flag, FitConst fc)
-{
-    constexpr int P = Traits<MODEL>::P;
-    constexpr int HALF = R / 2;
-    __shared__ float2 ltab[kLogTabBN];
-    log_tabb_load(ltab);
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n_dev) n = *n_dev;
-    if (i >= n) return;
-    const int roi = idx ? idx[i] : i;
-
-    float q[R * R], c1[R * R];
-    int xo, yo, fr;
-    load_roi<R>(rois + (size_t)roi * (R * (R + 1)), fc, q, c1, xo, yo, fr);
-
-    const float *wp = wle + (size_t)roi * QCS_WLE_FLOATS;
-    const float sl = wp[1], sr = wp[2], su = wp[3], sd = wp[4];
-    const int mt = (int)wp[5];
-    const bool mlefit = (mt == QCS_MOLTYPE_MLEFIT);
-
-    const float bkg = border_bkg<R>(q);
-    const float amp = q[HALF * R + HALF] - bkg;
-    float x[P], wx[R], wy[R];
-    if (MODEL == MODEL_GS2D) {
-        // bfgsMLELoc_Gauss2D :188-228, PreEstimation_GS2D :548-574
-        float ws = fminf(fminf(sl, sr), fminf(su, sd));
-        ws = fminf(ws, ((float)R / 2.0f) / 2.35f);
-        const float ps = 1.0f / ((2.0f * ws) * ws);
-        x[0] = amp * 0.0078125f;
-        x[1] = (float)HALF + 0.5f;
-        x[2] = (float)HALF + 0.5f;
-        x[3] = ps * 10.0f;
-        x[4] = bkg * 0.015625f;
-        if (!mlefit) {
-            ws = ws / 1.2f;
-            ws = fminf(ws, ((float)R / 2.0f) / 2.35f);
-        }
-        if (fc.WLEEn == 0 && mt != QCS_MOLTYPE_MULTIFIT) ws = (float)R;
-        wle_weights<R>(ws, ws, mlefit, wx, wy);
-    } else {
-        // bfgsMLELoc_AS3D :188-228, PreEstimation_AS3D :578-606
-        float wsx = fminf(sl, sr), wsy = fminf(su, sd);
-        x[0] = amp * 0.0078125f;
-        x[1] = (float)HALF + 0.5f;
-        x[2] = (float)HALF + 0.5f;
-        x[3] = 10.0f * (0.5f / (wsx * wsx));
-        x[4] = 10.0f * (0.5f / (wsy * wsy));
-        x[5] = bkg * 0.015625f;
-        if (!mlefit) {
-            const float cap = ((float)R / 1.6f) / 2.35f;
-            wsx = fminf(wsx, cap);
-            wsy = fminf(wsy, cap);
-        }
-        if (fc.WLEEn == 0 && mt != QCS_MOLTYPE_MULTIFIT) { wsx = (float)R; wsy = (float)R; }
-        wle_weights<R>(wsx, wsy, mlefit, wx, wy);
-    }
-
-    __shared__ float cold[fit_wg_waves<MODEL, R>()][(P * P + 2 * P) * 64];   // per wave
-    bfgs_fit<MODEL, R, FAST>(q, c1, wx, wy, x, &cold[threadIdx.x >> 6][threadIdx.x & 63], ltab);
-
-    float row[QCS_REC_FLOATS];
-    bool ok;
-    float snr;
-    bool valid;
-    const float QE = fc.QE;
-    if (MODEL == MODEL_GS2D) {
-        // bfgsMLELoc_Gauss2D :236-308
-        const float lb = (float)R / 2.0f - 1.5f, ub = (float)R / 2.0f + 1.5f;
-        const float smax = fc.MultiEmitterFitEn ? ((float)R / 2.0f) / 2.35f : ((float)R / 1.5f) / 2.35f;
-        const float pp = (x[0] * 128.0f) / QE;
-        const float bg = (x[4] * 64.0f) / QE;
-        float fx = x[1], fy = x[2];
-        float sg = sqrtf(0.5f / (x[3] * 0.1f));
-        fx = (fx != fx) ? -1.0f : fx;
-        fy = (fy != fy) ? -1.0f : fy;
-        sg = (sg != sg) ? -1.0f : sg;
-        snr = (sqrtf(QE) * pp) / sqrtf(pp + bg);
-        const float tp = (((pp * 2.0f) * 3.141593f) * sg) * sg;
-        valid = !(bg != bg);
-        ok = valid && snr > 4.0f && sg <= smax && sg >= 0.6f && fx > lb && fx < ub && fy > lb && fy < ub;
-        row[0] = pp; row[1] = (fx - (float)HALF) + (float)xo; row[2] = (fy - (float)HALF) + (float)yo;
-        row[3] = 0.0f; row[4] = sg; row[5] = sg; row[6] = tp; row[7] = bg; row[8] = snr;
-        row[9] = 0.0f; row[10] = 0.0f; row[11] = (float)fr;
-    } else {
-        // bfgsMLELoc_AS3D :237-335
-        const float lb = (float)R / 2.0f - 2.5f, ub = (float)R / 2.0f + 2.5f;
-        const float smax = fc.MultiEmitterFitEn ? ((float)R / 2.0f) / 2.35f : ((float)R / 1.5f) / 2.35f;
-        const float pe = x[0] * 128.0f, be = x[5] * 64.0f;
-        float fx = x[1], fy = x[2];
-        float sx = sqrtf(0.5f / (x[3] * 0.1f));
-        float sy = sqrtf(0.5f / (x[4] * 0.1f));
-        fx = (fx != fx) ? -1.0f : fx;
-        fy = (fy != fy) ? -1.0f : fy;
-        sx = (sx != sx) ? -1.0f : sx;
-        sy = (sy != sy) ? -1.0f : sy;
-        snr = pe / sqrtf(pe + be);
-        const float pp = pe / QE, bg = be / QE;
-        const float tp = (((pp * 2.0f) * 3.141593f) * sx) * sy;
-        const float dif = (sx * sx) - (sy * sy);
-        const float z = (dif >= 0.0f) ? zpoly(fc.pG, dif, fc.ZDepthCorrFactor) : zpoly(fc.pL, dif, fc.ZDepthCorrFactor);
-        const float ms = (sx + sy) / 2.0f;
-        valid = !(bg != bg);
-        ok = valid && snr > 3.5f && ms > 0.8f && ms < smax && fx > lb && fx < ub && fy > lb && fy < ub;
-        row[0] = pp; row[1] = (fx - (float)HALF) + (float)xo; row[2] = (fy - (float)HALF) + (float)yo;
-        row[3] = z; row[4] = sx; row[5] = sy; row[6] = tp; row[7] = bg; row[8] = snr;
-        row[9] = 0.0f; row[10] = 0.0f; row[11] = (float)fr;
-    }
-    if (!ok) {
-#pragma unroll
-        for (int k = 0; k < QCS_REC_FLOATS; k++) row[k] = 0.0f;
-    }
-    float4 *dst = reinterpret_cast<float4 *>(loc + (size_t)roi * QCS_REC_FLOATS);
-    dst[0] = make_float4(row[0], row[1], row[2], row[3]);
-    dst[1] = make_float4(row[4], row[5], row[6], row[7]);
-    dst[2] = make_float4(row[8], row[9], row[10], row[11]);
-    if (flag) flag[roi] = (!ok && valid && snr > 6.0f) ? 1 : 0;
-}
-
-#include "fit_multi.inc"
 
 // ---------------------------------------------------------------------------------------------
 // Diagonal-Fisher CRLB of x and y (GaussianCRLB_Calc_top, LocPrecCalc_GaussianCRLB.h:64-128):
@@ -640,61 +106,51 @@ __global__ void __launch_bounds__(64) crlb_kernel(float *__restrict__ loc, int n
 }
 
 // ---------------------------------------------------------------------------------------------
-template <int MODEL, int R, bool FAST>
-static void launch_1e(hipStream_t s, const uint16_t *rois, const float *wle, const int *idx, int n, const int *n_dev,
-                      float *loc, int *flag, const FitConst &fc)
+// Lanes per ROI of a one-emitter call of n ROIs (fit_split.h).  A group of G lanes shortens the
+// serial chain of loss evaluations and puts G times as many waves on the chip, but repeats the
+// parameter arithmetic in every lane; so small calls take the widest group that pays, and each
+// line below lies where the narrower one measured faster (us per call with its CRLB, wide / narrow):
+//   5x5   8 lanes to 24,000 ROIs (143 / 151 at 20,000, 214 / 203 at 40,000), 4 to 64,000 (203 / 214,
+//         296 / 273 at 80,000), 2 to 240,000 (430 / 501 at 160,000; elliptical 1240 / 1068 at 320,000), then 1
+//   7x7   8 to 24,000 (177 / 183, 270 / 258), 4 to 400,000 (1274 / 1343 at 320,000, 3829 / 3614 at
+//         1,000,000; elliptical to 200,000: 987 / 1115 at 160,000, 1870 / 1726 at 320,000), then 1
+//   9x9   16 to 28,000 (270 / 321, 471 / 446), 4 to 110,000 (688 / 744, 1247 / 1151), then 2
+//   11x11 16 to 28,000 (311 / 333, 545 / 539), then 4 (two rows' worth of pixels per lane and more
+//         hold the other sizes back: 2991 against 4082 with 2 lanes at 320,000)
+//   13, 15  16 at every size (13: 1150 against 1364 and 1799 with 8 and 4 at 80,000)
+//   17x17 16 to 20,000 (1082 / 1346, 1842 / 1840 at 40,000), then 8
+static int lanes_1e(int model, int R, int n)
 {
-    constexpr int T = 64 * fit_wg_waves<MODEL, R>();
-    hipLaunchKernelGGL((fit_1e_kernel<MODEL, R, FAST>), dim3((unsigned)((n + T - 1) / T)), dim3(T), 0, s, rois, wle, idx, n,
-                       n_dev, loc, flag, fc);
+    const bool el = model == MODEL_AS3D;
+    switch (R) {
+    case 5: return n <= 24000 ? 8 : n <= 64000 ? 4 : n <= 240000 ? 2 : 1;
+    case 7: return n <= 24000 ? 8 : n <= (el ? 200000 : 400000) ? 4 : 1;
+    case 9: return n <= 28000 ? 16 : n <= 110000 ? 4 : 2;
+    case 11: return n <= 28000 ? 16 : 4;
+    case 17: return n <= 20000 ? 16 : 8;
+    default: return 16;
+    }
 }
 
-template <int MODEL, bool FAST>
-static int launch_1e_r(int R, hipStream_t s, const uint16_t *rois, const float *wle, const int *idx, int n,
-                       const int *n_dev, float *loc, int *flag, const FitConst &fc)
+// The same for the multi-emitter stages, by the cascade's ROI count (a stage fits a part of them;
+// us per cascade, wide / narrow): 8 lanes to 50,000 at 5x5 and 7x7 (7x7: 1519 / 1770 at 60,000, 3631 /
+// 3099 at 200,000; elliptical 833 / 909 at 20,000, 1806 / 1570 at 60,000), 16 to 100,000 at 9x9 and 11x11
+// (9x9: 2318 / 3282 at 60,000, 6284 / 5864 at 200,000; elliptical to 30,000: 1121 / 1345 at 20,000,
+// 2408 / 1839 at 60,000), then 4; 16 at 13x13 (3792 against 8780 at 60,000).
+static int lanes_me(int model, int R, int n)
 {
-    switch (R) {
-    case 5: launch_1e<MODEL, 5, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    case 7: launch_1e<MODEL, 7, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    case 9: launch_1e<MODEL, 9, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    case 11: launch_1e<MODEL, 11, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    case 13: launch_1e<MODEL, 13, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    case 15: launch_1e<MODEL, 15, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    case 17: launch_1e<MODEL, 17, FAST>(s, rois, wle, idx, n, n_dev, loc, flag, fc); break;
-    default: return fail(QCS_ERR_ARG, "ROISize %d not supported by the fitter (odd, 5..17)", R);
-    }
-    QCS_HIP(hipGetLastError());
-    return QCS_OK;
+    if (R <= 7) return n <= 50000 ? 8 : 4;
+    if (R <= 11) return n <= (model == MODEL_AS3D2E ? 30000 : 100000) ? 16 : 4;
+    return 16;
 }
 
 int fit_launch_1e(const qcs_params &p, const uint16_t *d_rois, const float *d_wle, const int *d_idx, int n,
                   const int *d_n, float *d_loc, int *d_flag, hipStream_t s)
 {
     if (n <= 0) return QCS_OK;
-    const FitConst fc = make_fit_const(p);
-    const bool as3d = (p.LocType == QCS_LOCTYPE_AS3D);
-    const bool fast = (p.FitMath == QCS_MATH_FAST);
-    if (as3d)
-        return fast ? launch_1e_r<MODEL_AS3D, true>(p.ROISize, s, d_rois, d_wle, d_idx, n, d_n, d_loc, d_flag, fc)
-                    : launch_1e_r<MODEL_AS3D, false>(p.ROISize, s, d_rois, d_wle, d_idx, n, d_n, d_loc, d_flag, fc);
-    return fast ? launch_1e_r<MODEL_GS2D, true>(p.ROISize, s, d_rois, d_wle, d_idx, n, d_n, d_loc, d_flag, fc)
-                : launch_1e_r<MODEL_GS2D, false>(p.ROISize, s, d_rois, d_wle, d_idx, n, d_n, d_loc, d_flag, fc);
-}
-
-template <int MODEL, bool FAST>
-static int launch_me_r(int R, dim3 grid, hipStream_t s, const uint16_t *rois, const float *wle, const int *list,
-                       const int *n_dev, float *loc, float *second, int *fs, int *ff, const FitConst &fc)
-{
-    switch (R) {
-    case 5: hipLaunchKernelGGL((fit_me_kernel<MODEL, 5, FAST>), grid, dim3(64), 0, s, rois, wle, list, n_dev, loc, second, fs, ff, fc); break;
-    case 7: hipLaunchKernelGGL((fit_me_kernel<MODEL, 7, FAST>), grid, dim3(64), 0, s, rois, wle, list, n_dev, loc, second, fs, ff, fc); break;
-    case 9: hipLaunchKernelGGL((fit_me_kernel<MODEL, 9, FAST>), grid, dim3(64), 0, s, rois, wle, list, n_dev, loc, second, fs, ff, fc); break;
-    case 11: hipLaunchKernelGGL((fit_me_kernel<MODEL, 11, FAST>), grid, dim3(64), 0, s, rois, wle, list, n_dev, loc, second, fs, ff, fc); break;
-    case 13: hipLaunchKernelGGL((fit_me_kernel<MODEL, 13, FAST>), grid, dim3(64), 0, s, rois, wle, list, n_dev, loc, second, fs, ff, fc); break;
-    default: return fail(QCS_ERR_ARG, "ROISize %d not supported by the multi-emitter fitter (odd, 5..13)", R);
-    }
-    QCS_HIP(hipGetLastError());
-    return QCS_OK;
+    const int R = p.ROISize, model = (p.LocType == QCS_LOCTYPE_AS3D) ? MODEL_AS3D : MODEL_GS2D;
+    const SplitArgs a{d_rois, d_wle, d_idx, n, d_n, d_loc, nullptr, d_flag, nullptr};
+    return fit_split_1e(model, R, lanes_1e(model, R, n), p.FitMath == QCS_MATH_FAST, a, make_fit_const(p), s);
 }
 
 // multi-emitter stage over list[j], j < *n_dev (grid sized for n_max)
@@ -702,21 +158,8 @@ int fit_launch_me(const qcs_params &p, int model, const uint16_t *d_rois, const 
                   const int *d_n, float *d_loc, float *d_second, int *d_fs, int *d_ff, hipStream_t s)
 {
     if (n_max <= 0) return QCS_OK;
-    const FitConst fc = make_fit_const(p);
-    const dim3 grid((n_max + 63) / 64);
-    const bool fast = (p.FitMath == QCS_MATH_FAST);
-    const int R = p.ROISize;
-    switch (model) {
-    case MODEL_2E:
-        return fast ? launch_me_r<MODEL_2E, true>(R, grid, s, d_rois, d_wle, d_list, d_n, d_loc, d_second, d_fs, d_ff, fc)
-                    : launch_me_r<MODEL_2E, false>(R, grid, s, d_rois, d_wle, d_list, d_n, d_loc, d_second, d_fs, d_ff, fc);
-    case MODEL_3E:
-        return fast ? launch_me_r<MODEL_3E, true>(R, grid, s, d_rois, d_wle, d_list, d_n, d_loc, d_second, d_fs, d_ff, fc)
-                    : launch_me_r<MODEL_3E, false>(R, grid, s, d_rois, d_wle, d_list, d_n, d_loc, d_second, d_fs, d_ff, fc);
-    default:
-        return fast ? launch_me_r<MODEL_AS3D2E, true>(R, grid, s, d_rois, d_wle, d_list, d_n, d_loc, d_second, d_fs, d_ff, fc)
-                    : launch_me_r<MODEL_AS3D2E, false>(R, grid, s, d_rois, d_wle, d_list, d_n, d_loc, d_second, d_fs, d_ff, fc);
-    }
+    const SplitArgs a{d_rois, d_wle, d_list, n_max, d_n, d_loc, d_second, d_fs, d_ff};
+    return fit_split_me(model, p.ROISize, lanes_me(model, p.ROISize, n_max), p.FitMath == QCS_MATH_FAST, a, make_fit_const(p), s);
 }
 
 int crlb_launch(const qcs_params &p, float *d_loc, int n, const int *d_n, hipStream_t s)
