@@ -96,6 +96,17 @@ struct DSplit {   // D[i] in registers for i < NREG, else at p[(i - NREG) * 64]
     __device__ __forceinline__ float &operator[](int i) { return (NREG > 0 && i < NREG) ? r[i] : p[(i - NREG) * 64]; }
 };
 
+// ln x for normal x: v_log_f32 times ln 2 in two parts, the arithmetic of __logf without its scaling of
+// subnormal and selection of infinite arguments (five instructions instead of twelve, a sixth of a
+// pixel's).  The losses take it of mu / q with mu >= 1e-6 and q below 2^17 / QE, which is normal; an
+// infinite mu makes the loss NaN either way.
+__device__ __forceinline__ float cf_logf(float x)
+{
+    const float r = __builtin_amdgcn_logf(x);
+    const float t = r * 0x1.62e42ep-1f;
+    return t + fmaf(r, 0x1.efa39ep-25f, fmaf(r, 0x1.62e42ep-1f, -t));
+}
+
 // loss sum((mu - q) - q ln(mu / q)) (the Poisson negative log-likelihood up to a constant) and,
 // if G, its gradient with respect to theta (physical units)
 template <int KK, int R, bool G, class QA>
@@ -144,7 +155,7 @@ __device__ __forceinline__ float cf_lossgrad_q(const QA &qa, const float (&th)[C
                 mu = fmaxf(mu, 1e-6f);
                 const float q = qa(r * R + c);
                 // deviance form: terms are O(1), so the FP32 sum resolves loss changes of ~1e-4
-                L += (mu - q) - q * __logf(mu * __builtin_amdgcn_rcpf(q));
+                L += (mu - q) - q * cf_logf(mu * __builtin_amdgcn_rcpf(q));
                 if (G) {
                     const float w = 1.0f - q * __builtin_amdgcn_rcpf(mu);
                     gb += w;
@@ -219,7 +230,7 @@ __device__ __forceinline__ float cf_lossgrad_q(const QA &qa, const float (&th)[C
                 }
                 mu = fmaxf(mu, 1e-6f);
                 const float q = qa(r * R + c);
-                L += (mu - q) - q * __logf(mu * __builtin_amdgcn_rcpf(q));
+                L += (mu - q) - q * cf_logf(mu * __builtin_amdgcn_rcpf(q));
                 if (G) {
                     const float w = 1.0f - q * __builtin_amdgcn_rcpf(mu);
                     gb += w;
@@ -1122,9 +1133,19 @@ struct CfqSet {
     int init_mode;   // start of this set's fits (CF_INIT_*; a launch may mix them)
 };
 
+// Fits that the one-lane waves of a launch leave to the split launch: records (CQ<KK>::XW floats),
+// their count, room for cap of them; a wave leaves its fits when its queue is dry and at most
+// `most` of its lanes still run one.
+struct CqLeft {
+    float *rec;
+    int *cnt;
+    int cap, most;
+};
+
 // arguments of one persistent launch (up to three ROI sizes, each with its own queue head)
 struct CfqArgs {
     CfqSet set[3];
+    CqLeft left[3];
     int nsets;
     int *heads;
     CFitConst c;

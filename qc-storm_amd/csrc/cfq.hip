@@ -16,24 +16,18 @@
 //     costs one evaluation where the one-pass kernel spends two;
 //   likelihood pass (one lane per work item): FP64 log-likelihood at the final parameters.
 //
+// Small launches, and the last fits of large ones (which a wave leaves once its queue is dry and
+// few of its lanes still run), go to the split kernel (cfs.hip), 16 to 64 lanes per fit.
+//
 // A launch holds up to three sets of ROIs (sizes 7, 9, 11, each with its own queue): every wave
 // drains the sets in order with its LDS sized for the largest.  Each step's arithmetic is that
 // of the one-pass kernel, so both give bit-identical parameters, iteration counts and flags (the
 // evaluation counts differ by the saved gradient evaluations).
 #include <string.h>
 #include <type_traits>
-#include "cfit_dev.h"
+#include "cfq.h"
 
 namespace qcs {
-
-// record of one work item: theta, loss, gradient, "identity start" flag, packed D0, padding
-template <int KK> struct CQ {
-    static constexpr int P = CP<KK>::P, NS = CP<KK>::NS;
-    static constexpr int OL = P, OG = P + 1, OF = 2 * P + 1, OD = 2 * P + 2;
-    static constexpr int W = (2 * P + 2 + NS + 3) & ~3;   // floats, a multiple of 4
-};
-
-enum { CQ_IDLE = 0, CQ_DIR = 1, CQ_LS = 2 };
 
 template <int KK, int R>
 __global__ void __launch_bounds__(64) cfq_prep_kernel(CfqSet S, CFitConst c)
@@ -114,7 +108,7 @@ template <class LY> using CqQ = typename std::conditional<LY::QU16, uint16_t, fl
 constexpr int CQ_CHUNK = 64;   // most items a wave takes from the queue with one atomic
 
 template <int KK, int R, class LY>
-__device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CFitConst &c, CqQ<LY> *qsh, float *Dsh)
+__device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CqLeft &left, const CFitConst &c, CqQ<LY> *qsh, float *Dsh)
 {
     using Q = CQ<KK>;
     constexpr int P = Q::P;
@@ -224,7 +218,39 @@ __device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CFitCo
         direction();
         refill();      // lanes whose fit converged just now
         direction();
-        if (dry && __all(st == CQ_IDLE)) break;
+        if (dry) {
+            const unsigned long long act = __ballot(st != CQ_IDLE);
+            if (act == 0ull) break;
+            // The queue is empty and few of the wave's fits still run: they go to the split launch
+            // (cfs.hip), which takes each of them further in a fraction of the time.
+            if (left.rec && __popcll(act) <= left.most) {
+                const int at = wave_append(left.cnt, st != CQ_IDLE);
+                if (at >= 0 && at < left.cap) {
+                    float *o = left.rec + (size_t)at * Q::XW;
+#pragma unroll
+                    for (int i = 0; i < P; i++) {
+                        o[i] = th[i];
+                        o[Q::OG + i] = g[i];
+                        o[Q::OX + CX_DU + i] = du[i];
+                    }
+                    o[Q::OL] = L;
+                    o[Q::OF] = first ? 1.0f : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < Q::NS; i++) o[Q::OD + i] = D[i];
+                    o[Q::OX + CX_SLOPE] = slope;
+                    o[Q::OX + CX_ALPHA] = alpha;
+                    o[Q::OX + CX_DMAX] = dmax;
+                    int *h = reinterpret_cast<int *>(o + Q::OX);
+                    h[CX_ROI] = roi;
+                    h[CX_ST] = st;
+                    h[CX_T] = t;
+                    h[CX_ITERS] = iters;
+                    h[CX_EVALS] = evals;
+                    h[CX_PIN] = pin_run;
+                }
+                break;
+            }
+        }
         if (st != CQ_LS) continue;
         float tn[P], gt[P];
 #pragma unroll
@@ -285,12 +311,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CqLayou
     for (int si = 0; si < a.nsets; si++) {
         const int R = a.set[si].R;
         if constexpr (RMAX >= 11) {
-            if (R == 11) cfq_run<KK, 11, LY>(a.set[si], a.heads + si, a.c, qsh, Dsh);
+            if (R == 11) cfq_run<KK, 11, LY>(a.set[si], a.heads + si, a.left[si], a.c, qsh, Dsh);
         }
         if constexpr (RMAX >= 9) {
-            if (R == 9) cfq_run<KK, 9, LY>(a.set[si], a.heads + si, a.c, qsh, Dsh);
+            if (R == 9) cfq_run<KK, 9, LY>(a.set[si], a.heads + si, a.left[si], a.c, qsh, Dsh);
         }
-        if (R == 7) cfq_run<KK, 7, LY>(a.set[si], a.heads + si, a.c, qsh, Dsh);
+        if (R == 7) cfq_run<KK, 7, LY>(a.set[si], a.heads + si, a.left[si], a.c, qsh, Dsh);
     }
 }
 
@@ -312,15 +338,16 @@ __global__ void __launch_bounds__(64) cfq_ll_kernel(CfqSet S, CFitConst c)
 
 // ---- host -----------------------------------------------------------------------------------
 
-static int cq_rec_w(int KK)
+// words of a work item's record and of a left fit's
+static void cq_rec_w(int KK, int &w, int &xw)
 {
     switch (KK) {
-    case 1: return CQ<1>::W;
-    case 2: return CQ<2>::W;
-    case 3: return CQ<3>::W;
-    case 11: return CQ<11>::W;
-    case 12: return CQ<12>::W;
-    default: return CQ<13>::W;
+    case 1: w = CQ<1>::W; xw = CQ<1>::XW; break;
+    case 2: w = CQ<2>::W; xw = CQ<2>::XW; break;
+    case 3: w = CQ<3>::W; xw = CQ<3>::XW; break;
+    case 11: w = CQ<11>::W; xw = CQ<11>::XW; break;
+    case 12: w = CQ<12>::W; xw = CQ<12>::XW; break;
+    default: w = CQ<13>::W; xw = CQ<13>::XW; break;
     }
 }
 
@@ -347,6 +374,27 @@ static int cq_waves_per_cu(int KK, int RMAX)
     return v;
 }
 
+// Whether a launch of `items` fits goes to the split kernel (cfs.hip) as a whole, and if not how
+// many running fits a one-lane wave of an empty queue leaves to it (most).  Measured, us per launch
+// with prep and likelihood (split / best one-lane with leaving / one-lane alone):
+//   2D 7x7, K = 1  8,000: 150 / 166 / 402   16,000: 220 / 176 / 452   262,144: 2621 / 581 / 830
+//           K = 2  16,000: 429 / 420 / 1093  32,000: 589 / 572 / 1325  262,144: 3153 / 1306 / 1767
+//           K = 3  32,000: 801 / 852 / 1762  64,000: 1235 / 1040 / 1780  262,144: 4054 / 1891 / 2455
+//   elliptical 9x9, K = 1  8,192: 378 / 605 / 2398  16,461: 674 / 600 / 2384  262,144: 3461 / 1430 / 4335
+//           K = 2  8,192: 1238 / 1708 / 10466  16,461: 3180 / 2071 / 10046  262,144: 10734 / 7626 / 17499
+//           K = 3  16,461: 4401 / 5510 / 22605  262,144: 23268 / 32635 / 51638 (a quarter of its fits run to
+//                  the iteration cap, at 160 evaluations a fit): split at every size
+// Leaving early pays while the one-lane waves are few (16 of 64 lanes in 2D, 32 elliptical); beyond
+// 49,152 fits, 8 (2D K = 1, 64,000: 250 against 291 at 16 and 345 at 4), elliptical K = 2 still 32.
+static bool cq_route(int KK, long long items, int &most)
+{
+    const bool el = KK > CF_ELLIPTIC;
+    const int K = el ? KK - CF_ELLIPTIC : KK;
+    static const int line[3] = {12000, 28000, 40000};
+    most = el ? (items <= 49152 || K == 2 ? 32 : 8) : (items <= 49152 ? 16 : 8);
+    return el ? (K == 3 || items <= 12000) : items <= line[K - 1];
+}
+
 int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_t s)
 {
     if (K < 1 || K > 3) return fail(QCS_ERR_ARG, "emitter count %d not in 1..3", K);
@@ -355,7 +403,8 @@ int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_
     memset(&a, 0, sizeof(a));
     a.c = cfit_const(ctx->p, ctx->tune, K, CF_INIT_HEUR);
     const int KK = cf_kk(ctx->p, K);
-    const int W = cq_rec_w(KK);
+    int W, XW;
+    cq_rec_w(KK, W, XW);
     size_t total = 0;
     int rmax = 0;
     long long items = 0;
@@ -371,8 +420,17 @@ int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_
         rmax = x.R > rmax ? x.R : rmax;
     }
     if (items == 0) return QCS_OK;
+    int cus = 0;
+    QCS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    int wpc = cq_waves_per_cu(KK, rmax);
+    if (ctx->tune.waves_per_cu > 0 && ctx->tune.waves_per_cu < wpc) wpc = ctx->tune.waves_per_cu;
+    long long waves = (items + 63) / 64;
+    if (waves > (long long)cus * wpc) waves = (long long)cus * wpc;
+    int most;
+    const bool split = cq_route(KK, items, most);
+    const size_t lcap = split ? 0 : (size_t)waves * most;   // fits the waves may leave, per set
     int rc;
-    if ((rc = ctx->cf_queue.ensure(256 + total * sizeof(float)))) return rc;
+    if ((rc = ctx->cf_queue.ensure(256 + (total + lcap * XW * nsets) * sizeof(float)))) return rc;
     int *heads = ctx->cf_queue.as<int>();
     float *rec = reinterpret_cast<float *>(ctx->cf_queue.as<char>() + 256);
     // largest ROIs first: the longest fits start early and the tail stays short
@@ -391,27 +449,28 @@ int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_
         off += (size_t)x.n * W;
     }
     a.heads = heads;
-    fill_async(heads, 4, 0, s);
+    for (int i = 0; i < a.nsets && lcap > 0; i++) a.left[i] = CqLeft{rec + total + (size_t)i * lcap * XW, heads + 8 + i, (int)lcap, most};
+    fill_async(heads, 16, 0, s);
     for (int i = 0; i < a.nsets; i++) {
         const CfqSet &x = a.set[i];
         const dim3 grid((x.n + 63) / 64), block(64);
         CF_DISPATCH_KK(KK, CF_DISPATCH_R(x.R, hipLaunchKernelGGL((cfq_prep_kernel<KT, RT>), grid, block, 0, s, x, a.c)))
     }
     QCS_HIP(hipGetLastError());
-    int cus = 0;
-    QCS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    int wpc = cq_waves_per_cu(KK, rmax);
-    if (ctx->tune.waves_per_cu > 0 && ctx->tune.waves_per_cu < wpc) wpc = ctx->tune.waves_per_cu;
-    long long waves = (items + 63) / 64;
-    if (waves > (long long)cus * wpc) waves = (long long)cus * wpc;
-    const dim3 pgrid((unsigned)waves), block(64);
-    CF_DISPATCH_KK(KK, CF_DISPATCH_R(rmax, hipLaunchKernelGGL((cfq_kernel<KT, RT>), pgrid, block, 0, s, a)))
-    QCS_HIP(hipGetLastError());
+    if (split) {
+        if ((rc = cfs_launch(a, KK, rmax, items, cus, ctx->tune.waves_per_cu, s))) return rc;
+    } else {
+        const dim3 pgrid((unsigned)waves), block(64);
+        CF_DISPATCH_KK(KK, CF_DISPATCH_R(rmax, hipLaunchKernelGGL((cfq_kernel<KT, RT>), pgrid, block, 0, s, a)))
+        QCS_HIP(hipGetLastError());
+        a.heads = heads + 4;
+        if ((rc = cfs_launch(a, KK, rmax, (long long)lcap, cus, ctx->tune.waves_per_cu, s))) return rc;
+    }
     for (int i = 0; i < a.nsets; i++) {
         const CfqSet &x = a.set[i];
         if (!x.ll) continue;
         const dim3 grid((x.n + 63) / 64);
-        CF_DISPATCH_KK(KK, CF_DISPATCH_R(x.R, hipLaunchKernelGGL((cfq_ll_kernel<KT, RT>), grid, block, 0, s, x, a.c)))
+        CF_DISPATCH_KK(KK, CF_DISPATCH_R(x.R, hipLaunchKernelGGL((cfq_ll_kernel<KT, RT>), grid, dim3(64), 0, s, x, a.c)))
     }
     QCS_HIP(hipGetLastError());
     return QCS_OK;
