@@ -11,8 +11,9 @@
 //
 // Every layer is an "NT" GEMM (nn_gemm.h) over im2col rows: conv1 has 25 rows per ROI of 9 taps
 // padded to 16; conv2 9 rows of 288; conv3 reads conv2's output rows as one 576-wide row per ROI
-// (no copy).  Backward: dW = dY^T X and dX = dY W through transposed bf16 copies, col2im for
-// conv2 -> conv1, bias gradients by column sums.
+// (no copy); bias, ReLU and the bf16 rounding are the product's last step.  Backward: dX = dY W with
+// transposed weight copies and the ReLU below as the product's last step, col2im for conv2 -> conv1,
+// then every layer's dW = dY^T X and bias sums in one launch split over the rows (nn_gemm.h).
 #include <math.h>
 #include <string.h>
 #include <new>
@@ -37,14 +38,16 @@ constexpr int OW1 = 0, OB1 = OW1 + W1N, OW2 = OB1 + B1N, OB2 = OW2 + W2N, OW3 = 
 constexpr int CHUNK = 65536;  // ROIs per forward/backward pass (activation buffers scale with it)
 constexpr float CE_W = 4.0f;  // weight of the count cross-entropy against the parameter errors
 
-inline int rup16(int v) { return (v + 15) & ~15; }
 inline unsigned nblk(size_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-// per ROI: normalised image -> conv1 im2col rows, side features, (scale, bhat)
+// per ROI: normalised image -> conv1 im2col rows, side features (fc1's input columns 64..79), (scale,
+// bhat); clears *loss where given
 __global__ void prep_kernel(const uint16_t *__restrict__ rois, int n, float offset, float kadc, float inv_qe,
-                            uint16_t *__restrict__ x1, float *__restrict__ norm, uint16_t *__restrict__ side)
+                            uint16_t *__restrict__ x1, float *__restrict__ norm, uint16_t *__restrict__ a3,
+                            float *__restrict__ loss)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (loss && i == 0) *loss = 0.0f;
     if (i >= n) return;
     const uint16_t *src = rois + (size_t)i * NR * (NR + 1);
     float q[NRR];
@@ -78,34 +81,11 @@ __global__ void prep_kernel(const uint16_t *__restrict__ rois, int n, float offs
 #pragma unroll
             for (int t = 0; t < K1; t++) row[t] = (t < 9) ? xv[(py + t / 3) * NR + px + t % 3] : (uint16_t)0;
         }
-    uint16_t *sd = side + (size_t)i * NSIDE;
+    uint16_t *sd = a3 + (size_t)i * F0 + C3;
     sd[0] = f2bf(logf(scale) * 0.1f);
     sd[1] = f2bf(bh * is);
 #pragma unroll
     for (int t = 2; t < NSIDE; t++) sd[t] = 0;
-}
-
-// out(bf16, ldo) = act(Y + bias)
-__global__ void bias_act_kernel(const float *__restrict__ Y, const float *__restrict__ bias, int rows, int ncol, int ldy,
-                                uint16_t *__restrict__ out, int ldo)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * ncol) return;
-    const int r = (int)(i / ncol), c = (int)(i % ncol);
-    out[(size_t)r * ldo + c] = f2bf(fmaxf(Y[(size_t)r * ldy + c] + bias[c], 0.0f));
-}
-
-__global__ void out_bias_kernel(float *__restrict__ yo, const float *__restrict__ b, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n * NO) yo[i] += b[i % NO];
-}
-
-__global__ void side_kernel(const uint16_t *__restrict__ side, int n, uint16_t *__restrict__ a3)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * NSIDE) return;
-    a3[(size_t)(i / NSIDE) * F0 + C3 + i % NSIDE] = side[i];
 }
 
 // conv2 im2col: a1 [n*25][32] -> x2 [n*9][288], column (ty*3 + tx)*32 + ch; 4 channels per thread
@@ -124,8 +104,10 @@ __global__ void im2col2_kernel(const uint16_t *__restrict__ a1, int n, uint16_t 
     *reinterpret_cast<uint2 *>(x2 + ((roi * 9 + pos) * K2 + tap * C1 + c4 * 4)) = v;
 }
 
-// col2im for conv2: dx2 [n*9][288] -> da1 [n*25][32] (sum over the taps that read each input)
-__global__ void col2im2_kernel(const float *__restrict__ dx2, int n, float *__restrict__ da1)
+// col2im for conv2 and conv1's ReLU: dx2 [n*9][288] -> d [n*25][32] (sum over the taps that read each
+// input, where a1 > 0) in fp32 and bf16
+__global__ void col2im2_kernel(const float *__restrict__ dx2, const uint16_t *__restrict__ a1, int n, float *__restrict__ d,
+                               uint16_t *__restrict__ db)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)n * 25 * C1) return;
@@ -135,66 +117,34 @@ __global__ void col2im2_kernel(const float *__restrict__ dx2, int n, float *__re
     const size_t roi = t / 25;
     const int y1 = p1 / 5, x1 = p1 % 5;
     float s = 0.0f;
-    for (int ty = 0; ty < 3; ty++)
-        for (int tx = 0; tx < 3; tx++) {
-            const int py = y1 - ty, px = x1 - tx;
-            if (py < 0 || py >= 3 || px < 0 || px >= 3) continue;
-            s += dx2[(roi * 9 + py * 3 + px) * K2 + (ty * 3 + tx) * C1 + ch];
-        }
-    da1[i] = s;
-}
-
-// d = dA (x) [a > 0]: fp32 (dense rows x ncol) and bf16 copies
-__global__ void relu_back_kernel(const float *__restrict__ dA, int lda, const uint16_t *__restrict__ a, int ld_a, int rows,
-                                 int ncol, float *__restrict__ d, uint16_t *__restrict__ db)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * ncol) return;
-    const int r = (int)(i / ncol), c = (int)(i % ncol);
-    const float v = (bf2f(a[(size_t)r * ld_a + c]) > 0.0f) ? dA[(size_t)r * lda + c] : 0.0f;
-    d[i] = v;
-    db[i] = f2bf(v);
-}
-
-// bf16 transpose with zero padding: in [rows][cols] (ldi) -> out [colsp][rowsp]
-__global__ void transpose_kernel(const uint16_t *__restrict__ in, int rows, int cols, int ldi, uint16_t *__restrict__ out,
-                                 int rowsp, int colsp)
-{
-    __shared__ uint16_t tile[32][33];
-    const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 256 threads: 32 x 8
-    for (int k = ty; k < 32; k += 8) {
-        const int r = by + k, c = bx + tx;
-        tile[k][tx] = (r < rows && c < cols) ? in[(size_t)r * ldi + c] : (uint16_t)0;
+    if (bf2f(a1[i]) > 0.0f) {
+        for (int ty = 0; ty < 3; ty++)
+            for (int tx = 0; tx < 3; tx++) {
+                const int py = y1 - ty, px = x1 - tx;
+                if (py < 0 || py >= 3 || px < 0 || px >= 3) continue;
+                s += dx2[(roi * 9 + py * 3 + px) * K2 + (ty * 3 + tx) * C1 + ch];
+            }
     }
-    __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-        const int c = bx + k, r = by + tx;   // out[c][r] = in[r][c]
-        if (c < colsp && r < rowsp) out[(size_t)c * rowsp + r] = tile[tx][k];
-    }
+    d[i] = s;
+    db[i] = f2bf(s);
 }
 
-// out[c] += sum over a block of rows (out zeroed beforehand); grid.y splits the rows
-__global__ void colsum_kernel(const float *__restrict__ Y, int rows, int ncol, float *__restrict__ out)
-{
-    const int c = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int part = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6), nparts = gridDim.y * (blockDim.x >> 6);
-    if (c >= ncol) return;
-    float s = 0.0f;
-    for (int r = part; r < rows; r += nparts) s += Y[(size_t)r * ncol + c];
-    atomicAdd(&out[c], s);
-}
-
-__global__ void f2bf_kernel(const float *__restrict__ in, size_t n, uint16_t *__restrict__ out)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = f2bf(in[i]);
-}
-
-__global__ void fill0_kernel(float *__restrict__ p, int n)
+// bf16 copies of the weights: wb in the parameters' layout, and wt with the matrices of layers 2 to 5
+// transposed (each at its own offset), for the products that carry gradients back
+__global__ void refresh_kernel(const float *__restrict__ w, uint16_t *__restrict__ wb, uint16_t *__restrict__ wt)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
+    if (i >= NPARAM) return;
+    const uint16_t v = f2bf(w[i]);
+    wb[i] = v;
+    auto put = [&](int off, int rows, int cols) {
+        const int k = i - off;
+        if (k >= 0 && k < rows * cols) wt[off + (k % cols) * rows + k / cols] = v;
+    };
+    put(OW2, C2, K2);
+    put(OW3, C3, K3);
+    put(OW4, F1, F0);
+    put(OW5, NO, F1);
 }
 
 // Loss and gradient per ROI.  labels [n][16]: K (0 = ignore), (x, y, N) x 3 (ROI pixels,
@@ -202,7 +152,7 @@ __global__ void fill0_kernel(float *__restrict__ p, int n)
 // + (dN / (2 pi scale))^2 per slot + ds^2 + 10 (db / scale)^2.  Gradients are of the sum over the ROIs times
 // `wscale` (1 / total labelled ROIs of the step).
 __global__ void loss_kernel(const float *__restrict__ out, const float *__restrict__ labels, const float *__restrict__ norm,
-                            int n, float wscale, float *__restrict__ dY, float *__restrict__ loss_sum)
+                            int n, float wscale, float *__restrict__ dY, uint16_t *__restrict__ dB, float *__restrict__ loss_sum)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     float L = 0.0f;
@@ -237,7 +187,10 @@ __global__ void loss_kernel(const float *__restrict__ out, const float *__restri
             g[13] = 20.0f * eb;
         }
 #pragma unroll
-        for (int t = 0; t < NO; t++) d[t] = g[t] * wscale;
+        for (int t = 0; t < NO; t++) {
+            d[t] = g[t] * wscale;
+            dB[(size_t)i * NO + t] = f2bf(d[t]);
+        }
     }
     for (int off = 32; off > 0; off >>= 1) L += __shfl_down(L, off, 64);
     if ((threadIdx.x & 63) == 0 && L != 0.0f) atomicAdd(loss_sum, L);
@@ -419,13 +372,15 @@ __global__ void __launch_bounds__(64) fwd_fused_kernel(const uint16_t *__restric
 
 }  // namespace nnk
 
-void nn_gemm_nt(const uint16_t *A, const uint16_t *B, float *C, int M, int N, int K, int lda, int ldb, int ldc, bool acc,
+template <int EPI>
+void nn_gemm_nt(const uint16_t *A, const uint16_t *B, float *C, int M, int N, int K, int lda, int ldb, int ldc, const GemmEpi &ep,
                 hipStream_t s)
 {
     if (M <= 0 || N <= 0) return;
-    const dim3 grid((N + 63) / 64, (M + 63) / 64), block(256);
-    if (acc) hipLaunchKernelGGL(gemm_nt_kernel<true>, grid, block, 0, s, A, B, C, M, N, K, lda, ldb, ldc);
-    else hipLaunchKernelGGL(gemm_nt_kernel<false>, grid, block, 0, s, A, B, C, M, N, K, lda, ldb, ldc);
+    // 64 x 64 outputs per work-group where that gives every CU two, else 32 x 32
+    const dim3 g2((N + 63) / 64, (M + 63) / 64), g1((N + 31) / 32, (M + 31) / 32), block(256);
+    if ((long long)g2.x * g2.y >= 512) hipLaunchKernelGGL((gemm_nt_kernel<EPI, 2>), g2, block, 0, s, A, B, C, M, N, K, lda, ldb, ldc, ep);
+    else hipLaunchKernelGGL((gemm_nt_kernel<EPI, 1>), g1, block, 0, s, A, B, C, M, N, K, lda, ldb, ldc, ep);
 }
 
 }  // namespace qcs
@@ -436,154 +391,138 @@ using namespace qcs::nnk;
 struct qcs_net {
     int device = 0;
     long long steps = 0;
-    DevBuf w, g, m, v, wb, wt, loss;          // parameters (fp32 master, gradient, Adam moments), bf16 copy
-    DevBuf x1, a1, x2, a2, a3, a4, side, norm, yo, Y, dF, dG, dB, tA, tB;
+    DevBuf w, g, m, v, wb, wt, loss;          // parameters (fp32 master, gradient, Adam moments), bf16 copies
+    DevBuf x1, a1, x2, a2, a3, a4, norm, yo, dF;
+    DevBuf d[5], db[5];                       // gradients at the layers' outputs (1..5), fp32 and bf16
+    DevBuf part;                              // partial sums of the weight gradients
     HostBuf pin;
     bool ready = false;
 };
 
 namespace {
 
+constexpr int DCOL[5] = {25 * C1, 9 * C2, C3, F1, NO};   // values per ROI at each layer's output
+constexpr int WN[5] = {W1N + B1N, W2N + B2N, W3N + B3N, W4N + B4N, W5N + B5N};
+
 int net_alloc(qcs_net *nt)
 {
     const size_t N = CHUNK;
     int rc;
     if ((rc = nt->w.ensure(NPARAM * 4)) || (rc = nt->g.ensure(NPARAM * 4)) || (rc = nt->m.ensure(NPARAM * 4)) ||
-        (rc = nt->v.ensure(NPARAM * 4)) || (rc = nt->wb.ensure(NPARAM * 2)) || (rc = nt->wt.ensure((size_t)K3 * C3 * 2)) ||
+        (rc = nt->v.ensure(NPARAM * 4)) || (rc = nt->wb.ensure(NPARAM * 2)) || (rc = nt->wt.ensure(NPARAM * 2)) ||
         (rc = nt->loss.ensure(64)) || (rc = nt->x1.ensure(N * 25 * K1 * 2)) || (rc = nt->a1.ensure(N * 25 * C1 * 2)) ||
         (rc = nt->x2.ensure(N * 9 * K2 * 2)) || (rc = nt->a2.ensure(N * 9 * C2 * 2)) || (rc = nt->a3.ensure(N * F0 * 2)) ||
-        (rc = nt->a4.ensure(N * F1 * 2)) || (rc = nt->side.ensure(N * NSIDE * 2)) || (rc = nt->norm.ensure(N * 2 * 4)) ||
-        (rc = nt->yo.ensure(N * NO * 4)) || (rc = nt->Y.ensure(N * 25 * C1 * 4)) || (rc = nt->dF.ensure(N * 9 * K2 * 4)) ||
-        (rc = nt->dG.ensure(N * 25 * C1 * 4)) || (rc = nt->dB.ensure(N * 25 * C1 * 2)) ||
-        (rc = nt->tA.ensure(N * 25 * C1 * 2)) || (rc = nt->tB.ensure(N * 9 * K2 * 2)) || (rc = nt->pin.ensure(64)))
+        (rc = nt->a4.ensure(N * F1 * 2)) || (rc = nt->norm.ensure(N * 2 * 4)) || (rc = nt->yo.ensure(N * NO * 4)) ||
+        (rc = nt->dF.ensure(N * 9 * K2 * 4)) || (rc = nt->part.ensure((size_t)NPARAM * WG_PARTS * 4)) ||
+        (rc = nt->pin.ensure((NPARAM + 16) * 4)))
         return rc;
+    for (int l = 0; l < 5; l++)
+        if ((rc = nt->d[l].ensure(N * DCOL[l] * 4)) || (rc = nt->db[l].ensure(N * DCOL[l] * 2))) return rc;
     return QCS_OK;
-}
-
-void tr(const uint16_t *in, int rows, int cols, int ldi, uint16_t *out, hipStream_t s)
-{
-    const int rp = rup16(rows), cp = rup16(cols);
-    hipLaunchKernelGGL(transpose_kernel, dim3((cp + 31) / 32, (rp + 31) / 32), dim3(256), 0, s, in, rows, cols, ldi, out, rp, cp);
-}
-
-void colsum(const float *Y, int rows, int ncol, float *out, hipStream_t s)
-{
-    int parts = (rows + 4095) / 4096;
-    parts = parts < 1 ? 1 : (parts > 64 ? 64 : parts);
-    hipLaunchKernelGGL(colsum_kernel, dim3((ncol + 63) / 64, parts), dim3(256), 0, s, Y, rows, ncol, out);
 }
 
 void refresh_bf16(qcs_net *nt, hipStream_t s)
 {
-    hipLaunchKernelGGL(f2bf_kernel, dim3(nblk(NPARAM)), dim3(256), 0, s, nt->w.as<float>(), (size_t)NPARAM, nt->wb.as<uint16_t>());
+    hipLaunchKernelGGL(refresh_kernel, dim3(nblk(NPARAM)), dim3(256), 0, s, nt->w.as<float>(), nt->wb.as<uint16_t>(),
+                       nt->wt.as<uint16_t>());
 }
 
-// forward over n <= CHUNK ROIs: activations, outputs yo [n][16] and norm [n][2]
-int net_forward(qcs_net *nt, const qcs_params &p, const uint16_t *d_rois, int n, hipStream_t s)
+// forward over n <= CHUNK ROIs: activations, outputs yo [n][16] and norm [n][2]; clears *loss where given
+int net_forward(qcs_net *nt, const qcs_params &p, const uint16_t *d_rois, int n, float *loss, hipStream_t s)
 {
     const uint16_t *W = nt->wb.as<uint16_t>();
     const float *wf = nt->w.as<float>();
-    float *Y = nt->Y.as<float>();
     hipLaunchKernelGGL(prep_kernel, dim3(nblk(n, 64)), dim3(64), 0, s, d_rois, n, p.Offset, p.KAdc, 1.0f / p.QE,
-                       nt->x1.as<uint16_t>(), nt->norm.as<float>(), nt->side.as<uint16_t>());
-    nn_gemm_nt(nt->x1.as<uint16_t>(), W + OW1, Y, n * 25, C1, K1, K1, K1, C1, false, s);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((size_t)n * 25 * C1)), dim3(256), 0, s, Y, wf + OB1, n * 25, C1, C1,
-                       nt->a1.as<uint16_t>(), C1);
+                       nt->x1.as<uint16_t>(), nt->norm.as<float>(), nt->a3.as<uint16_t>(), loss);
+    auto out = [&](int ob, DevBuf &a, int ldo) {
+        GemmEpi e;
+        e.bias = wf + ob;
+        e.o = a.as<uint16_t>();
+        e.ldo = ldo;
+        return e;
+    };
+    nn_gemm_nt<EPI_RELU>(nt->x1.as<uint16_t>(), W + OW1, nullptr, n * 25, C1, K1, K1, K1, 0, out(OB1, nt->a1, C1), s);
     hipLaunchKernelGGL(im2col2_kernel, dim3(nblk((size_t)n * 81 * (C1 / 4))), dim3(256), 0, s, nt->a1.as<uint16_t>(), n,
                        nt->x2.as<uint16_t>());
-    nn_gemm_nt(nt->x2.as<uint16_t>(), W + OW2, Y, n * 9, C2, K2, K2, K2, C2, false, s);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((size_t)n * 9 * C2)), dim3(256), 0, s, Y, wf + OB2, n * 9, C2, C2,
-                       nt->a2.as<uint16_t>(), C2);
-    nn_gemm_nt(nt->a2.as<uint16_t>(), W + OW3, Y, n, C3, K3, K3, K3, C3, false, s);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((size_t)n * C3)), dim3(256), 0, s, Y, wf + OB3, n, C3, C3,
-                       nt->a3.as<uint16_t>(), F0);
-    hipLaunchKernelGGL(side_kernel, dim3(nblk((size_t)n * NSIDE)), dim3(256), 0, s, nt->side.as<uint16_t>(), n,
-                       nt->a3.as<uint16_t>());
-    nn_gemm_nt(nt->a3.as<uint16_t>(), W + OW4, Y, n, F1, F0, F0, F0, F1, false, s);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((size_t)n * F1)), dim3(256), 0, s, Y, wf + OB4, n, F1, F1,
-                       nt->a4.as<uint16_t>(), F1);
-    float *yo = nt->yo.as<float>();
-    nn_gemm_nt(nt->a4.as<uint16_t>(), W + OW5, yo, n, NO, F1, F1, F1, NO, false, s);
-    hipLaunchKernelGGL(out_bias_kernel, dim3(nblk((size_t)n * NO)), dim3(256), 0, s, yo, wf + OB5, n);
+    nn_gemm_nt<EPI_RELU>(nt->x2.as<uint16_t>(), W + OW2, nullptr, n * 9, C2, K2, K2, K2, 0, out(OB2, nt->a2, C2), s);
+    nn_gemm_nt<EPI_RELU>(nt->a2.as<uint16_t>(), W + OW3, nullptr, n, C3, K3, K3, K3, 0, out(OB3, nt->a3, F0), s);
+    nn_gemm_nt<EPI_RELU>(nt->a3.as<uint16_t>(), W + OW4, nullptr, n, F1, F0, F0, F0, 0, out(OB4, nt->a4, F1), s);
+    nn_gemm_nt<EPI_BIAS>(nt->a4.as<uint16_t>(), W + OW5, nt->yo.as<float>(), n, NO, F1, F1, F1, NO, out(OB5, nt->a4, 0), s);
     QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
 
-// accumulate the gradient of the loss over n <= CHUNK labelled ROIs (after net_forward) into g
-int net_backward(qcs_net *nt, const float *d_labels, int n, float wscale, hipStream_t s)
+// the gradient of the loss over n <= CHUNK labelled ROIs (after net_forward) into g (add: onto it)
+int net_backward(qcs_net *nt, const float *d_labels, int n, float wscale, bool add, hipStream_t s)
 {
-    const int n16 = rup16(n), n9 = rup16(9 * n), n25 = rup16(25 * n);
-    float *g = nt->g.as<float>(), *dF = nt->dF.as<float>(), *dG = nt->dG.as<float>();
-    uint16_t *W = nt->wb.as<uint16_t>(), *dB = nt->dB.as<uint16_t>(), *tA = nt->tA.as<uint16_t>(), *tB = nt->tB.as<uint16_t>(),
-             *wt = nt->wt.as<uint16_t>();
+    const uint16_t *WT = nt->wt.as<uint16_t>();
+    float *d[5], *dF = nt->dF.as<float>();
+    uint16_t *db[5];
+    for (int l = 0; l < 5; l++) {
+        d[l] = nt->d[l].as<float>();
+        db[l] = nt->db[l].as<uint16_t>();
+    }
     hipLaunchKernelGGL(loss_kernel, dim3(nblk(n, 64)), dim3(64), 0, s, nt->yo.as<float>(), d_labels, nt->norm.as<float>(), n,
-                       wscale, dG, nt->loss.as<float>());
-    // fc2
-    colsum(dG, n, NO, g + OB5, s);
-    hipLaunchKernelGGL(f2bf_kernel, dim3(nblk((size_t)n * NO)), dim3(256), 0, s, dG, (size_t)n * NO, dB);
-    tr(dB, n, NO, NO, tA, s);
-    tr(nt->a4.as<uint16_t>(), n, F1, F1, tB, s);
-    nn_gemm_nt(tA, tB, g + OW5, NO, F1, n16, n16, n16, F1, true, s);
-    tr(W + OW5, NO, F1, F1, wt, s);
-    nn_gemm_nt(dB, wt, dF, n, F1, NO, NO, NO, F1, false, s);
-    hipLaunchKernelGGL(relu_back_kernel, dim3(nblk((size_t)n * F1)), dim3(256), 0, s, dF, F1, nt->a4.as<uint16_t>(), F1, n, F1, dG,
-                       dB);
-    // fc1
-    colsum(dG, n, F1, g + OB4, s);
-    tr(dB, n, F1, F1, tA, s);
-    tr(nt->a3.as<uint16_t>(), n, F0, F0, tB, s);
-    nn_gemm_nt(tA, tB, g + OW4, F1, F0, n16, n16, n16, F0, true, s);
-    tr(W + OW4, F1, F0, F0, wt, s);
-    nn_gemm_nt(dB, wt, dF, n, F0, F1, F1, F1, F0, false, s);
-    hipLaunchKernelGGL(relu_back_kernel, dim3(nblk((size_t)n * C3)), dim3(256), 0, s, dF, F0, nt->a3.as<uint16_t>(), F0, n, C3, dG,
-                       dB);
-    // conv3 (input: a2 as [n][576])
-    colsum(dG, n, C3, g + OB3, s);
-    tr(dB, n, C3, C3, tA, s);
-    tr(nt->a2.as<uint16_t>(), n, K3, K3, tB, s);
-    nn_gemm_nt(tA, tB, g + OW3, C3, K3, n16, n16, n16, K3, true, s);
-    tr(W + OW3, C3, K3, K3, wt, s);
-    nn_gemm_nt(dB, wt, dF, n, K3, C3, C3, C3, K3, false, s);   // = d a2 [n*9][64]
-    hipLaunchKernelGGL(relu_back_kernel, dim3(nblk((size_t)n * 9 * C2)), dim3(256), 0, s, dF, C2, nt->a2.as<uint16_t>(), C2, n * 9,
-                       C2, dG, dB);
-    // conv2
-    colsum(dG, n * 9, C2, g + OB2, s);
-    tr(dB, n * 9, C2, C2, tA, s);
-    tr(nt->x2.as<uint16_t>(), n * 9, K2, K2, tB, s);
-    nn_gemm_nt(tA, tB, g + OW2, C2, K2, n9, n9, n9, K2, true, s);
-    tr(W + OW2, C2, K2, K2, wt, s);
-    nn_gemm_nt(dB, wt, dF, n * 9, K2, C2, C2, C2, K2, false, s);   // d x2 [n*9][288]
-    hipLaunchKernelGGL(col2im2_kernel, dim3(nblk((size_t)n * 25 * C1)), dim3(256), 0, s, dF, n, nt->Y.as<float>());
-    hipLaunchKernelGGL(relu_back_kernel, dim3(nblk((size_t)n * 25 * C1)), dim3(256), 0, s, nt->Y.as<float>(), C1,
-                       nt->a1.as<uint16_t>(), C1, n * 25, C1, dG, dB);
-    // conv1
-    colsum(dG, n * 25, C1, g + OB1, s);
-    tr(dB, n * 25, C1, C1, tA, s);
-    tr(nt->x1.as<uint16_t>(), n * 25, K1, K1, tB, s);
-    nn_gemm_nt(tA, tB, g + OW1, C1, K1, n25, n25, n25, K1, true, s);
+                       wscale, d[4], db[4], nt->loss.as<float>());
+    // through the layers' inputs; each product ends with the ReLU of the layer below
+    auto mask = [&](const DevBuf &a, int ldm, int l, int ldo) {
+        GemmEpi e;
+        e.m = static_cast<const uint16_t *>(a.ptr);
+        e.ldm = ldm;
+        e.o = db[l];
+        e.ldo = ldo;
+        return e;
+    };
+    nn_gemm_nt<EPI_MASK>(db[4], WT + OW5, d[3], n, F1, NO, NO, NO, F1, mask(nt->a4, F1, 3, F1), s);
+    nn_gemm_nt<EPI_MASK>(db[3], WT + OW4, d[2], n, C3, F1, F1, F1, C3, mask(nt->a3, F0, 2, C3), s);   // the side columns take none
+    nn_gemm_nt<EPI_MASK>(db[2], WT + OW3, d[1], n, K3, C3, C3, C3, K3, mask(nt->a2, K3, 1, K3), s);   // = d a2 [n*9][64]
+    nn_gemm_nt<EPI_F32>(db[1], WT + OW2, dF, n * 9, K2, C2, C2, C2, K2, GemmEpi(), s);                // d x2 [n*9][288]
+    hipLaunchKernelGGL(col2im2_kernel, dim3(nblk((size_t)n * 25 * C1)), dim3(256), 0, s, dF, nt->a1.as<uint16_t>(), n, d[0], db[0]);
+    // weights and biases of every layer
+    WgArgs a;
+    a.nl = 5;
+    a.blocks = 0;
+    a.partial = nt->part.as<float>();
+    const uint16_t *x[5] = {nt->x1.as<uint16_t>(), nt->x2.as<uint16_t>(), nt->a2.as<uint16_t>(), nt->a3.as<uint16_t>(), nt->a4.as<uint16_t>()};
+    const int per[5] = {25, 9, 1, 1, 1}, M[5] = {C1, C2, C3, F1, NO}, K[5] = {K1, K2, K3, F0, F1};
+    const int ow[5] = {OW1, OW2, OW3, OW4, OW5}, ob[5] = {OB1, OB2, OB3, OB4, OB5};
+    size_t poff = 0;
+    int most = 0;
+    for (int l = 0; l < 5; l++) {
+        const int rows = n * per[l];
+        int slice = (rows + WG_PARTS - 1) / WG_PARTS;
+        slice = (slice + 63) / 64 * 64;
+        const int parts = (rows + slice - 1) / slice;
+        a.l[l] = WgLayer{db[l], x[l], d[l], rows, M[l], K[l], K[l], parts, slice, a.blocks, ow[l], ob[l], poff};
+        a.blocks += parts * ((K[l] + 63) / 64);
+        poff += (size_t)parts * WN[l];
+        most = WN[l] > most ? WN[l] : most;
+    }
+    hipLaunchKernelGGL(wgrad_kernel, dim3(a.blocks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblk(most), 5), dim3(256), 0, s, a, nt->g.as<float>(), add ? 1 : 0);
     QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
 
-// gradient of the mean loss over all n ROIs (chunked) into g; *loss_out = mean loss
+// gradient of the mean loss over all n ROIs (chunked) into g; *loss_out = mean loss, h_grad the
+// gradient, through one pinned copy (either may be null)
 int net_gradient(qcs_net *nt, const qcs_params &p, const uint16_t *d_rois, const float *d_labels, int n, float *loss_out,
-                 hipStream_t s)
+                 float *h_grad, hipStream_t s)
 {
-    hipLaunchKernelGGL(fill0_kernel, dim3(nblk(NPARAM)), dim3(256), 0, s, nt->g.as<float>(), NPARAM);
-    hipLaunchKernelGGL(fill0_kernel, dim3(1), dim3(64), 0, s, nt->loss.as<float>(), 1);
     const float ws = 1.0f / (float)(n > 0 ? n : 1);
     for (int c0 = 0; c0 < n; c0 += CHUNK) {
         const int m = (n - c0) < CHUNK ? (n - c0) : CHUNK;
-        int rc = net_forward(nt, p, d_rois + (size_t)c0 * NR * (NR + 1), m, s);
+        int rc = net_forward(nt, p, d_rois + (size_t)c0 * NR * (NR + 1), m, c0 == 0 ? nt->loss.as<float>() : nullptr, s);
         if (rc) return rc;
-        if ((rc = net_backward(nt, d_labels + (size_t)c0 * NO, m, ws, s))) return rc;
+        if ((rc = net_backward(nt, d_labels + (size_t)c0 * NO, m, ws, c0 > 0, s))) return rc;
     }
-    if (loss_out) {
-        float *h = nt->pin.as<float>();
-        QCS_HIP(hipMemcpyAsync(h, nt->loss.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
-        QCS_HIP(hipStreamSynchronize(s));
-        *loss_out = h[0] * ws;
-    }
+    if (!loss_out && !h_grad) return QCS_OK;
+    float *h = nt->pin.as<float>();
+    if (loss_out) QCS_HIP(hipMemcpyAsync(h, nt->loss.ptr, sizeof(float), hipMemcpyDeviceToHost, s));
+    if (h_grad) QCS_HIP(hipMemcpyAsync(h + 16, nt->g.ptr, NPARAM * sizeof(float), hipMemcpyDeviceToHost, s));
+    QCS_HIP(hipStreamSynchronize(s));
+    if (loss_out) *loss_out = h[0] * ws;
+    if (h_grad) memcpy(h_grad, h + 16, NPARAM * sizeof(float));
     return QCS_OK;
 }
 
@@ -654,8 +593,12 @@ int qcs_net_destroy(qcs_net *nt)
 {
     if (!nt) return QCS_OK;
     DevBuf *b[] = {&nt->w, &nt->g, &nt->m, &nt->v, &nt->wb, &nt->wt, &nt->loss, &nt->x1, &nt->a1, &nt->x2, &nt->a2, &nt->a3,
-                   &nt->a4, &nt->side, &nt->norm, &nt->yo, &nt->Y, &nt->dF, &nt->dG, &nt->dB, &nt->tA, &nt->tB};
+                   &nt->a4, &nt->norm, &nt->yo, &nt->dF, &nt->part};
     for (auto *x : b) x->release();
+    for (int l = 0; l < 5; l++) {
+        nt->d[l].release();
+        nt->db[l].release();
+    }
     nt->pin.release();
     delete nt;
     return QCS_OK;
@@ -703,7 +646,7 @@ int qcs_net_forward_layers_dev(qcs_net *nt, const qcs_params *p, const uint16_t 
     hipStream_t s = (hipStream_t)stream;
     for (int c0 = 0; c0 < n; c0 += CHUNK) {
         const int m = (n - c0) < CHUNK ? (n - c0) : CHUNK;
-        int rc = net_forward(nt, *p, d_rois + (size_t)c0 * NR * (NR + 1), m, s);
+        int rc = net_forward(nt, *p, d_rois + (size_t)c0 * NR * (NR + 1), m, nullptr, s);
         if (rc) return rc;
         QCS_HIP(hipMemcpyAsync(d_out + (size_t)c0 * NO, nt->yo.ptr, (size_t)m * NO * 4, hipMemcpyDeviceToDevice, s));
         if (d_norm) QCS_HIP(hipMemcpyAsync(d_norm + (size_t)c0 * 2, nt->norm.ptr, (size_t)m * 8, hipMemcpyDeviceToDevice, s));
@@ -717,13 +660,7 @@ int qcs_net_grad_dev(qcs_net *nt, const qcs_params *p, const uint16_t *d_rois, c
     if (!nt || !p || n <= 0 || !d_rois || !d_labels) return fail(QCS_ERR_ARG, "invalid argument");
     if (p->ROISize != NR) return fail(QCS_ERR_ARG, "the warm-start network takes 7x7 ROIs");
     hipStream_t s = (hipStream_t)stream;
-    int rc = net_gradient(nt, *p, d_rois, d_labels, n, loss_out, s);
-    if (rc) return rc;
-    if (h_grad) {
-        QCS_HIP(hipStreamSynchronize(s));
-        QCS_HIP(hipMemcpy(h_grad, nt->g.ptr, NPARAM * 4, hipMemcpyDeviceToHost));
-    }
-    return QCS_OK;
+    return net_gradient(nt, *p, d_rois, d_labels, n, loss_out, h_grad, s);
 }
 
 int qcs_net_train_step_dev(qcs_net *nt, const qcs_params *p, const uint16_t *d_rois, const float *d_labels, int n, float lr,
@@ -732,7 +669,7 @@ int qcs_net_train_step_dev(qcs_net *nt, const qcs_params *p, const uint16_t *d_r
     if (!nt || !p || n <= 0 || !d_rois || !d_labels || !(lr > 0.0f)) return fail(QCS_ERR_ARG, "invalid argument");
     if (p->ROISize != NR) return fail(QCS_ERR_ARG, "the warm-start network takes 7x7 ROIs");
     hipStream_t s = (hipStream_t)stream;
-    int rc = net_gradient(nt, *p, d_rois, d_labels, n, loss_out, s);
+    int rc = net_gradient(nt, *p, d_rois, d_labels, n, loss_out, nullptr, s);
     if (rc) return rc;
     nt->steps++;
     const float b1 = 0.9f, b2 = 0.999f;
@@ -747,7 +684,7 @@ int qcs_net_train_step_dev(qcs_net *nt, const qcs_params *p, const uint16_t *d_r
 int qcs_dev_gemm_nt_bf16(const uint16_t *d_a, const uint16_t *d_b, float *d_c, int M, int N, int K, void *stream)
 {
     if (!d_a || !d_b || !d_c || M <= 0 || N <= 0 || K <= 0 || (K % 16) != 0) return fail(QCS_ERR_ARG, "invalid argument");
-    nn_gemm_nt(d_a, d_b, d_c, M, N, K, K, K, N, false, (hipStream_t)stream);
+    nn_gemm_nt<EPI_F32>(d_a, d_b, d_c, M, N, K, K, K, N, GemmEpi(), (hipStream_t)stream);
     QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
