@@ -530,70 +530,153 @@ __global__ void __launch_bounds__(256) var_reduce_kernel(ExtractConst c, const u
     }
 }
 
-// ---- 3. exclusive scan of int counts (3-pass) -----------------------------------------------
+// ---- 3. exclusive scan of int counts ----------------------------------------------------------
+// Items at and past *n_dev count as zero.  Up to SCAN_ONE items, one tile of 16 waves, are one launch
+// (4,096 items 3.7 us); more items take two, tile totals and then the tiles, each of which adds up the
+// totals before it: 20,480 items 9.3 us and 65,536 items 9.6 us, where one work-group walking the
+// tiles takes 13 and 35 us, and tile totals, their scan and an addition were three launches of 4 us.
 constexpr int SCAN_BLOCK = 256, SCAN_ITEMS = 16, SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
+constexpr int SCAN_ONE_T = 1024, SCAN_ONE = SCAN_ONE_T * SCAN_ITEMS;
 
-__device__ __forceinline__ int block_exclusive_scan(int v, int *sh)
+__device__ __forceinline__ int wave_inclusive_sum(int v)
 {
-    const int tid = threadIdx.x;
-    sh[tid] = v;
-    __syncthreads();
-    for (int off = 1; off < SCAN_BLOCK; off <<= 1) {
-        const int t = (tid >= off) ? sh[tid - off] : 0;
-        __syncthreads();
-        sh[tid] += t;
-        __syncthreads();
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(v, o, 64);
+        if (lane >= o) v += t;
     }
-    const int incl = sh[tid];
-    __syncthreads();
-    return incl - v;
+    return v;
 }
 
-__global__ void __launch_bounds__(SCAN_BLOCK) scan_tiles_kernel(const int *__restrict__ in, int n, int *__restrict__ out,
+// One tile of 16 items a thread over W waves: chunk c of the tile is 4 consecutive items a thread, so a
+// wave's loads cover whole lines.  v becomes each item's prefix within the tile; returns the tile's
+// sum.  sh: 4 W + 1 ints.
+template <int W>
+__device__ __forceinline__ int tile_exclusive_sum(int (&v)[4][4], int *sh)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int pre[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        const int s = (v[c][0] + v[c][1]) + (v[c][2] + v[c][3]);
+        const int incl = wave_inclusive_sum(s);
+        if (lane == 63) sh[c * W + w] = incl;
+        pre[c] = incl - s;
+    }
+    __syncthreads();
+    if (w == 0) {
+        const int t = lane < 4 * W ? sh[lane] : 0;
+        const int incl = wave_inclusive_sum(t);
+        if (lane < 4 * W) sh[lane] = incl - t;
+        if (lane == 63) sh[4 * W] = incl;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        int p = pre[c] + sh[c * W + w];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int x = v[c][k];
+            v[c][k] = p;
+            p += x;
+        }
+    }
+    return sh[4 * W];
+}
+
+template <int W>
+__device__ __forceinline__ void tile_load(int (&v)[4][4], const int *__restrict__ in, int base, int m)
+{
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = base + (c * W * 64 + (int)threadIdx.x) * 4 + k;
+            v[c][k] = i < m ? in[i] : 0;
+        }
+}
+
+template <int W>
+__device__ __forceinline__ void tile_store(const int (&v)[4][4], int *__restrict__ out, int base, int n, int add)
+{
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = base + (c * W * 64 + (int)threadIdx.x) * 4 + k;
+            if (i < n) out[i] = v[c][k] + add;
+        }
+}
+
+// where the grand total goes besides tile_sums[ntiles]: *out = (add: *out +) total
+struct ScanTotal {
+    int *out;
+    int add;
+};
+__device__ __forceinline__ void scan_put_total(const ScanTotal &t, int total)
+{
+    if (t.out) *t.out = t.add ? *t.out + total : total;
+}
+
+__global__ void __launch_bounds__(SCAN_ONE_T) scan_one_kernel(const int *__restrict__ in, int n, const int *__restrict__ n_dev,
+                                                              int *__restrict__ out, int *__restrict__ total, ScanTotal tot)
+{
+    constexpr int W = SCAN_ONE_T / 64;
+    __shared__ int sh[4 * W + 1];
+    int v[4][4];
+    tile_load<W>(v, in, 0, n_dev ? min(*n_dev, n) : n);
+    const int all = tile_exclusive_sum<W>(v, sh);
+    tile_store<W>(v, out, 0, n, 0);
+    if (threadIdx.x == 0) {
+        *total = all;
+        scan_put_total(tot, all);
+    }
+}
+
+// sum of v over a work-group of SCAN_BLOCK threads; sh: one int a wave
+__device__ __forceinline__ int block_sum(int v, int *sh)
+{
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = 0;
+#pragma unroll
+    for (int w = 0; w < SCAN_BLOCK / 64; w++) v += sh[w];
+    return v;
+}
+
+__global__ void __launch_bounds__(SCAN_BLOCK) scan_tiles_kernel(const int *__restrict__ in, int n, const int *__restrict__ n_dev,
                                                                 int *__restrict__ tile_sums)
 {
-    __shared__ int sh[SCAN_BLOCK];
-    const int base = blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
-    int v[SCAN_ITEMS], s = 0;
+    __shared__ int sh[SCAN_BLOCK / 64];
+    const int m = n_dev ? min(*n_dev, n) : n;
+    int v[4][4], s = 0;
+    tile_load<SCAN_BLOCK / 64>(v, in, blockIdx.x * SCAN_TILE, m);
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        v[k] = (base + k < n) ? in[base + k] : 0;
-        s += v[k];
-    }
-    int run = block_exclusive_scan(s, sh);
-#pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        if (base + k < n) out[base + k] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == SCAN_BLOCK - 1) tile_sums[blockIdx.x] = run;
+    for (int c = 0; c < 4; c++) s += (v[c][0] + v[c][1]) + (v[c][2] + v[c][3]);
+    s = block_sum(s, sh);
+    if (threadIdx.x == 0) tile_sums[blockIdx.x] = s;
 }
 
-// single work-group scan of the tile sums (ntiles <= SCAN_TILE), total at tile_sums[ntiles]
-__global__ void __launch_bounds__(SCAN_BLOCK) scan_sums_kernel(int *__restrict__ tile_sums, int ntiles)
+// total at tile_sums[ntiles]
+__global__ void __launch_bounds__(SCAN_BLOCK) scan_apply_kernel(const int *__restrict__ in, int n, const int *__restrict__ n_dev,
+                                                                int *__restrict__ out, int *__restrict__ tile_sums, int ntiles,
+                                                                ScanTotal tot)
 {
-    __shared__ int sh[SCAN_BLOCK];
-    const int base = threadIdx.x * SCAN_ITEMS;
-    int v[SCAN_ITEMS], s = 0;
-#pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        v[k] = (base + k < ntiles) ? tile_sums[base + k] : 0;
-        s += v[k];
+    constexpr int W = SCAN_BLOCK / 64;
+    __shared__ int sh[4 * W + 1], shb[W];
+    const int m = n_dev ? min(*n_dev, n) : n;
+    int v[4][4], s = 0;
+    tile_load<W>(v, in, blockIdx.x * SCAN_TILE, m);
+    for (int t = threadIdx.x; t < (int)blockIdx.x; t += SCAN_BLOCK) s += tile_sums[t];
+    const int before = block_sum(s, shb);
+    const int all = tile_exclusive_sum<W>(v, sh);
+    tile_store<W>(v, out, blockIdx.x * SCAN_TILE, n, before);
+    if (threadIdx.x == 0 && (int)blockIdx.x == ntiles - 1) {
+        tile_sums[ntiles] = before + all;
+        scan_put_total(tot, before + all);
     }
-    int run = block_exclusive_scan(s, sh);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        if (base + k < ntiles) tile_sums[base + k] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == SCAN_BLOCK - 1) tile_sums[ntiles] = run;
-}
-
-__global__ void __launch_bounds__(256) scan_add_kernel(int *__restrict__ out, int n, const int *__restrict__ tile_sums)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] += tile_sums[i / SCAN_TILE];
 }
 
 // ---- 4. per-batch bookkeeping ----------------------------------------------------------------
@@ -774,33 +857,37 @@ void fill_async(int *p, size_t n, int v, hipStream_t s)
 
 int scan_tile_count(size_t n) { return (int)((n + SCAN_TILE - 1) / SCAN_TILE); }
 
-int scan_exclusive(const int *in, int n, int *out, int *tile_sums, hipStream_t s)
+int scan_exclusive(const int *in, int n, int *out, int *tile_sums, hipStream_t s, const int *n_dev, int *total, bool add)
 {
     if (n <= 0) return QCS_OK;
     const int ntiles = scan_tile_count((size_t)n);
     if (ntiles > SCAN_TILE) return fail(QCS_ERR_ARG, "scan of %d items exceeds the supported size", n);
-    hipLaunchKernelGGL(scan_tiles_kernel, dim3(ntiles), dim3(SCAN_BLOCK), 0, s, in, n, out, tile_sums);
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(SCAN_BLOCK), 0, s, tile_sums, ntiles);
-    hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, out, n, tile_sums);
+    const ScanTotal t{total, add ? 1 : 0};
+    if (n <= SCAN_ONE) {
+        hipLaunchKernelGGL(scan_one_kernel, dim3(1), dim3(SCAN_ONE_T), 0, s, in, n, n_dev, out, tile_sums + ntiles, t);
+    } else {
+        hipLaunchKernelGGL(scan_tiles_kernel, dim3(ntiles), dim3(SCAN_BLOCK), 0, s, in, n, n_dev, tile_sums);
+        hipLaunchKernelGGL(scan_apply_kernel, dim3(ntiles), dim3(SCAN_BLOCK), 0, s, in, n, n_dev, out, tile_sums, ntiles, t);
+    }
     QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
 
 __global__ void __launch_bounds__(256) scatter_kernel(const int *__restrict__ flags, const int *__restrict__ offs, int n,
                                                       const int *__restrict__ src, const int *__restrict__ base_dev,
-                                                      int base_const, int *__restrict__ out)
+                                                      int base_const, int *__restrict__ out, const int *__restrict__ n_dev)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n || !flags[j]) return;
+    if (j >= n || (n_dev && j >= *n_dev) || !flags[j]) return;
     const int base = base_dev ? *base_dev : base_const;
     out[base + offs[j]] = src ? src[j] : j;
 }
 
 int compact_scatter(const int *flags, const int *offs, int n, const int *src, const int *base_dev, int base_const, int *out,
-                    hipStream_t s)
+                    hipStream_t s, const int *n_dev)
 {
     if (n <= 0) return QCS_OK;
-    hipLaunchKernelGGL(scatter_kernel, dim3((n + 255) / 256), dim3(256), 0, s, flags, offs, n, src, base_dev, base_const, out);
+    hipLaunchKernelGGL(scatter_kernel, dim3((n + 255) / 256), dim3(256), 0, s, flags, offs, n, src, base_dev, base_const, out, n_dev);
     QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
@@ -891,9 +978,7 @@ static int extract_candidates(qcs_ctx *ctx, const qcs_params &p, const uint16_t 
     else
         hipLaunchKernelGGL((walk_kernel<1, false>), wgrid, dim3(64), 0, s, d_frames, c, var_sums, tvbuf, cand, mark, row_count);
     QCS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(scan_tiles_kernel, dim3(ntiles), dim3(SCAN_BLOCK), 0, s, row_count, (int)nrows, row_off, tile_sums);
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(SCAN_BLOCK), 0, s, tile_sums, ntiles);
-    hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)((nrows + 255) / 256)), dim3(256), 0, s, row_off, (int)nrows, tile_sums);
+    if ((rc = scan_exclusive(row_count, (int)nrows, row_off, tile_sums, s))) return rc;
     hipLaunchKernelGGL(batch_kernel, dim3(1), dim3(64), 0, s, c, row_off, tile_sums, (int)nrows, ntiles, info);
     hipLaunchKernelGGL(emit_kernel, dim3((unsigned)((nrows + EMIT_WAVES - 1) / EMIT_WAVES)), dim3(64 * EMIT_WAVES), 0, s, c, cand,
                        row_off, row_count, (int)nrows, info, xyb);

@@ -183,25 +183,33 @@ int crlb_launch(const qcs_params &p, float *d_loc, int n, const int *d_n, hipStr
 //   2E list  = ROIs with WLE type MultiFit, in index order, then rejected 1E fits with SNR > 6
 //   3E list  = rejected first emitters of the 2E stage, in 2E-list order (2D only)
 //   appended = accepted second emitters of the 2E stage, then of the 3E stage, in list order
-// All counts stay on the device; one read-back at the end.
-
-__global__ void cascade_classify_kernel(const float *__restrict__ wle, int n, int *__restrict__ f1, int *__restrict__ f2)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int mt = (int)wle[(size_t)i * QCS_WLE_FLOATS + QCS_WLE_FLUOTYPE];
-    f1[i] = (mt <= QCS_MOLTYPE_WLEFIT) ? 1 : 0;
-    f2[i] = (mt <= QCS_MOLTYPE_WLEFIT) ? 0 : 1;
-}
+// All counts stay on the device; one read-back at the end.  The list building is launches, not
+// work: 19 of them beside the fits (13 up to 16,384 ROIs), where a clear, a scan, a count and a tail
+// clear per flag array were 48 (20,480 ROIs: 1056 -> 959 us).
 
 // cnt layout: [0] n1, [1] n2 classified, [2] n2 total, [3] n3, [4] seconds from 2E, [5] seconds
 // from 3E, [6] rejected, [7] rows, [8] loc_cap
-__global__ void cascade_count_kernel(const int *__restrict__ tile_sums, int ntiles, int *__restrict__ cnt, int slot, int mode)
+__global__ void cascade_classify_kernel(const float *__restrict__ wle, int n, int *__restrict__ f1, int *__restrict__ rr,
+                                        int *__restrict__ cnt, int loc_cap)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const int total = tile_sums[ntiles];
-    if (mode == 0) cnt[slot] = total;
-    else if (mode == 1) cnt[slot] += total;   // accumulate (2E list = classified + re-routed)
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x < 16) cnt[threadIdx.x] = threadIdx.x == 8 ? loc_cap : 0;
+    if (i >= n) return;
+    const int mt = (int)wle[(size_t)i * QCS_WLE_FLOATS + QCS_WLE_FLUOTYPE];
+    f1[i] = (mt <= QCS_MOLTYPE_WLEFIT) ? 1 : 0;
+    rr[i] = 0;
+}
+
+// the 1E list and the classified part of the 2E list (the others), both in index order, with their counts
+__global__ void __launch_bounds__(256) cascade_lists_kernel(const int *__restrict__ f1, const int *__restrict__ offs, int n,
+                                                            int *__restrict__ list1, int *__restrict__ list2, int *__restrict__ cnt)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) cnt[1] = cnt[2] = n - cnt[0];
+    if (i >= n) return;
+    const int o = offs[i];
+    if (f1[i]) list1[o] = i;
+    else list2[i - o] = i;
 }
 
 __global__ void cascade_rows_kernel(int n, int *__restrict__ cnt)
@@ -229,15 +237,6 @@ __global__ void __launch_bounds__(256) append_kernel(const int *__restrict__ fla
     dst[0] = src[0];
     dst[1] = src[1];
     dst[2] = src[2];
-}
-
-__global__ void cascade_set_kernel(int *p, int v) { *p = v; }
-
-// flags of entries j >= *n_list are cleared so a scan over n entries counts only the list
-__global__ void clear_tail_kernel(int *__restrict__ f, int n, const int *__restrict__ n_list)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < n && j >= *n_list) f[j] = 0;
 }
 
 size_t cascade_scratch_bytes(int n)
@@ -270,10 +269,9 @@ int fit_cascade_launch(const qcs_params &p, Timer *tm, const uint16_t *d_rois, c
                        int loc_cap, const CascadeBufs &b, hipStream_t s)
 {
     const bool as3d = (p.LocType == QCS_LOCTYPE_AS3D);
-    const int ntiles = scan_tile_count((size_t)n);
     int rc;
     int *list1 = b.list1, *list2 = b.list2, *list3 = b.list3;
-    int *f1 = b.flag, *f2 = f1 + n, *rr = f2 + n, *fs2 = rr + n, *ff2 = fs2 + n, *fs3 = ff2 + n;
+    int *f1 = b.flag, *rr = f1 + 2 * n, *fs2 = rr + n, *ff2 = fs2 + n, *fs3 = ff2 + n;
     int *offs = fs3 + n, *tsum = offs + n;
     int *ff3 = f1;   // f1 is free again once the 1E list is built
     float *sec2 = b.rows, *sec3 = sec2 + (size_t)QCS_REC_FLOATS * n;
@@ -283,57 +281,34 @@ int fit_cascade_launch(const qcs_params &p, Timer *tm, const uint16_t *d_rois, c
     auto tb = [&](hipEvent_t *ev) { *ev = nullptr; return tm ? timer_begin(*tm, s, ev) : QCS_OK; };
     auto te = [&](int cat, hipEvent_t ev) { return tm ? timer_end(*tm, cat, s, ev, n) : QCS_OK; };
 
-    fill_async(cnt, 16, 0, s);
-    hipLaunchKernelGGL(cascade_set_kernel, dim3(1), dim3(1), 0, s, cnt + 8, loc_cap);
-    fill_async(rr, n, 0, s);
-    fill_async(fs2, n, 0, s);
-    fill_async(ff2, n, 0, s);
-    fill_async(fs3, n, 0, s);
-    hipLaunchKernelGGL(cascade_classify_kernel, g, dim3(256), 0, s, d_wle, n, f1, f2);
-    // 1E list and classified part of the 2E list
-    if ((rc = scan_exclusive(f1, n, offs, tsum, s)) || (rc = compact_scatter(f1, offs, n, nullptr, nullptr, 0, list1, s)))
-        return rc;
-    hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 0, 0);
-    if ((rc = scan_exclusive(f2, n, offs, tsum, s)) || (rc = compact_scatter(f2, offs, n, nullptr, nullptr, 0, list2, s)))
-        return rc;
-    hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 1, 0);
-    hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 2, 0);
+    hipLaunchKernelGGL(cascade_classify_kernel, g, dim3(256), 0, s, d_wle, n, f1, rr, cnt, loc_cap);
+    if ((rc = scan_exclusive(f1, n, offs, tsum, s, nullptr, cnt + 0))) return rc;
+    hipLaunchKernelGGL(cascade_lists_kernel, g, dim3(256), 0, s, f1, offs, n, list1, list2, cnt);
     // one-emitter stage; rejected fits with SNR > 6 flag themselves in rr
     hipEvent_t ev;
     if ((rc = tb(&ev))) return rc;
     if ((rc = fit_launch_1e(p, d_rois, d_wle, list1, n, cnt + 0, d_loc, rr, s))) return rc;
     if ((rc = te(TM_FIT1E, ev))) return rc;
     // re-routed ROIs join the 2E list after the classified ones, in index order
-    if ((rc = scan_exclusive(rr, n, offs, tsum, s)) || (rc = compact_scatter(rr, offs, n, nullptr, cnt + 1, 0, list2, s)))
+    if ((rc = scan_exclusive(rr, n, offs, tsum, s, nullptr, cnt + 2, true)) ||
+        (rc = compact_scatter(rr, offs, n, nullptr, cnt + 1, 0, list2, s)))
         return rc;
-    hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 2, 1);
-    // two-emitter stage
+    // two-emitter stage (every entry of its list writes fs2 and ff2)
     if ((rc = tb(&ev))) return rc;
     if ((rc = fit_launch_me(p, as3d ? MODEL_AS3D2E : MODEL_2E, d_rois, d_wle, list2, n, cnt + 2, d_loc, sec2, fs2, ff2, s)))
         return rc;
     if ((rc = te(TM_FITME, ev))) return rc;
-    hipLaunchKernelGGL(clear_tail_kernel, g, dim3(256), 0, s, fs2, n, cnt + 2);
-    hipLaunchKernelGGL(clear_tail_kernel, g, dim3(256), 0, s, ff2, n, cnt + 2);
-    if ((rc = scan_exclusive(fs2, n, offs, tsum, s))) return rc;
+    if ((rc = scan_exclusive(fs2, n, offs, tsum, s, cnt + 2, cnt + 4))) return rc;
     hipLaunchKernelGGL(append_kernel, g, dim3(256), 0, s, fs2, offs, cnt + 2, sec2, cnt, -1, n, loc_cap, d_loc);
-    hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 4, 0);
-    if ((rc = scan_exclusive(ff2, n, offs, tsum, s))) return rc;
-    if (as3d) {
-        hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 6, 0);
-    } else {
-        if ((rc = compact_scatter(ff2, offs, n, list2, nullptr, 0, list3, s))) return rc;
-        hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 3, 0);
-        fill_async(ff3, n, 0, s);
+    if ((rc = scan_exclusive(ff2, n, offs, tsum, s, cnt + 2, cnt + (as3d ? 6 : 3)))) return rc;
+    if (!as3d) {
+        if ((rc = compact_scatter(ff2, offs, n, list2, nullptr, 0, list3, s, cnt + 2))) return rc;
         if ((rc = tb(&ev))) return rc;
         if ((rc = fit_launch_me(p, MODEL_3E, d_rois, d_wle, list3, n, cnt + 3, d_loc, sec3, fs3, ff3, s))) return rc;
         if ((rc = te(TM_FITME, ev))) return rc;
-        hipLaunchKernelGGL(clear_tail_kernel, g, dim3(256), 0, s, fs3, n, cnt + 3);
-        hipLaunchKernelGGL(clear_tail_kernel, g, dim3(256), 0, s, ff3, n, cnt + 3);
-        if ((rc = scan_exclusive(fs3, n, offs, tsum, s))) return rc;
+        if ((rc = scan_exclusive(fs3, n, offs, tsum, s, cnt + 3, cnt + 5))) return rc;
         hipLaunchKernelGGL(append_kernel, g, dim3(256), 0, s, fs3, offs, cnt + 3, sec3, cnt, 4, n, loc_cap, d_loc);
-        hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 5, 0);
-        if ((rc = scan_exclusive(ff3, n, offs, tsum, s))) return rc;
-        hipLaunchKernelGGL(cascade_count_kernel, dim3(1), dim3(1), 0, s, tsum, ntiles, cnt, 6, 0);
+        if ((rc = scan_exclusive(ff3, n, offs, tsum, s, cnt + 3, cnt + 6))) return rc;
     }
     hipLaunchKernelGGL(cascade_rows_kernel, dim3(1), dim3(1), 0, s, n, cnt);
     QCS_HIP(hipGetLastError());

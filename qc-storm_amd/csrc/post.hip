@@ -8,9 +8,8 @@
 //   FluoRenderWithPrec_3D  DLL/ImgRender/ImageRender_3d.cu:60-147
 //
 // Sorted compaction: the reference launches one kernel per frame and appends with an atomic
-// counter (within-frame order arbitrary, O(frames x rows) work).  Here the kept rows are compacted
-// in row order (scan), then stably radix-sorted by frame (sort.hip), so rows of one frame keep their
-// original order.  Rendering splats each localization's 7 x 7 Gaussian with float atomics, as the
+// counter (within-frame order arbitrary, O(frames x rows) work).  Here the kept rows are stably
+// radix-sorted by frame (sort.hip), so rows of one frame keep their original order.  Rendering splats each localization's 7 x 7 Gaussian with float atomics, as the
 // reference does, but into LDS: localizations are binned by 64 x 64 tile of the SR image (a
 // footprint that straddles a tile edge is listed in each tile it touches), one work-group
 // accumulates a tile with LDS atomics and then adds it to the image with one coalesced
@@ -22,27 +21,6 @@
 
 namespace qcs {
 
-// float -> int truncation with NaN -> 0 and saturation (the CUDA conversion the reference relies on)
-__device__ __forceinline__ int f2i_sat(float v)
-{
-    if (v != v) return 0;
-    if (v >= 2147483647.0f) return 2147483647;
-    if (v <= -2147483648.0f) return (-2147483647 - 1);
-    return (int)v;
-}
-
-__global__ void __launch_bounds__(256) keep_sorted_kernel(const float *__restrict__ loc, int n, int first, int end,
-                                                          int *__restrict__ flag, unsigned *__restrict__ key)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float *r = loc + (size_t)i * QCS_REC_FLOATS;
-    const int pp = f2i_sat(r[QCS_POS_PPHO]), fr = f2i_sat(r[QCS_POS_FRME]);
-    const bool k = ((float)pp > 1.0f) && fr >= first && fr <= end;
-    flag[i] = k ? 1 : 0;
-    key[i] = k ? (unsigned)(fr - first) : 0u;
-}
-
 __global__ void __launch_bounds__(256) keep_any_kernel(const float *__restrict__ loc, int n, int *__restrict__ flag)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -50,24 +28,13 @@ __global__ void __launch_bounds__(256) keep_any_kernel(const float *__restrict__
     flag[i] = (loc[(size_t)i * QCS_REC_FLOATS + QCS_POS_PPHO] > 1.0f) ? 1 : 0;
 }
 
-// gather kept rows: keys_out[pos] = key, idx_out[pos] = row
-__global__ void __launch_bounds__(256) gather_keys_kernel(const int *__restrict__ flag, const int *__restrict__ offs,
-                                                          const unsigned *__restrict__ key, int n,
-                                                          unsigned *__restrict__ kout, int *__restrict__ iout)
+__global__ void __launch_bounds__(256) copy_kept_kernel(const float *__restrict__ loc, int n, const int *__restrict__ flag,
+                                                        const int *__restrict__ offs, float *__restrict__ out)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n || !flag[i]) return;
-    kout[offs[i]] = key[i];
-    iout[offs[i]] = i;
-}
-
-__global__ void __launch_bounds__(256) copy_rows_kernel(const float *__restrict__ loc, const int *__restrict__ idx,
-                                                        const int *__restrict__ m_dev, float *__restrict__ out)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= *m_dev) return;
-    const float4 *src = reinterpret_cast<const float4 *>(loc + (size_t)idx[j] * QCS_REC_FLOATS);
-    float4 *dst = reinterpret_cast<float4 *>(out + (size_t)j * QCS_REC_FLOATS);
+    const float4 *src = reinterpret_cast<const float4 *>(loc + (size_t)i * QCS_REC_FLOATS);
+    float4 *dst = reinterpret_cast<float4 *>(out + (size_t)offs[i] * QCS_REC_FLOATS);
     dst[0] = src[0];
     dst[1] = src[1];
     dst[2] = src[2];
@@ -130,10 +97,11 @@ __device__ __forceinline__ void splat_tiles(const Splat &q, int &tx0, int &tx1, 
 // {pp, rs, fx, fy} and {z, (iy - y0) << 16 | (ix - x0) & 0xffff (tile-relative), 0, 0}.
 constexpr int RENT = 2;   // float4 words per entry
 
-// pass 1 (cursor == null): localizations per tile; pass 2: the per-tile lists of prepared entries
+// pass 1 (ent == null): localizations per tile; pass 2: the per-tile lists of prepared entries, which
+// count tcnt down again (the tile kernel takes the counts from the offsets)
 __global__ void __launch_bounds__(256) render_bin_kernel(const float *__restrict__ loc, int n, RenderConst c,
                                                          int *__restrict__ tcnt, const int *__restrict__ toff,
-                                                         int *__restrict__ cursor, float4 *__restrict__ ent)
+                                                         float4 *__restrict__ ent)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -144,11 +112,11 @@ __global__ void __launch_bounds__(256) render_bin_kernel(const float *__restrict
     for (int ty = ty0; ty <= ty1; ty++)
         for (int tx = tx0; tx <= tx1; tx++) {
             const int t = ty * c.tiles_x + tx;
-            if (!cursor) {
+            if (!ent) {
                 atomicAdd(&tcnt[t], 1);
                 continue;
             }
-            const size_t e = (size_t)(toff[t] + atomicAdd(&cursor[t], 1)) * RENT;
+            const size_t e = (size_t)(toff[t] + atomicSub(&tcnt[t], 1) - 1) * RENT;
             const int rx = q.ix - tx * RTILE, ry = q.iy - ty * RTILE;   // within [-3, RTILE + 2]
             ent[e] = make_float4(q.pp, q.rs, q.fx, q.fy);
             ent[e + 1] = make_float4(q.z, __int_as_float((int)(((unsigned)ry << 16) | ((unsigned)rx & 0xffffu))), 0.0f, 0.0f);
@@ -166,7 +134,7 @@ constexpr int RBLK = 256;
 constexpr int RVEC = RTILE * RTILE / (4 * RBLK);   // float4 image words per thread
 constexpr int RSTR = RTILE;   // LDS row stride of the tile accumulators
 template <bool ZON, bool FRESH>
-__global__ void __launch_bounds__(RBLK) render_tile_kernel(RenderConst c, const int *__restrict__ tcnt, const int *__restrict__ toff,
+__global__ void __launch_bounds__(RBLK) render_tile_kernel(RenderConst c, const int *__restrict__ toff,
                                                            const float4 *__restrict__ ent, float *__restrict__ img,
                                                            float *__restrict__ zimg)
 {
@@ -177,7 +145,7 @@ __global__ void __launch_bounds__(RBLK) render_tile_kernel(RenderConst c, const 
     __shared__ float s_z[ZON ? RBLK : 1];
     __shared__ int s_xy[RBLK];
     const int t = blockIdx.x;
-    const int cnt = tcnt[t], first = toff[t];
+    const int first = toff[t], cnt = toff[t + 1] - first;
     if (!FRESH && cnt == 0) return;   // uniform over the work-group
     const int x0 = (t % c.tiles_x) * RTILE, y0 = (t / c.tiles_x) * RTILE;
     const bool aligned = ((reinterpret_cast<uintptr_t>(img) | (ZON ? reinterpret_cast<uintptr_t>(zimg) : 0)) & 15) == 0;
@@ -334,27 +302,26 @@ int render_launch(qcs_ctx *ctx, const float *d_loc, int n, float *d_img, float *
     const size_t ntile = (size_t)c.tiles_x * c.tiles_y;
     if (ntile > (size_t)INT32_MAX / 8 || (size_t)n * 4 > (size_t)INT32_MAX) return fail(QCS_ERR_ARG, "SR image or row count too large");
     const int nst = scan_tile_count(ntile);
-    // tile counts, offsets (+ scan sums), cursors, then the entries (16-byte aligned; a footprint
-    // touches <= 4 tiles)
-    const size_t head = (ntile * 3 + (size_t)nst + 1 + 3) & ~(size_t)3;
+    // tile counts, offsets (one more than tiles), scan sums, then the entries (16-byte aligned; a
+    // footprint touches <= 4 tiles)
+    const size_t head = (ntile * 2 + 1 + (size_t)nst + 1 + 3) & ~(size_t)3;
     const size_t words = head + (size_t)n * 4 * RENT * 4;
     int rc;
     if ((rc = ctx->rn_buf.ensure(words * sizeof(int)))) return rc;
-    int *tcnt = ctx->rn_buf.as<int>(), *toff = tcnt + ntile, *tsum = toff + ntile, *cursor = tsum + nst + 1;
+    int *tcnt = ctx->rn_buf.as<int>(), *toff = tcnt + ntile, *tsum = toff + ntile + 1;
     float4 *ent = reinterpret_cast<float4 *>(ctx->rn_buf.as<int>() + head);
     fill_async(tcnt, ntile, 0, s);
-    fill_async(cursor, ntile, 0, s);
     const dim3 g1((n + 255) / 256), b1(256);
-    hipLaunchKernelGGL(render_bin_kernel, g1, b1, 0, s, d_loc, n, c, tcnt, nullptr, nullptr, nullptr);
-    if ((rc = scan_exclusive(tcnt, (int)ntile, toff, tsum, s))) return rc;
-    hipLaunchKernelGGL(render_bin_kernel, g1, b1, 0, s, d_loc, n, c, tcnt, toff, cursor, ent);
+    hipLaunchKernelGGL(render_bin_kernel, g1, b1, 0, s, d_loc, n, c, tcnt, nullptr, nullptr);
+    if ((rc = scan_exclusive(tcnt, (int)ntile, toff, tsum, s, nullptr, toff + ntile))) return rc;
+    hipLaunchKernelGGL(render_bin_kernel, g1, b1, 0, s, d_loc, n, c, tcnt, toff, ent);
     const dim3 tg((unsigned)ntile), tb(RBLK);
     if (c.is3d && d_zimg) {
-        if (fresh) hipLaunchKernelGGL((render_tile_kernel<true, true>), tg, tb, 0, s, c, tcnt, toff, ent, d_img, d_zimg);
-        else hipLaunchKernelGGL((render_tile_kernel<true, false>), tg, tb, 0, s, c, tcnt, toff, ent, d_img, d_zimg);
+        if (fresh) hipLaunchKernelGGL((render_tile_kernel<true, true>), tg, tb, 0, s, c, toff, ent, d_img, d_zimg);
+        else hipLaunchKernelGGL((render_tile_kernel<true, false>), tg, tb, 0, s, c, toff, ent, d_img, d_zimg);
     } else {
-        if (fresh) hipLaunchKernelGGL((render_tile_kernel<false, true>), tg, tb, 0, s, c, tcnt, toff, ent, d_img, nullptr);
-        else hipLaunchKernelGGL((render_tile_kernel<false, false>), tg, tb, 0, s, c, tcnt, toff, ent, d_img, nullptr);
+        if (fresh) hipLaunchKernelGGL((render_tile_kernel<false, true>), tg, tb, 0, s, c, toff, ent, d_img, nullptr);
+        else hipLaunchKernelGGL((render_tile_kernel<false, false>), tg, tb, 0, s, c, toff, ent, d_img, nullptr);
     }
     QCS_HIP(hipGetLastError());
     return QCS_OK;
@@ -380,41 +347,19 @@ extern "C" int qcs_compact_sorted_dev(qcs_ctx *c, const float *d_loc, int n, int
     if (!c || n < 0 || (n > 0 && (!d_loc || !d_out))) return fail(QCS_ERR_ARG, "invalid argument");
     if (n == 0 || end < first) return QCS_OK;
     hipStream_t s = (hipStream_t)stream;
-    const int ntiles = scan_tile_count((size_t)n);
-    // flag, offsets, tile sums, keys in/out, indices; sort workspace
-    const size_t words = (size_t)n * 5 + ntiles + 1;
+    if (n > 1 << 24) return fail(QCS_ERR_ARG, "compaction of %d rows exceeds the supported size", n);
     int rc;
-    if ((rc = c->fit_flag.ensure(sizeof(int) * words)) || (rc = c->fit_rows.ensure(sizeof(int) * radix_sort_tmp_ints(n))) ||
-        (rc = c->fit_idx1.ensure(sizeof(int) * (size_t)n)) || (rc = c->fit_cnt.ensure(64)) || (rc = c->pin_cnt.ensure(64)))
+    if ((rc = c->fit_rows.ensure(sizeof(int) * sort_rows_tmp_ints(n, first, end))) || (rc = c->fit_cnt.ensure(64)) ||
+        (rc = c->pin_cnt.ensure(64)))
         return rc;
-    int *flag = c->fit_flag.as<int>(), *offs = flag + n, *tsum = offs + n;
-    unsigned *key = reinterpret_cast<unsigned *>(tsum + ntiles + 1), *kin = key + n, *kout = kin + n;
-    int *iin = c->fit_idx1.as<int>();
-    int *iout = flag;   // flag is dead after the gather
-    const dim3 g((n + 255) / 256);
+    int *d_m = c->fit_cnt.as<int>(), *h = c->pin_cnt.as<int>();
     hipEvent_t ev;
     if ((rc = timer_begin(c->timer, s, &ev))) return rc;
-    hipLaunchKernelGGL(keep_sorted_kernel, g, dim3(256), 0, s, d_loc, n, first, end, flag, key);
-    if ((rc = scan_exclusive(flag, n, offs, tsum, s))) return rc;
-    hipLaunchKernelGGL(gather_keys_kernel, g, dim3(256), 0, s, flag, offs, key, n, kin, iin);
-    QCS_HIP(hipGetLastError());
-    int *h = c->pin_cnt.as<int>();
-    QCS_HIP(hipMemcpyAsync(h, tsum + ntiles, sizeof(int), hipMemcpyDeviceToHost, s));
-    QCS_HIP(hipStreamSynchronize(s));
-    const int m = h[0];
-    if (m > 0) {
-        int bits = 1;
-        while (bits < 32 && ((unsigned)(end - first) >> bits) != 0) bits++;
-        unsigned *kres;
-        int *ires;
-        if ((rc = radix_sort_pairs_u32(kin, iin, kout, iout, m, bits, c->fit_rows.as<int>(), s, &kres, &ires))) return rc;
-        fill_async(c->fit_cnt.as<int>(), 1, m, s);
-        hipLaunchKernelGGL(copy_rows_kernel, dim3((m + 255) / 256), dim3(256), 0, s, d_loc, ires, c->fit_cnt.as<int>(), d_out);
-        QCS_HIP(hipGetLastError());
-    }
+    if ((rc = sort_rows_by_frame(d_loc, n, first, end, d_out, d_m, c->fit_rows.as<int>(), s))) return rc;
     if ((rc = timer_end(c->timer, TM_COMPACT, s, ev, n))) return rc;
+    QCS_HIP(hipMemcpyAsync(h, d_m, sizeof(int), hipMemcpyDeviceToHost, s));
     QCS_HIP(hipStreamSynchronize(s));
-    if (n_out) *n_out = m;
+    if (n_out) *n_out = h[0];
     return QCS_OK;
 }
 
@@ -426,15 +371,11 @@ extern "C" int qcs_compact_dev(qcs_ctx *c, const float *d_loc, int n, float *d_o
     hipStream_t s = (hipStream_t)stream;
     const int ntiles = scan_tile_count((size_t)n);
     int rc;
-    if ((rc = c->fit_flag.ensure(sizeof(int) * ((size_t)n * 2 + ntiles + 1))) || (rc = c->fit_idx1.ensure(sizeof(int) * (size_t)n)) ||
-        (rc = c->pin_cnt.ensure(64)))
-        return rc;
+    if ((rc = c->fit_flag.ensure(sizeof(int) * ((size_t)n * 2 + ntiles + 1))) || (rc = c->pin_cnt.ensure(64))) return rc;
     int *flag = c->fit_flag.as<int>(), *offs = flag + n, *tsum = offs + n;
-    int *idx = c->fit_idx1.as<int>();
     hipLaunchKernelGGL(keep_any_kernel, dim3((n + 255) / 256), dim3(256), 0, s, d_loc, n, flag);
     if ((rc = scan_exclusive(flag, n, offs, tsum, s))) return rc;
-    if ((rc = compact_scatter(flag, offs, n, nullptr, nullptr, 0, idx, s))) return rc;
-    hipLaunchKernelGGL(copy_rows_kernel, dim3((n + 255) / 256), dim3(256), 0, s, d_loc, idx, tsum + ntiles, d_out);
+    hipLaunchKernelGGL(copy_kept_kernel, dim3((n + 255) / 256), dim3(256), 0, s, d_loc, n, flag, offs, d_out);
     QCS_HIP(hipGetLastError());
     int *h = c->pin_cnt.as<int>();
     QCS_HIP(hipMemcpyAsync(h, tsum + ntiles, sizeof(int), hipMemcpyDeviceToHost, s));

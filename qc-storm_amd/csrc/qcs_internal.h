@@ -96,23 +96,27 @@ int noalloc_scratch_init(int device);
 int render_launch(qcs_ctx *ctx, const float *d_loc, int n, float *d_img, float *d_zimg, bool fresh, hipStream_t s);
 int max_disp_launch(const float *d_img, size_t npx, int *d_out, hipStream_t s);
 
-// device utilities (extract.hip): exclusive scan of n ints (total at tile_sums[ntiles]),
-// constant fill, stable compaction out[base + k] = src ? src[j] : j for flagged j.
+// device utilities (extract.hip): exclusive scan of n ints (total at tile_sums[ntiles], and set in or
+// added to *total where given; with n_dev the items from *n_dev on count as zero),
+// constant fill, stable compaction out[base + k] = src ? src[j] : j for flagged j (< *n_dev).
 int scan_tile_count(size_t n);
-int scan_exclusive(const int *in, int n, int *out, int *tile_sums, hipStream_t s);
+int scan_exclusive(const int *in, int n, int *out, int *tile_sums, hipStream_t s, const int *n_dev = nullptr, int *total = nullptr,
+                   bool add = false);
 void fill_async(int *p, size_t n, int v, hipStream_t s);
 int compact_scatter(const int *flags, const int *offs, int n, const int *src, const int *base_dev, int base_const,
-                    int *out, hipStream_t s);
+                    int *out, hipStream_t s, const int *n_dev = nullptr);
 
 // stable LSD radix sort of (key, int) pairs by the low `bits` key bits (sort.hip): k0/v0 hold the
 // input, k1/v1 the same sizes; *kres/*vres receive whichever pair holds the result.  tmp holds
 // radix_sort_tmp_ints(n) ints.  Inclusive prefix maximum of n ints (tmp: max_scan_tmp_ints(n)).
 size_t radix_sort_tmp_ints(int n);
-int radix_sort_pairs_u32(unsigned *k0, int *v0, unsigned *k1, int *v1, int n, int bits, int *tmp, hipStream_t s,
-                         unsigned **kres, int **vres);
 int radix_sort_pairs_u64(unsigned long long *k0, int *v0, unsigned long long *k1, int *v1, int n, int bits, int *tmp,
                          hipStream_t s, unsigned long long **kres, int **vres);
 size_t max_scan_tmp_ints(int n);
+// rows with photons of frames first..end, stably sorted by frame, into d_out, their number into *d_m;
+// tmp holds sort_rows_tmp_ints(n, first, end) ints
+size_t sort_rows_tmp_ints(int n, int first, int end);
+int sort_rows_by_frame(const float *d_loc, int n, int first, int end, float *d_out, int *d_m, int *tmp, hipStream_t s);
 int scan_inclusive_max(const int *in, int n, int *out, int *tmp, hipStream_t s);
 
 }  // namespace qcs

@@ -1,19 +1,24 @@
-// sort.hip -- stable LSD radix sort of (key, index) pairs and an inclusive max-scan (gfx950).
+// sort.hip -- stable LSD radix sort of (key, index) pairs, of localization rows by frame, and an
+// inclusive max-scan (gfx950).
 //
-// The localization path sorts rows by frame (frame-sorted compaction), by (frame, cell) keys
-// (neighbour counts of the statistics, link search of consecutive-frame merging).  Each pass
-// sorts by one 8-bit digit:
-//   radix_hist_kernel     one work-group per tile of 2048 keys: LDS digit histogram, written
+// The localization path sorts rows by frame (frame-sorted compaction) and by (frame, cell) keys
+// (link search of consecutive-frame merging).  Each pass sorts by one 8-bit digit:
+//   radix_hist_kernel     one work-group per tile of 2048 items: LDS digit histogram, written
 //                         digit-major (counts[d * ntiles + tile]);
 //   scan                  exclusive scan of the 256 x ntiles counts (digit-major), so a tile's
 //                         slice of digit d starts after every earlier digit and every earlier
 //                         tile's keys of digit d;
-//   radix_scatter_kernel  the tile again, 256 keys per round in index order: each wave finds the
+//   radix_scatter_kernel  the tile again, 256 items per round in index order: each wave finds the
 //                         lanes holding its digit by 8 ballots (one per digit bit), ranks itself
 //                         among the lower lanes, adds the counts of the lower waves (LDS) and the
 //                         tile's running base of the digit.
 // Equal digits keep their input order (stable), so the passes from the lowest digit up sort the
 // keys stably; there are no atomics on the data path, so the result is deterministic.
+//
+// A pass reads its items from a source and writes them to a destination.  The row sort's first pass
+// reads the rows themselves, where rows that are not kept count nowhere, and its last pass writes
+// rows: up to 256 frames are one pass of three launches with no flags, no list and no key arrays,
+// and the number of kept rows stays on the device until the end.
 #include <limits.h>
 #include "qcs_internal.h"
 
@@ -26,42 +31,104 @@ constexpr int SI = 8;                    // keys per thread per tile
 constexpr int STILE = SB * SI;           // keys per tile
 constexpr int RADIX = 256;
 
+// sources: get() gives the item's key and value, false if there is none
 template <typename K>
-__global__ void __launch_bounds__(SB) radix_hist_kernel(const K *__restrict__ keys, int n, int shift, int ntiles,
-                                                        int *__restrict__ counts)
+struct PairSrc {
+    const K *k;
+    const int *v;
+    int n;
+    const int *n_dev;   // items on the device, or null
+    __device__ __forceinline__ int count() const { return n_dev ? min(*n_dev, n) : n; }
+    __device__ __forceinline__ bool key(int i, int m, K &key) const
+    {
+        if (i >= m) return false;
+        key = k[i];
+        return true;
+    }
+    __device__ __forceinline__ int val(int i) const { return v[i]; }
+};
+
+// float -> int truncation with NaN -> 0 and saturation (the CUDA conversion the reference relies on)
+__device__ __forceinline__ int f2i_sat(float v)
+{
+    if (v != v) return 0;
+    if (v >= 2147483647.0f) return 2147483647;
+    if (v <= -2147483648.0f) return (-2147483647 - 1);
+    return (int)v;
+}
+
+// the rows with photons of frames first..end (RemoveZero_SortFrame), key = frame - first
+struct RowSrc {
+    const float *loc;
+    int n, first, end;
+    __device__ __forceinline__ int count() const { return n; }
+    __device__ __forceinline__ bool key(int i, int m, unsigned &key) const
+    {
+        if (i >= m) return false;
+        const float *r = loc + (size_t)i * QCS_REC_FLOATS;
+        const int pp = f2i_sat(r[QCS_POS_PPHO]), fr = f2i_sat(r[QCS_POS_FRME]);
+        key = (unsigned)fr - (unsigned)first;
+        return ((float)pp > 1.0f) && fr >= first && fr <= end;
+    }
+    __device__ __forceinline__ int val(int i) const { return i; }
+};
+
+template <typename K>
+struct PairDst {
+    K *k;
+    int *v;
+    __device__ __forceinline__ void put(int pos, K key, int val) const
+    {
+        k[pos] = key;
+        v[pos] = val;
+    }
+};
+
+struct RowDst {
+    const float *loc;
+    float *out;
+    __device__ __forceinline__ void put(int pos, unsigned, int val) const
+    {
+        const float4 *src = reinterpret_cast<const float4 *>(loc + (size_t)val * QCS_REC_FLOATS);
+        float4 *dst = reinterpret_cast<float4 *>(out + (size_t)pos * QCS_REC_FLOATS);
+        dst[0] = src[0];
+        dst[1] = src[1];
+        dst[2] = src[2];
+    }
+};
+
+template <typename K, class Src>
+__global__ void __launch_bounds__(SB) radix_hist_kernel(Src src, int shift, int ntiles, int *__restrict__ counts)
 {
     __shared__ int h[RADIX];
     const int tid = threadIdx.x;
     h[tid] = 0;
     __syncthreads();
-    const int t0 = blockIdx.x * STILE;
+    const int t0 = blockIdx.x * STILE, m = src.count();
 #pragma unroll
     for (int k = 0; k < SI; k++) {
-        const int i = t0 + k * SB + tid;
-        if (i < n) atomicAdd(&h[(int)((keys[i] >> shift) & (K)(RADIX - 1))], 1);
+        K key;
+        if (src.key(t0 + k * SB + tid, m, key)) atomicAdd(&h[(int)((key >> shift) & (K)(RADIX - 1))], 1);
     }
     __syncthreads();
     counts[(size_t)tid * ntiles + blockIdx.x] = h[tid];
 }
 
-template <typename K>
-__global__ void __launch_bounds__(SB) radix_scatter_kernel(const K *__restrict__ kin, const int *__restrict__ vin,
-                                                           K *__restrict__ kout, int *__restrict__ vout, int n, int shift,
-                                                           int ntiles, const int *__restrict__ offs)
+template <typename K, class Src, class Dst>
+__global__ void __launch_bounds__(SB) radix_scatter_kernel(Src src, Dst dst, int shift, int ntiles, const int *__restrict__ offs)
 {
     __shared__ int base[RADIX];
     __shared__ int wcnt[SB / 64][RADIX];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     base[tid] = offs[(size_t)tid * ntiles + blockIdx.x];
-    const int t0 = blockIdx.x * STILE;
+    const int t0 = blockIdx.x * STILE, n = src.count();
     for (int k = 0; k < SI; k++) {
 #pragma unroll
         for (int w = 0; w < SB / 64; w++) wcnt[w][tid] = 0;
         __syncthreads();
         const int i = t0 + k * SB + tid;
-        const bool valid = i < n;
-        const K key = valid ? kin[i] : (K)0;
-        const int val = valid ? vin[i] : 0;
+        K key = 0;
+        const bool valid = src.key(i, n, key);
         const int d = (int)((key >> shift) & (K)(RADIX - 1));
         unsigned long long m = __ballot(valid);
 #pragma unroll
@@ -75,8 +142,7 @@ __global__ void __launch_bounds__(SB) radix_scatter_kernel(const K *__restrict__
         if (valid) {
             int pos = base[d] + rank;
             for (int w = 0; w < wv; w++) pos += wcnt[w][d];
-            kout[pos] = key;
-            vout[pos] = val;
+            dst.put(pos, key, src.val(i));
         }
         __syncthreads();
         int add = 0;
@@ -155,31 +221,21 @@ __global__ void __launch_bounds__(256) max_scan_add_kernel(int *__restrict__ out
     out[i] = out[i] > c ? out[i] : c;
 }
 
-template <typename K>
-int radix_sort_impl(K *k0, int *v0, K *k1, int *v1, int n, int bits, int *tmp, hipStream_t s, K **kres, int **vres)
+// one pass over up to n items; counts -> offs -> tsum are the ints of radix_sort_tmp_ints(n);
+// *total (may be null) receives the number of items
+template <typename K, class Src, class Dst>
+int radix_pass(const Src &src, const Dst &dst, int n, int shift, int *tmp, int *total, hipStream_t s)
 {
-    *kres = k0;
-    *vres = v0;
-    if (n <= 0 || bits <= 0) return QCS_OK;
     const int ntiles = (n + STILE - 1) / STILE;
     const long long ncount = (long long)RADIX * ntiles;
     if (ncount > 16LL * 1024 * 1024) return fail(QCS_ERR_ARG, "sort of %d keys exceeds the supported size", n);
     int *counts = tmp, *offs = tmp + ncount, *tsum = offs + ncount;
-    K *ki = k0, *ko = k1;
-    int *vi = v0, *vo = v1;
-    const int maxbits = (int)(8 * sizeof(K));
-    for (int shift = 0; shift < bits && shift < maxbits; shift += 8) {
-        hipLaunchKernelGGL((radix_hist_kernel<K>), dim3(ntiles), dim3(SB), 0, s, ki, n, shift, ntiles, counts);
-        QCS_HIP(hipGetLastError());
-        int rc = scan_exclusive(counts, (int)ncount, offs, tsum, s);
-        if (rc) return rc;
-        hipLaunchKernelGGL((radix_scatter_kernel<K>), dim3(ntiles), dim3(SB), 0, s, ki, vi, ko, vo, n, shift, ntiles, offs);
-        QCS_HIP(hipGetLastError());
-        K *tk = ki; ki = ko; ko = tk;
-        int *tv = vi; vi = vo; vo = tv;
-    }
-    *kres = ki;
-    *vres = vi;
+    hipLaunchKernelGGL((radix_hist_kernel<K, Src>), dim3(ntiles), dim3(SB), 0, s, src, shift, ntiles, counts);
+    QCS_HIP(hipGetLastError());
+    const int rc = scan_exclusive(counts, (int)ncount, offs, tsum, s, nullptr, total);
+    if (rc) return rc;
+    hipLaunchKernelGGL((radix_scatter_kernel<K, Src, Dst>), dim3(ntiles), dim3(SB), 0, s, src, dst, shift, ntiles, offs);
+    QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
 
@@ -192,16 +248,46 @@ size_t radix_sort_tmp_ints(int n)
     return 2 * ncount + (size_t)scan_tile_count(ncount) + 1;
 }
 
-int radix_sort_pairs_u32(unsigned *k0, int *v0, unsigned *k1, int *v1, int n, int bits, int *tmp, hipStream_t s,
-                         unsigned **kres, int **vres)
-{
-    return radix_sort_impl<unsigned>(k0, v0, k1, v1, n, bits, tmp, s, kres, vres);
-}
-
 int radix_sort_pairs_u64(unsigned long long *k0, int *v0, unsigned long long *k1, int *v1, int n, int bits, int *tmp,
                          hipStream_t s, unsigned long long **kres, int **vres)
 {
-    return radix_sort_impl<unsigned long long>(k0, v0, k1, v1, n, bits, tmp, s, kres, vres);
+    using K = unsigned long long;
+    K *ki = k0, *ko = k1;
+    int *vi = v0, *vo = v1;
+    for (int shift = 0; n > 0 && shift < bits && shift < 64; shift += 8) {
+        const int rc = radix_pass<K>(PairSrc<K>{ki, vi, n, nullptr}, PairDst<K>{ko, vo}, n, shift, tmp, nullptr, s);
+        if (rc) return rc;
+        K *tk = ki; ki = ko; ko = tk;
+        int *tv = vi; vi = vo; vo = tv;
+    }
+    *kres = ki;
+    *vres = vi;
+    return QCS_OK;
+}
+
+size_t sort_rows_tmp_ints(int n, int first, int end)
+{
+    return radix_sort_tmp_ints(n) + (((unsigned)end - (unsigned)first) > 255u ? (size_t)n * 4 : 0);
+}
+
+int sort_rows_by_frame(const float *d_loc, int n, int first, int end, float *d_out, int *d_m, int *tmp, hipStream_t s)
+{
+    const unsigned span = ((unsigned)end - (unsigned)first);
+    const RowSrc rows{d_loc, n, first, end};
+    const RowDst out{d_loc, d_out};
+    int rc;
+    if (span <= 255u) return radix_pass<unsigned>(rows, out, n, 0, tmp, d_m, s);
+    unsigned *k0 = reinterpret_cast<unsigned *>(tmp + radix_sort_tmp_ints(n)), *k1 = k0 + n;
+    int *v0 = reinterpret_cast<int *>(k1 + n), *v1 = v0 + n;
+    if ((rc = radix_pass<unsigned>(rows, PairDst<unsigned>{k0, v0}, n, 0, tmp, d_m, s))) return rc;
+    for (int shift = 8; shift < 32 && (span >> shift) != 0; shift += 8) {
+        const PairSrc<unsigned> src{k0, v0, n, d_m};
+        if (shift + 8 >= 32 || (span >> (shift + 8)) == 0) return radix_pass<unsigned>(src, out, n, shift, tmp, nullptr, s);
+        if ((rc = radix_pass<unsigned>(src, PairDst<unsigned>{k1, v1}, n, shift, tmp, nullptr, s))) return rc;
+        unsigned *tk = k0; k0 = k1; k1 = tk;
+        int *tv = v0; v0 = v1; v1 = tv;
+    }
+    return QCS_OK;
 }
 
 size_t max_scan_tmp_ints(int n) { return (size_t)(((size_t)(n > 0 ? n : 1) + MTILE - 1) / MTILE) + 1; }

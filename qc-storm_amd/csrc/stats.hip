@@ -10,17 +10,21 @@
 //   GetFirstFrame, GetLastFrame                    DLL/bfgsMLE_Loc_top/bfgs_top.cu:345-381
 //
 // The row pass builds the four histograms in LDS per work-group (one global add per non-empty
-// bin) and the sums in FP64.  The reference counts neighbours by an all-pairs scan of every
-// frame's molecules, one frame per launch with a host synchronisation each; here the molecules
-// of all frames are sorted once by (frame, cell of the neighbour radius) and each scans the 3x3
-// cells around its own, which visits every pair closer than the radius: the counts are the
-// same integers.
+// bin) and the sums in FP64, one add per work-group.  The reference counts neighbours by an
+// all-pairs scan of every frame's molecules, one frame per launch with a host synchronisation
+// each; here the molecules of all frames go into a hash table of (frame, cell of the neighbour
+// radius) buckets (count, scan, scatter) and each scans the buckets of the 3x3 cells around its own,
+// which visits every pair closer than the radius: the counts are the same integers.
+// The batch is small (an output call has some ten thousand rows), so launches and waits are what
+// it costs: the frame range stays on the device and everything is read back once, eight launches
+// and one wait.  Sorting the molecules by (frame, cell) and searching the sorted keys took 19
+// launches and five waits, and each search is a chain of fifteen dependent loads (20,480 rows:
+// neighbours 28.8 -> 10 us, row pass 28.6 -> 6 us; with compaction and rendering 417 -> 215 us).
 #include <limits.h>
 #include <stddef.h>
 #include <algorithm>
 #include <math.h>
 #include <string.h>
-#include <vector>
 #include "qcs_internal.h"
 
 namespace qcs {
@@ -33,22 +37,44 @@ constexpr int SB = QCS_STAT_BINS, SL = 400;
 struct StatAcc {
     int hist[4][SB];
     double sum[4];   // loc prec, peak SNR, PSF width, background
-    int valid, first_idx, last_idx, kept, n0, n1, pad[2];
+    // first and last rows with a frame: row index above, frame (int) below; none: ~0 and 0
+    unsigned long long first, last;
+    int valid, kept, n0, n1;
 };
+
+// frames the density looks at: both ends are dropped when more than 3 (GetFirstFrame, GetLastFrame)
+struct FrameRange {
+    int fs, fe;
+};
+__host__ __device__ inline FrameRange frame_range(const StatAcc &a)
+{
+    FrameRange r;
+    r.fs = a.first == ~0ull ? 0 : (int)(unsigned)a.first;
+    r.fe = a.last == 0ull ? 0 : (int)(unsigned)a.last;
+    if ((long long)r.fe - r.fs + 1 > 3) {
+        r.fs++;
+        r.fe--;
+    }
+    return r;
+}
 
 // bin of a quotient value / width, clamped to [0, SB - 1] (the reference converts to int with
 // saturation and clamps; clamping the float first gives the same bin without an out-of-range
 // conversion)
 __device__ __forceinline__ int sbin(float q) { return q >= (float)SB ? SB - 1 : (q > 0.0f ? (int)q : 0); }
 
-__global__ void __launch_bounds__(256) stat_rows_kernel(const float *__restrict__ loc, int n, StatAcc *__restrict__ acc)
+constexpr int RT = 512;   // threads of a row pass work-group
+
+__global__ void __launch_bounds__(RT) stat_rows_kernel(const float *__restrict__ loc, int n, StatAcc *__restrict__ acc)
 {
     __shared__ int h[4][SB];
-    for (int k = threadIdx.x; k < 4 * SB; k += blockDim.x) (&h[0][0])[k] = 0;
+    __shared__ double ws[4][RT / 64];
+    __shared__ int wi[3][RT / 64];
+    for (int k = threadIdx.x; k < 4 * SB; k += RT) (&h[0][0])[k] = 0;
     __syncthreads();
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     int valid = 0, first = INT_MAX, last = -1;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int i = blockIdx.x * RT + threadIdx.x; i < n; i += gridDim.x * RT) {
         const float *r = loc + (size_t)i * QCS_REC_FLOATS;
         const int fr = (int)r[QCS_POS_FRME];
         if (fr != 0) {
@@ -78,112 +104,126 @@ __global__ void __launch_bounds__(256) stat_rows_kernel(const float *__restrict_
         last = max(last, __shfl_down(last, off, 64));
     }
     if ((threadIdx.x & 63) == 0) {
-        for (int k = 0; k < 4; k++)
-            if (s[k] != 0.0) atomicAdd(&acc->sum[k], s[k]);
-        if (valid) atomicAdd(&acc->valid, valid);
-        if (first != INT_MAX) atomicMin(&acc->first_idx, first);
-        if (last >= 0) atomicMax(&acc->last_idx, last);
+        const int w = threadIdx.x >> 6;
+        for (int k = 0; k < 4; k++) ws[k][w] = s[k];
+        wi[0][w] = valid;
+        wi[1][w] = first;
+        wi[2][w] = last;
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < 4 * SB; k += blockDim.x) {
+    if (threadIdx.x < 7) {
+        const int k = threadIdx.x;
+        if (k < 4) {
+            double t = 0.0;
+            for (int w = 0; w < RT / 64; w++) t += ws[k][w];
+            if (t != 0.0) atomicAdd(&acc->sum[k], t);
+        } else if (k == 4) {
+            int t = 0;
+            for (int w = 0; w < RT / 64; w++) t += wi[0][w];
+            if (t) atomicAdd(&acc->valid, t);
+        } else if (k == 5) {
+            int t = INT_MAX;
+            for (int w = 0; w < RT / 64; w++) t = min(t, wi[1][w]);
+            if (t != INT_MAX)
+                atomicMin(&acc->first, ((unsigned long long)(unsigned)t << 32) |
+                                           (unsigned)(int)loc[(size_t)t * QCS_REC_FLOATS + QCS_POS_FRME]);
+        } else {
+            int t = -1;
+            for (int w = 0; w < RT / 64; w++) t = max(t, wi[2][w]);
+            if (t >= 0)
+                atomicMax(&acc->last, ((unsigned long long)(unsigned)t << 32) |
+                                          (unsigned)(int)loc[(size_t)t * QCS_REC_FLOATS + QCS_POS_FRME]);
+        }
+    }
+    for (int k = threadIdx.x; k < 4 * SB; k += RT) {
         const int v = (&h[0][0])[k];
         if (v) atomicAdd(&(&acc->hist[0][0])[k], v);
     }
 }
 
-// density cell key of every molecule of frames fs..fe at least 5 px inside the image
-// (FillerMoleculesInCurFrame); other rows get the key `none`, sorted behind them.  Cells are
-// `cell` = radius * (1 + 2^-10) wide: two molecules whose float distance test passes are then at
-// most one cell apart in x and in y even after the rounding of the quotients.
-__global__ void __launch_bounds__(256) stat_keys_kernel(const float *__restrict__ loc, int n, int fs, int fe, int W, int H,
-                                                        float cell, int ncx, int ncy, unsigned long long none,
-                                                        unsigned long long *__restrict__ keys, int *__restrict__ vals,
-                                                        StatAcc *__restrict__ acc)
+// The neighbour grid.  Cells are `cell` = radius * (1 + 2^-10) wide: two molecules whose float
+// distance test passes are then at most one cell apart in x and in y even after the rounding of the
+// quotients.  A molecule's bucket is a hash of its frame and cell; the cells around one molecule may
+// share a bucket, so an entry carries its frame and cell and counts for its own cell only.
+struct Grid {
+    int W, H, ncx, lb;   // 2^lb buckets
+    float cell, r2;
+};
+__device__ __forceinline__ int bucket(const Grid &g, int frame, unsigned c)
+{
+    unsigned u = c * 2654435769u + (unsigned)frame * 2246822519u;
+    u ^= u >> 15;
+    u *= 739982445u;
+    return (int)(u >> (32 - g.lb));
+}
+__device__ __forceinline__ unsigned cell_id(const Grid &g, int cx, int cy) { return (unsigned)cy * (unsigned)g.ncx + (unsigned)cx; }
+
+// Molecules of frames fs..fe at least 5 px inside the image (FillerMoleculesInCurFrame).  Pass 1
+// (ent == null): molecules per bucket; pass 2: the entries {x, y, frame, cell}, counting cnt down.
+__global__ void __launch_bounds__(256) stat_bins_kernel(const float *__restrict__ loc, int n, Grid g, const StatAcc *__restrict__ acc,
+                                                        int *__restrict__ cnt, const int *__restrict__ offs, float4 *__restrict__ ent)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool kept = false;
-    if (i < n) {
-        const float *r = loc + (size_t)i * QCS_REC_FLOATS;
-        const float X = r[QCS_POS_XPOS], Y = r[QCS_POS_YPOS];
-        const int x = (int)X, y = (int)Y, cf = (int)r[QCS_POS_FRME];
-        unsigned long long key = none;
-        if (x >= 5 && x < W - 5 && y >= 5 && y < H - 5 && cf >= fs && cf <= fe) {
-            const int cx = (int)(X / cell), cy = (int)(Y / cell);
-            key = ((unsigned long long)(cf - fs) * (unsigned long long)ncy + (unsigned long long)cy) * (unsigned long long)ncx +
-                  (unsigned long long)cx;
-            kept = true;
-        }
-        keys[i] = key;
-        vals[i] = i;
-    }
-    const unsigned long long m = __ballot(kept);
-    if (m && (threadIdx.x & 63) == 0) atomicAdd(&acc->kept, __popcll(m));
+    if (i >= n) return;
+    const FrameRange fr = frame_range(*acc);
+    const float *r = loc + (size_t)i * QCS_REC_FLOATS;
+    const float X = r[QCS_POS_XPOS], Y = r[QCS_POS_YPOS];
+    const int x = (int)X, y = (int)Y, cf = (int)r[QCS_POS_FRME];
+    if (!(x >= 5 && x < g.W - 5 && y >= 5 && y < g.H - 5 && cf >= fr.fs && cf <= fr.fe)) return;
+    const unsigned c = cell_id(g, (int)(X / g.cell), (int)(Y / g.cell));
+    const int b = bucket(g, cf, c);
+    if (!ent) atomicAdd(&cnt[b], 1);
+    else ent[offs[b] + atomicSub(&cnt[b], 1) - 1] = make_float4(X, Y, __int_as_float(cf), __int_as_float((int)c));
 }
 
-__device__ __forceinline__ int lower_bound_key(const unsigned long long *__restrict__ keys, int m, unsigned long long k)
+// Neighbours within the radius in the same frame (CalcOverlapFluoNum): molecules with 0 and with 1.
+// 16 lanes per molecule, one per cell of the 3x3 block: the nine bucket walks are one round of
+// loads instead of nine.  A molecule finds itself once, at distance 0.
+__global__ void __launch_bounds__(256) stat_neigh_kernel(const float4 *__restrict__ ent, const int *__restrict__ offs, Grid g,
+                                                         int nb, StatAcc *__restrict__ acc)
 {
-    int lo = 0, hi = m;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (keys[mid] < k) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
-// neighbours within the radius in the same frame (CalcOverlapFluoNum): molecules with 0 and 1
-__global__ void __launch_bounds__(256) stat_neigh_kernel(const float *__restrict__ loc, const unsigned long long *__restrict__ keys,
-                                                         const int *__restrict__ vals, int m, int ncx, int ncy, float r2,
-                                                         StatAcc *__restrict__ acc)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    int c0 = 0, c1 = 0;
-    if (p < m) {
-        const unsigned long long key = keys[p];
-        const int row = vals[p];
-        const int cx = (int)(key % (unsigned long long)ncx);
-        const unsigned long long fy = key / (unsigned long long)ncx;
-        const int cy = (int)(fy % (unsigned long long)ncy);
-        const unsigned long long fbase = (fy / (unsigned long long)ncy) * (unsigned long long)ncy;
-        const float X = loc[(size_t)row * QCS_REC_FLOATS + QCS_POS_XPOS], Y = loc[(size_t)row * QCS_REC_FLOATS + QCS_POS_YPOS];
-        int cnt = 0;
-        for (int dy = -1; dy <= 1; dy++) {
-            const int yy = cy + dy;
-            if (yy < 0 || yy >= ncy) continue;
-            for (int dx = -1; dx <= 1; dx++) {
-                const int xx = cx + dx;
-                if (xx < 0 || xx >= ncx) continue;
-                const unsigned long long k2 = (fbase + (unsigned long long)yy) * (unsigned long long)ncx + (unsigned long long)xx;
-                for (int q = lower_bound_key(keys, m, k2); q < m && keys[q] == k2; q++) {
-                    const int o = vals[q];
-                    if (o == row) continue;
-                    const float ox = loc[(size_t)o * QCS_REC_FLOATS + QCS_POS_XPOS] - X;
-                    const float oy = loc[(size_t)o * QCS_REC_FLOATS + QCS_POS_YPOS] - Y;
-                    cnt += (ox * ox + oy * oy) <= r2;
-                }
+    __shared__ int wc[2][4];
+    const int m = offs[nb];
+    if (blockIdx.x == 0 && threadIdx.x == 0) acc->kept = m;
+    const int p = (int)(blockIdx.x * 16 + (threadIdx.x >> 4)), l = threadIdx.x & 15;
+    int cnt = 0;
+    if (p < m && l < 9) {
+        const float4 e = ent[p];
+        const int cx = (int)(e.x / g.cell) + l % 3 - 1, cy = (int)(e.y / g.cell) + l / 3 - 1;
+        const int cf = __float_as_int(e.z);
+        if (cx >= 0 && cy >= 0) {
+            const unsigned c = cell_id(g, cx, cy);
+            const int b = bucket(g, cf, c);
+            for (int q = offs[b]; q < offs[b + 1]; q++) {
+                const float4 o = ent[q];
+                const float ox = o.x - e.x, oy = o.y - e.y;
+                cnt += (ox * ox + oy * oy) <= g.r2 && __float_as_int(o.z) == cf && (unsigned)__float_as_int(o.w) == c;
             }
         }
-        c0 = cnt == 0;
-        c1 = cnt == 1;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        c0 += __shfl_down(c0, off, 64);
-        c1 += __shfl_down(c1, off, 64);
-    }
+    for (int off = 8; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 16);
+    const bool lead = p < m && l == 0;
+    const int c0 = __popcll(__ballot(lead && cnt == 1)), c1 = __popcll(__ballot(lead && cnt == 2));
     if ((threadIdx.x & 63) == 0) {
-        if (c0) atomicAdd(&acc->n0, c0);
-        if (c1) atomicAdd(&acc->n1, c1);
+        wc[0][threadIdx.x >> 6] = c0;
+        wc[1][threadIdx.x >> 6] = c1;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const int t = wc[threadIdx.x][0] + wc[threadIdx.x][1] + wc[threadIdx.x][2] + wc[threadIdx.x][3];
+        if (t) atomicAdd(threadIdx.x ? &acc->n1 : &acc->n0, t);
     }
 }
 
-__global__ void stat_init_kernel(StatAcc *acc)
+// accumulator and bucket counts; one writer per word
+__global__ void stat_init_kernel(StatAcc *acc, int *cnt, int nb)
 {
-    // one writer per word: first_idx starts at INT_MAX, last_idx at -1, everything else at 0
     int *p = reinterpret_cast<int *>(acc);
-    const int nw = (int)(sizeof(StatAcc) / sizeof(int));
-    const int wf = (int)(offsetof(StatAcc, first_idx) / sizeof(int)), wl = (int)(offsetof(StatAcc, last_idx) / sizeof(int));
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nw; k += gridDim.x * blockDim.x)
-        p[k] = k == wf ? INT_MAX : (k == wl ? -1 : 0);
+    const int nw = (int)(sizeof(StatAcc) / sizeof(int)), wf = (int)(offsetof(StatAcc, first) / sizeof(int));
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nw + nb; k += gridDim.x * blockDim.x) {
+        if (k < nw) p[k] = (k == wf || k == wf + 1) ? -1 : 0;
+        else cnt[k - nw] = 0;
+    }
 }
 
 // GetHistogramMeanData (statisticsInfo_rc.cu:44-74), float arithmetic in bin order
@@ -232,23 +272,35 @@ extern "C" int qcs_loc_stats_dev(qcs_ctx *ctx, const float *d_loc, int n, qcs_lo
     if (n == 0) return QCS_OK;
     hipStream_t s = (hipStream_t)stream;
     const qcs_params &p = ctx->p;
-    // scratch: accumulator, keys and values (double-buffered for the sort), sort workspace
-    const size_t temp = sizeof(int) * radix_sort_tmp_ints(n);
-    const size_t acc_b = (sizeof(StatAcc) + 255) & ~(size_t)255, keys_b = ((size_t)n * 8 + 255) & ~(size_t)255,
-                 vals_b = ((size_t)n * 4 + 255) & ~(size_t)255;
+    if (n > 1 << 27) return fail(QCS_ERR_ARG, "statistics of %d rows exceed the supported size", n);
+    const float rad = (p.LocType == QCS_LOCTYPE_GS2D) ? 10.0f : 20.0f;
+    Grid g;
+    g.W = p.ImageWidth;
+    g.H = p.ImageHigh;
+    g.cell = rad * 1.0009765625f;
+    g.ncx = (int)((float)p.ImageWidth / g.cell) + 2;
+    g.r2 = rad * rad;
+    for (g.lb = 8; g.lb < 24 && (1 << g.lb) < n; g.lb++) {}   // a bucket per molecule, as far as one scan goes
+    const int nb = 1 << g.lb;
+    // scratch: accumulator, entries, bucket counts, offsets (one more than buckets), scan sums
+    const size_t acc_b = (sizeof(StatAcc) + 255) & ~(size_t)255, ent_b = (size_t)n * sizeof(float4);
     int rc;
-    if ((rc = ctx->st_buf.ensure(acc_b + 2 * keys_b + 2 * vals_b + temp + 256))) return rc;
-    char *b = ctx->st_buf.as<char>();
-    StatAcc *acc = reinterpret_cast<StatAcc *>(b);
-    unsigned long long *k_in = reinterpret_cast<unsigned long long *>(b + acc_b), *k_out = reinterpret_cast<unsigned long long *>(b + acc_b + keys_b);
-    int *v_in = reinterpret_cast<int *>(b + acc_b + 2 * keys_b), *v_out = reinterpret_cast<int *>(b + acc_b + 2 * keys_b + vals_b);
-    void *tmp = b + acc_b + 2 * keys_b + 2 * vals_b;
-    hipLaunchKernelGGL(stat_init_kernel, dim3(8), dim3(256), 0, s, acc);
-    const int blocks = (int)std::min<size_t>(((size_t)n + 255) / 256, 1024);
-    hipLaunchKernelGGL(stat_rows_kernel, dim3(blocks), dim3(256), 0, s, d_loc, n, acc);
+    if ((rc = ctx->st_buf.ensure(acc_b + ent_b + sizeof(int) * (2 * (size_t)nb + 1 + scan_tile_count((size_t)nb) + 1))) ||
+        (rc = ctx->pin_cnt.ensure(sizeof(StatAcc))))
+        return rc;
+    char *buf = ctx->st_buf.as<char>();
+    StatAcc *acc = reinterpret_cast<StatAcc *>(buf), *h = ctx->pin_cnt.as<StatAcc>();
+    float4 *ent = reinterpret_cast<float4 *>(buf + acc_b);
+    int *cnt = reinterpret_cast<int *>(buf + acc_b + ent_b), *offs = cnt + nb, *tsum = offs + nb + 1;
+    const dim3 gr((n + 255) / 256), blk(256);
+    hipLaunchKernelGGL(stat_init_kernel, dim3(std::min((nb + 2047) / 2048 + 1, 1024)), blk, 0, s, acc, cnt, nb);
+    hipLaunchKernelGGL(stat_rows_kernel, dim3(std::min((n + RT - 1) / RT, 512)), dim3(RT), 0, s, d_loc, n, acc);
+    hipLaunchKernelGGL(stat_bins_kernel, gr, blk, 0, s, d_loc, n, g, acc, cnt, nullptr, nullptr);
     QCS_HIP(hipGetLastError());
-    std::vector<char> hb(sizeof(StatAcc));
-    StatAcc *h = reinterpret_cast<StatAcc *>(hb.data());
+    if ((rc = scan_exclusive(cnt, nb, offs, tsum, s, nullptr, offs + nb))) return rc;
+    hipLaunchKernelGGL(stat_bins_kernel, gr, blk, 0, s, d_loc, n, g, acc, cnt, offs, ent);
+    hipLaunchKernelGGL(stat_neigh_kernel, dim3((unsigned)(((size_t)n + 15) / 16)), blk, 0, s, ent, offs, g, nb, acc);
+    QCS_HIP(hipGetLastError());
     QCS_HIP(hipMemcpyAsync(h, acc, sizeof(StatAcc), hipMemcpyDeviceToHost, s));
     QCS_HIP(hipStreamSynchronize(s));
     memcpy(out->hist_total_photon, h->hist[0], sizeof(out->hist_total_photon));
@@ -268,52 +320,16 @@ extern "C" int qcs_loc_stats_dev(qcs_ctx *ctx, const float *d_loc, int n, qcs_lo
     out->mean_psf_width = (float)(out->sum_psf_width / vn);
     out->mean_psf_width_ctl = out->mean_psf_width * (-out->mean_peak_snr);
 
-    // frame range (GetFirstFrame / GetLastFrame), both ends dropped when more than 3 frames
-    int fs = 0, fe = 0;
-    float fv;
-    if (h->first_idx != INT_MAX) {
-        QCS_HIP(hipMemcpy(&fv, d_loc + (size_t)h->first_idx * QCS_REC_FLOATS + QCS_POS_FRME, sizeof(float), hipMemcpyDeviceToHost));
-        fs = (int)fv;
-    }
-    if (h->last_idx >= 0) {
-        QCS_HIP(hipMemcpy(&fv, d_loc + (size_t)h->last_idx * QCS_REC_FLOATS + QCS_POS_FRME, sizeof(float), hipMemcpyDeviceToHost));
-        fe = (int)fv;
-    }
-    if (fe - fs + 1 > 3) {
-        fs++;
-        fe--;
-    }
-    out->density_first_frame = fs;
-    out->density_last_frame = fe;
-    if (fe < fs) return QCS_OK;
-    const float rad = (p.LocType == QCS_LOCTYPE_GS2D) ? 10.0f : 20.0f;
-    const float cell = rad * 1.0009765625f;
-    const int ncx = (int)((float)p.ImageWidth / cell) + 2, ncy = (int)((float)p.ImageHigh / cell) + 2;
-    const unsigned long long none = (unsigned long long)(fe - fs + 1) * (unsigned long long)ncy * (unsigned long long)ncx;
-    int bits = 1;
-    while (bits < 64 && (none >> bits) != 0ull) bits++;
-    const dim3 g((n + 255) / 256), blk(256);
-    hipLaunchKernelGGL(stat_keys_kernel, g, blk, 0, s, d_loc, n, fs, fe, p.ImageWidth, p.ImageHigh, cell, ncx, ncy, none, k_in, v_in, acc);
-    QCS_HIP(hipGetLastError());
-    unsigned long long *k_sorted;
-    int *v_sorted;
-    if ((rc = radix_sort_pairs_u64(k_in, v_in, k_out, v_out, n, bits, static_cast<int *>(tmp), s, &k_sorted, &v_sorted))) return rc;
-    int kept = 0;
-    QCS_HIP(hipMemcpyAsync(&kept, &acc->kept, sizeof(int), hipMemcpyDeviceToHost, s));
-    QCS_HIP(hipStreamSynchronize(s));
-    if (kept > 0) {
-        hipLaunchKernelGGL(stat_neigh_kernel, dim3((kept + 255) / 256), blk, 0, s, d_loc, k_sorted, v_sorted, kept, ncx, ncy, rad * rad,
-                           acc);
-        QCS_HIP(hipGetLastError());
-    }
-    int cnt[2] = {0, 0};
-    QCS_HIP(hipMemcpyAsync(cnt, &acc->n0, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
-    QCS_HIP(hipStreamSynchronize(s));
+    const FrameRange fr = frame_range(*h);
+    out->density_first_frame = fr.fs;
+    out->density_last_frame = fr.fe;
+    if (fr.fe < fr.fs) return QCS_OK;
+    const int kept = h->kept;
     out->density_total = kept;
-    out->density_n0 = cnt[0];
-    out->density_n1 = cnt[1];
+    out->density_n0 = h->n0;
+    out->density_n1 = h->n1;
     if (kept > 50) {
-        const float r0 = (float)cnt[0] / (float)kept, r1 = (float)cnt[1] / (float)kept;
+        const float r0 = (float)h->n0 / (float)kept, r1 = (float)h->n1 / (float)kept;
         float d = activation_density(r0, r1, rad * p.PixelSize / 1000);
         d = p.MultiEmitterFitEn ? d * d * 0.5098f + d * 0.6364f : d * d * 0.8082f + d * 0.519f;
         out->loc_density_2d = d;

@@ -1,0 +1,81 @@
+"""The scans, the row sort and the neighbour table at the edges of their launches, exactly as the oracle:
+one-launch and two-launch scans and their tiles, one to four digits of the frame, rows at every digit's end,
+bucket tables of the smallest and of larger sizes."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as O
+import qcstorm as Q
+from test_gpu_stats import _check
+from test_gpu_stats import _rows as _stat_rows
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(n, seed, frames):
+    rng = np.random.default_rng(seed)
+    loc = rng.normal(0, 1, (n, 12)).astype(np.float32)
+    loc[:, 0] = rng.choice([0.0, 0.5, 1.0, 1.5, 2.0, 400.0, np.nan], n)
+    loc[:, 11] = rng.choice(frames, n)
+    return loc
+
+
+# 2048 rows are a tile of the sort, 4096 / 16384 items a tile of the two-launch / one-launch scan; the sort
+# scans 256 counts a tile, so 131,072 rows (64 tiles) are the last with one launch
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 2047, 2048, 2049, 4097, 16383, 16384, 16385, 20481, 131072, 131073])
+def test_rows_sorted_and_unsorted(gpu, n):
+    loc = _rows(n, n, np.arange(1, 40))
+    ctx = Q.Context(Q.default_params(ImageWidth=64, ImageHigh=64))
+    d = torch.from_numpy(loc).cuda()
+    out = torch.full_like(d, -7.0)
+    m = ctx.compact_sorted_dev(d, n, 3, 30, out)
+    ref = O.compact_sorted(loc, 3, 30)
+    assert m == len(ref)
+    np.testing.assert_array_equal(out[:m].cpu().numpy(), ref)
+    assert bool((out[m:] == -7.0).all())
+    out.fill_(-7.0)
+    m = ctx.compact_dev(d, n, out)
+    keep = loc[loc[:, 0] > 1.0]
+    assert m == len(keep)
+    np.testing.assert_array_equal(out[:m].cpu().numpy(), keep)
+    assert bool((out[m:] == -7.0).all())
+
+
+@pytest.mark.parametrize("first,end", [(0, 0), (5, 260), (5, 261), (-300, -45), (-300, 65235), (-300, 65236), (0, 1 << 24),
+                                       (-(1 << 24), 1 << 24), (-(1 << 31), (1 << 31) - 1)])
+def test_frame_digits(gpu, first, end):
+    n = 5000
+    mid = (first + end) // 2
+    frames = np.array([first - 1, first, first + 1, first + 255, first + 256, mid, mid + 1, end - 256, end - 1, end, end + 1, np.nan,
+                       np.inf, -np.inf], np.float64).astype(np.float32)
+    loc = _rows(n, 3, frames)
+    ctx = Q.Context(Q.default_params(ImageWidth=64, ImageHigh=64))
+    d = torch.from_numpy(loc).cuda()
+    out = torch.empty_like(d)
+    m = ctx.compact_sorted_dev(d, n, first, end, out)
+    # the oracle counts every frame of the range: past 2^25 of them its definition is written out here
+    if end - first < 1 << 25:
+        ref = O.compact_sorted(loc, first, end)
+    else:
+        with np.errstate(invalid="ignore"):
+            fr = np.clip(np.nan_to_num(loc[:, 11].astype(np.float64), nan=0.0), -2.0**31, 2.0**31 - 1).astype(np.int64)
+        keep = np.flatnonzero((np.trunc(np.nan_to_num(loc[:, 0])) > 1) & (fr >= first) & (fr <= end))
+        ref = loc[keep[np.argsort(fr[keep], kind="stable")]]
+    assert m == len(ref) and m > 0
+    np.testing.assert_array_equal(out[:m].cpu().numpy(), ref)
+
+
+# 256 buckets are the fewest; 512 rows are a work-group of the row pass, 16 molecules one of the neighbour pass
+@pytest.mark.parametrize("n,nframes,dense", [(1, 1, False), (2, 1, True), (17, 2, True), (255, 3, True), (257, 4, True), (513, 5, False),
+                                             (4099, 2, True), (16385, 500, True), (40000, 6, True)])
+def test_stats_table(gpu, n, nframes, dense):
+    p = Q.default_params(ImageWidth=333, ImageHigh=250)
+    _check(p, _stat_rows(n, n, nframes, 333, 250, dense))
+
+
+def test_stats_far_apart_frames(gpu):
+    p = Q.default_params(ImageWidth=100, ImageHigh=64)
+    loc = _stat_rows(700, 9, 5, 100, 64, True)
+    loc[:, 11] = np.sort(np.random.default_rng(1).choice([-70000.0, -3.0, 0.0, 1.0, 123456.0], 700)).astype(np.float32)
+    _check(p, loc)
