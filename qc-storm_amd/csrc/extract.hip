@@ -16,7 +16,7 @@
 //   1. walk_kernel<0>     background-removed values over each batch's variance region
 //   2. var_reduce_kernel  exact integer sums of the variance samples per batch
 //   3. walk_kernel<1>     one wave per 56-column strip walks down the rows: raw rows enter a
-//                         9-row LDS ring, background removal, 5-tap H and V smoothing (uint16
+//                         16-row LDS ring, background removal, 5-tap H and V smoothing (uint16
 //                         truncation after each pass, as the reference stores them), 3x3
 //                         local-maximum test against the batch's thresholds.  Candidates and
 //                         marks leave as one 56-bit ballot mask per row and strip; per-row
@@ -74,7 +74,8 @@ struct ExtractConst {
     int cap;               // output capacity
     int start_frame;
     int nseg;              // SEGW-column segments per row (one walking wave each)
-    int walk_rows;         // image rows per walking wave
+    int walk_rows;         // image rows per walking wave of the full pass
+    int var_rows;          // ... of the variance region's
     float taps[5];
     const int *start_dev;  // when set: the call's first frame number is read here at run time (graph replays)
 };
@@ -143,12 +144,16 @@ __device__ __forceinline__ void batch_thresholds(const ExtractConst &c, const un
 //              gpuImageConv_Seperable_H/V, SE/LDROIExtraction_ImageFiltering.cu:286-470);
 //   detection of rows r-3..r once sv(r+1) exists (gpuROIFindingLD,
 //   SE/LDROIExtraction_ROIExtraction.cu:25-164).
-// Only the raw rows go through LDS (one barrier per step, after they are staged).  The other
-// cross-lane values -- the neighbours' background sums, tv of lanes l-2..l+2 for the H pass and
-// sv of lanes l-1, l+1 for detection -- move between lanes by DPP wave shifts, which keeps the
-// step's chain of dependent LDS round trips short; the lanes whose results are used never reach
-// past the wave, and a strip at the image border takes its clamped columns by readlane.  hc stays
-// in a lane-local LDS ring, sv in registers.
+// Only the raw rows go through LDS (one barrier per step, after they are staged), as the 16-bit
+// pairs (R(x), R(x+1)) of every column: the sums take two neighbouring terms per instruction from
+// pairs that start at any column, and a pair read whole is an aligned word with one bank a lane.
+// (Reading eight 16-bit columns at the lane's odd address as one 16-byte word kept the LDS busy 92% of
+// the pass, 83% of it in stalls for the alignment.)  Everything else moves between lanes by DPP wave
+// shifts, mostly inside the instruction that uses it -- the neighbours' background sums, tv of
+// lanes l-2..l+2 for the H pass, sv of lanes l-1, l+1 for detection -- and between rows in registers;
+// the lanes whose results are used never reach past the wave, and a strip at the image border takes
+// its clamped columns by readlane.  Rows with no pixel at the threshold, most of them, stop there.
+// What bounds the full pass is instruction issue: 32 frames of 2048 x 2048, 720 -> 410 us.
 // MODE 0 computes tv only, over the variance region, into tvbuf; MODE 1 is the full pass.
 // Wave shifts by one lane (DPP wave_shr:1 / wave_shl:1).  Bound control writes 0 where the
 // source lane is outside the wave (lane 0 for prev, lane 63 for next), so no old value is needed.
@@ -157,15 +162,39 @@ __device__ __forceinline__ int lane_next(int v) { return __builtin_amdgcn_mov_dp
 __device__ __forceinline__ float lane_prev(float v) { return __int_as_float(lane_prev(__float_as_int(v))); }
 __device__ __forceinline__ float lane_next(float v) { return __int_as_float(lane_next(__float_as_int(v))); }
 
+// acc[k] += x[k] of lane l - 1 (PREV) or l + 1, times w, for four rows: the shift is part of the
+// instruction (the compiler makes it a move of its own before a multiply-add).  A DPP operand needs two
+// wait states after the instruction that wrote it, once for the four.
+template <bool PREV>
+__device__ __forceinline__ void fma_shifted(float (&acc)[4], const float (&x)[4], float w)
+{
+    if constexpr (PREV)
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %4, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %1, %5, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %2, %6, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %3, %7, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w));
+    else
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %4, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %1, %5, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %2, %6, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %3, %7, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w));
+}
+
 // two 16-bit lanes of a 32-bit register
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u16x2 as_u16x2(uint32_t w) { return __builtin_bit_cast(u16x2, w); }
 __device__ __forceinline__ u16x2 swap16(u16x2 v) { return __builtin_shufflevector(v, v, 1, 0); }
 __device__ __forceinline__ u16x2 pmin16(u16x2 a, u16x2 b) { return __builtin_elementwise_min(a, b); }
 constexpr u16x2 kOnes16 = {1, 1};
+typedef uint32_t __attribute__((may_alias)) u32_alias;
 
 constexpr int SEGW = 56;             // output columns per wave
-constexpr int RAWW = 72;             // raw row width in LDS
+constexpr int RAWW = 72;             // raw columns per row in LDS
+constexpr int ROWW = 2 * RAWW + 2;   // 16-bit words per row of pairs: column x is words 2x + 2 and 2x + 1
 constexpr int VAR_MAX = 512;         // region side bound (2 * 256)
 
 constexpr int WALK_RS = 4;   // image rows per step
@@ -179,7 +208,7 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
                                           uint16_t *__restrict__ tvbuf,
                                           unsigned long long *__restrict__ cand_mask,
                                           unsigned long long *__restrict__ mark_mask,
-                                          int *__restrict__ row_count, uint16_t (*raw)[RAWW], float (*hcs)[64])
+                                          int *__restrict__ row_count, uint16_t (*raw)[ROWW])
 {
     constexpr int RS = WALK_RS;
     constexpr int NR = WALK_NR;
@@ -199,9 +228,9 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
         ry0 = BH / 2 - S;
         x0 = rx0 + blockIdx.x * SEGW;
         if (x0 >= rx0 + 2 * S) return;
-        ys = ry0 + blockIdx.y * c.walk_rows;
+        ys = ry0 + blockIdx.y * c.var_rows;
         if (ys >= ry0 + 2 * S) return;
-        ye = min(ys + c.walk_rows, ry0 + 2 * S);
+        ye = min(ys + c.var_rows, ry0 + 2 * S);
         rb = ys;          // steps compute tv rows r .. r+3
         rlast = ye - 1;
     } else {
@@ -215,7 +244,6 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
     // ring slots are relative to rb; a step starts at rb + 4 * (4n + PH), so in interior steps the
     // slots are compile-time functions of the phase PH
     auto slot = [&](int v) { return (v - rb + 2 * NR) & (NR - 1); };
-    auto ring8 = [&](int v) { return (v - rb + 16) & 7; };
     const int xc = x0 - 4 + l;
     const int xcl = clampi(xc, 0, W - 1);
     // halo columns: lanes 0..3 -> x0-8+l (slot l), lanes 4..7 -> x0+60+(l-4) (slot 68+l-4)
@@ -227,11 +255,25 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
     };
     auto ld = [&](int v, uint16_t &main, uint16_t &halo) { ldp(img + (unsigned)(clampi(v, 0, BH - 1) * W), main, halo); };
 
+    // Column x of a row: the first half of pair x and the second half of pair x - 1.  The latter's place
+    // is kept from the compiler, which else joins the two into one store at an odd word: any LDS access
+    // that is not aligned to its size takes 64 cycles, one a lane, an aligned one 3 to 5.
+    int m2 = 2 * (l + 4) + 1, h2 = 2 * hslot + 1;
+    asm("" : "+v"(m2), "+v"(h2));
+    auto put = [&](int rs, uint16_t m, uint16_t h) {
+        raw[rs][2 * (l + 4) + 2] = m;
+        raw[rs][m2] = m;
+        if (l < 8) {
+            raw[rs][2 * hslot + 2] = h;
+            raw[rs][h2] = h;
+        }
+    };
+    auto col = [&](int rs, int x) { return (uint32_t)raw[rs][2 * x + 2]; };
+    auto pair = [&](int rs, int x) { return *reinterpret_cast<const u32_alias *>(&raw[rs][2 * x + 2]); };
     for (int v = rb - 4; v < rb + 4; v++) {
         uint16_t m, h;
         ld(v, m, h);
-        raw[slot(v)][l + 4] = m;
-        if (l < 8) raw[slot(v)][hslot] = h;
+        put(slot(v), m, h);
     }
     uint16_t pf[RS], pfh[RS];
 #pragma unroll
@@ -247,6 +289,9 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
     const int g0 = xc & ~31;
     const int li = max(min(((xc - 1 < g0) ? g0 : xc - 1) - (x0 - 4), 63), 0);
     const int ri = max(min(((xc + 1 > g0 + 31) ? g0 + 31 : xc + 1) - (x0 - 4), 63), 0);
+    // weights of the three sums in the background, -1/24 each
+    const float wc = -(float)(1 + (li == l ? 1 : 0) + (ri == l ? 1 : 0)) / 24.0f, wl = li == l ? 0.0f : -1.0f / 24.0f,
+                wr = ri == l ? 0.0f : -1.0f / 24.0f;
     int hci[5];   // H-pass source lanes (columns clamped to the image)
 #pragma unroll
     for (int t = 0; t < 5; t++) hci[t] = max(min(clampi(xc - 2 + t, 0, W - 1) - (x0 - 4), 63), 0);
@@ -255,24 +300,35 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
     const int half = c.R / 2;
     const bool out_lane = (l >= 4 && l < 4 + SEGW);
     const bool det_col = out_lane && xc < W && xc >= half && xc < W - half;
+    const float thc = det_col ? th : 3.0e38f;   // no value reaches it outside the detection columns
     const int ylo = max(ys - 1, 0), yhi = min(ye, BH - 1);   // sv rows this wave needs
     unsigned long long *cmask = cand_mask + (size_t)b * c.B * c.H * c.nseg + seg;
     unsigned long long *mmask = mark_mask + (size_t)b * c.B * c.H * c.nseg + seg;
     int *rcount = row_count + (size_t)b * c.B * c.H;
     const int nseg = c.nseg, H = c.H;
     int ryd = ((rb - 3) % H + H) % H;   // frame row of detection row r-3 for the current step
-    // raw columns xc+4 (rows r-4 .. r+6) and xc-4 (rows r-3 .. r+7) of the current step; an
-    // interior step after another step keeps the previous step's seven newest rows of each and
-    // reads four from LDS (a walk's first step may be interior: then all eleven are read)
-    int colR[RS + 7], colL[RS + 7];
-    u16x2 CR[RS + 6], CL[RS + 6];
-    bool have_cols = false;   // uniform
-    // the lane's V-smoothed rows r-4 .. r+RS-3: [0, 2) from the previous step, [2, RS+2) this
-    // step's V pass; detection takes lanes l-1 and l+1 of them by DPP wave shifts
-    float svr[RS + 2];
-    int lor[RS + 2];
+    // 16-bit pairs (col[m], col[m+1]) of raw column xc+4 from row r-4 and of column xc-4 from row r-3.  A
+    // step keeps the previous step's six newest; of the new ones, column xc+4 is in the pairs that
+    // the sums read (rows r+4 .. r+6 in this step's, r+3 in the last step's), and so is the centre
+    // of the rows (in the last step's).
+    uint32_t CR[RS + 6], CL[RS + 6], b3, cen[RS];
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < RS + 2; i++) { svr[i] = 0.0f; lor[i] = 0; }
+    for (int m = 0; m < 6; m++) {   // as a step before the first would leave them
+        CR[RS + m] = col(slot(rb + m - 4), l + 8) | col(slot(rb + m - 3), l + 8) << 16;
+        CL[RS + m] = col(slot(rb + m - 3), l) | col(slot(rb + m - 2), l) << 16;
+    }
+    b3 = col(slot(rb + 3), l + 8) << 16;
+#pragma unroll
+    for (int k = 0; k < RS; k++) cen[k] = col(slot(rb + k), l + 4) << 16;
+    // the lane's H-smoothed rows r-4 .. r+RS-1 and V-smoothed rows r-4 .. r+RS-3: the last RS rows are
+    // this step's; detection takes lanes l-1 and l+1 of the latter by DPP wave shifts
+    float hcr[RS + 4], svr[RS + 2];
+#pragma unroll
+    for (int i = 0; i < RS + 4; i++) hcr[i] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < RS + 2; i++) svr[i] = 0.0f;
+    const unsigned moff = (unsigned)l * (unsigned)c.nseg;   // lanes 0 .. RS-1: their row of a step's masks
 
     // One step of 4 rows.  EDGE: rows near the batch or walk ends (bounds checks, clamped rows,
     // dynamic ring slots); otherwise every row is in range and PH fixes the ring slots.
@@ -280,13 +336,9 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
         constexpr bool EDGE = decltype(edge_tag)::value;
         constexpr int PH = decltype(ph_tag)::value;
         auto rs = [&](int off) { if constexpr (EDGE) return slot(r + off); else return (4 * PH + off + 2 * NR) & (NR - 1); };
-        auto h8 = [&](int off) { if constexpr (EDGE) return ring8(r + off); else return (4 * PH + off + 16) & 7; };
         // stage rows r+4 .. r+7 (loaded one step ago), then prefetch rows r+8 .. r+11
 #pragma unroll
-        for (int k = 0; k < RS; k++) {
-            raw[rs(4 + k)][l + 4] = pf[k];
-            if (l < 8) raw[rs(4 + k)][hslot] = pfh[k];
-        }
+        for (int k = 0; k < RS; k++) put(rs(4 + k), pf[k], pfh[k]);
         if constexpr (EDGE) {
 #pragma unroll
             for (int k = 0; k < RS; k++) ld(r + 8 + k, pf[k], pfh[k]);
@@ -297,70 +349,50 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
         }
         __syncthreads();
         // background sums of rows r .. r+3
-        // CR[m] / CL[m]: the 16-bit pairs (col[m], col[m+1]) of the two columns
-        auto pack = [&](int m) {
-            CR[m] = as_u16x2((uint32_t)colR[m] | ((uint32_t)colR[m + 1] << 16));
-            CL[m] = as_u16x2((uint32_t)colL[m] | ((uint32_t)colL[m + 1] << 16));
-        };
-        if (EDGE || !have_cols) {
 #pragma unroll
-            for (int i = 0; i < RS + 7; i++) {
-                colR[i] = raw[rs(i - 4)][l + 8];
-                colL[i] = raw[rs(i - 3)][l];
-            }
-#pragma unroll
-            for (int m = 0; m < RS + 6; m++) pack(m);
-            have_cols = true;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 7; i++) {
-                colR[i] = colR[i + RS];
-                colL[i] = colL[i + RS];
-            }
-#pragma unroll
-            for (int i = 7; i < RS + 7; i++) {
-                colR[i] = raw[rs(i - 4)][l + 8];
-                colL[i] = raw[rs(i - 3)][l];
-            }
-#pragma unroll
-            for (int m = 0; m < 6; m++) {
-                CR[m] = CR[m + RS];
-                CL[m] = CL[m + RS];
-            }
-#pragma unroll
-            for (int m = 6; m < RS + 6; m++) pack(m);
+        for (int m = 0; m < 6; m++) {
+            CR[m] = CR[m + RS];
+            CL[m] = CL[m + RS];
         }
         // Two terms per instruction: term i takes rA[l+i], colR[k+i], rB[l+8-i] and colL[k+7-i],
         // so terms 2j and 2j+1 read the 16-bit pairs (rA[l+2j], rA[l+2j+1]) and
         // (colR[k+2j], colR[k+2j+1]) in order and (rB[l+7-2j], rB[l+8-2j]) and
         // (colL[k+6-2j], colL[k+7-2j]) with their halves swapped.  Packed 16-bit minima, then a
         // dot product with (1, 1) adds both halves into the 32-bit sum.
-        int bkv[RS];
+        float bkv[RS];
+        uint32_t cn[RS], cl = CL[5] >> 16;
 #pragma unroll
         for (int k = 0; k < RS; k++) {
-            uint4 A, B;   // rA[l .. l+7], rB[l+1 .. l+8]
-            __builtin_memcpy(&A, &raw[rs(k - 4)][l], sizeof A);
-            __builtin_memcpy(&B, &raw[rs(k + 4)][l + 1], sizeof B);
-            const uint32_t aw[4] = {A.x, A.y, A.z, A.w}, bw[4] = {B.w, B.z, B.y, B.x};
+            CR[6 + k] = __builtin_amdgcn_perm(b3, CR[5 + k], 0x07060302);   // the upper halves of both
+            const uint32_t c = col(rs(k + 4), l);
+            CL[6 + k] = cl | c << 16;
+            cl = c;
             uint32_t bk = 0;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const u16x2 m1 = pmin16(as_u16x2(aw[j]), CR[k + 2 * j]);
-                const u16x2 m2 = pmin16(swap16(as_u16x2(bw[j])), swap16(CL[k + 6 - 2 * j]));
+                const uint32_t bp = pair(rs(k + 4), l + 7 - 2 * j);
+                if (j == 0) b3 = bp;
+                if (j == 2) cn[k] = bp;
+                const u16x2 m1 = pmin16(as_u16x2(pair(rs(k - 4), l + 2 * j)), as_u16x2(CR[k + 2 * j]));
+                const u16x2 m2 = pmin16(swap16(as_u16x2(bp)), swap16(as_u16x2(CL[k + 6 - 2 * j])));
                 bk = __builtin_amdgcn_udot2(pmin16(m1, m2), kOnes16, bk, false);
             }
-            bkv[k] = (int)bk;
+            bkv[k] = (float)bk;
         }
-        // the neighbours' sums by DPP wave shifts: li is l - 1 or l, ri is l or l + 1
-        int tvk[RS];
+        // tv = max(raw - ceil(S / 24), 0), S the three sums' total, as trunc(max(raw - S / 24 + 1/48, 0)) in
+        // float: raw - S / 24 is a multiple of 1/24, so with the 1/48 it is that far from every integer,
+        // and the four roundings (2^-9 each, no value reaches 2^16) and those of the weights
+        // (65535 * 2^-24) add up to less than 0.012.
+        float tvk[RS];
 #pragma unroll
         for (int k = 0; k < RS; k++) {
-            const int bm = lane_prev(bkv[k]), bp = lane_next(bkv[k]);
-            const int bl = li == l ? bkv[k] : bm, br = ri == l ? bkv[k] : bp;
-            const int rawc = raw[rs(k)][l + 4];
-            const int t = rawc - (bl + bkv[k] + br + 23) / 24;
-            tvk[k] = t > 0 ? t : 0;
+            tvk[k] = __builtin_fmaf(bkv[k], wc, (float)(cen[k] >> 16) + 1.0f / 48.0f);
+            cen[k] = cn[k];
         }
+        fma_shifted<true>(tvk, bkv, wl);
+        fma_shifted<false>(tvk, bkv, wr);
+#pragma unroll
+        for (int k = 0; k < RS; k++) tvk[k] = __builtin_truncf(fmaxf(tvk[k], 0.0f));
         if constexpr (MODE == 0) {
 #pragma unroll
             for (int k = 0; k < RS; k++) {
@@ -370,92 +402,129 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
             }
             return;
         }
-        // H pass into the lane's ring (rows inside the batch only).  The values of lanes l-2 .. l+2
-        // come by DPP wave shifts; a strip at the image border takes its clamped columns from the
-        // border lane (readlane).  Lanes 3 .. 60, the ones whose results are used, never read a
-        // lane outside the wave.
+        // H pass.  The values of lanes l-2 .. l+2 come by DPP wave shifts; a strip at the image border
+        // takes its clamped columns from the border lane (readlane).  Lanes 3 .. 60, the ones whose
+        // results are used, never read a lane outside the wave.  Rows outside the batch repeat its
+        // first and last row.
+        float h0 = hcr[RS], h1 = hcr[RS + 1], h2 = hcr[RS + 2], h3 = hcr[RS + 3], hn[RS];
+        float hv[RS];
+        if constexpr (!SMOOTH) {
 #pragma unroll
-        for (int k = 0; k < RS; k++) {
-            if (EDGE && (r + k < 0 || r + k >= BH)) continue;   // uniform
-            float hc;
-            if constexpr (SMOOTH) {
-                const float v0 = (float)tvk[k];
-                const float m1 = lane_prev(v0), m2 = lane_prev(m1);   // lanes l-1, l-2
-                const float p1 = lane_next(v0), p2 = lane_next(p1);   // lanes l+1, l+2
-                float src[5] = {m2, m1, v0, p1, p2};
-                if constexpr (BORDER) {
+            for (int k = 0; k < RS; k++) hv[k] = tvk[k];
+        } else {
+            // no value is negative: the first tap's product has the bits of fma(src, tap, 0)
+            float m1[RS], p1[RS];   // lanes l-1, l+1
+#pragma unroll
+            for (int k = 0; k < RS; k++) {
+                m1[k] = lane_prev(tvk[k]);
+                p1[k] = lane_next(tvk[k]);
+            }
+            if constexpr (BORDER) {
+#pragma unroll
+                for (int k = 0; k < RS; k++) {
+                    const float v0 = tvk[k];
+                    float src[5] = {lane_prev(m1[k]), m1[k], v0, p1[k], lane_next(p1[k])};
                     const float vl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v0), lane_lo));
                     const float vr = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v0), lane_hi));
 #pragma unroll
                     for (int t = 0; t < 5; t++) src[t] = hci[t] == lane_lo ? vl : (hci[t] == lane_hi ? vr : src[t]);
-                }
-                float acc = 0.0f;
+                    float acc = src[0] * tap[0];
 #pragma unroll
-                for (int t = 0; t < 5; t++) acc = __builtin_fmaf(src[t], tap[t], acc);
-                acc = acc > 65535.0f ? 65535.0f : acc;
-                hc = __builtin_truncf(acc);   // acc >= 0: the uint16 store's truncation
+                    for (int t = 1; t < 5; t++) acc = __builtin_fmaf(src[t], tap[t], acc);
+                    hv[k] = acc;
+                }
             } else {
-                hc = (float)tvk[k];
+#pragma unroll
+                for (int k = 0; k < RS; k++) hv[k] = 0.0f;
+                fma_shifted<true>(hv, m1, tap[0]);
+#pragma unroll
+                for (int k = 0; k < RS; k++)
+                    hv[k] = __builtin_fmaf(p1[k], tap[3], __builtin_fmaf(tvk[k], tap[2], __builtin_fmaf(m1[k], tap[1], hv[k])));
+                fma_shifted<false>(hv, p1, tap[4]);
             }
-            hcs[h8(k)][l] = hc;
+#pragma unroll
+            for (int k = 0; k < RS; k++) hv[k] = __builtin_truncf(fminf(hv[k], 65535.0f));   // >= 0: the uint16 store's truncation
         }
-        // V pass: sv rows r-2 .. r+1 (hc rows clamped to the batch), held as integral floats, and
-        // whether each is at most th1
 #pragma unroll
         for (int k = 0; k < RS; k++) {
-            const int y = r - 2 + k;
-            if (EDGE && (y < ylo || y > yhi)) continue;   // uniform
-            float sv;
+            if (EDGE && r + k >= BH) {   // uniform
+                hn[k] = k > 0 ? hn[k - 1] : h3;
+                continue;
+            }
+            hn[k] = hv[k];
+            if (EDGE && r + k <= 0) {   // uniform
+                h0 = h1 = h2 = h3 = hv[k];
+#pragma unroll
+                for (int i = 0; i < k; i++) hn[i] = hv[k];
+            }
+        }
+        hcr[0] = h0;
+        hcr[1] = h1;
+        hcr[2] = h2;
+        hcr[3] = h3;
+#pragma unroll
+        for (int k = 0; k < RS; k++) hcr[RS + k] = hn[k];
+        // V pass: sv rows r-2 .. r+1, held as integral floats
+#pragma unroll
+        for (int k = 0; k < RS; k++) {
+            float sv = hcr[k + 2];
             if constexpr (SMOOTH) {
-                float acc = 0.0f;
+                float acc = hcr[k] * tap[0];
 #pragma unroll
-                for (int t = 0; t < 5; t++) {
-                    float hv;
-                    if constexpr (EDGE) hv = hcs[ring8(clampi(y - 2 + t, 0, BH - 1))][l];
-                    else hv = hcs[h8(k - 4 + t)][l];
-                    acc = __builtin_fmaf(hv, tap[t], acc);
-                }
-                acc = acc > 65535.0f ? 65535.0f : acc;
-                sv = __builtin_truncf(acc);
-            } else {
-                sv = hcs[h8(k - 2)][l];
+                for (int t = 1; t < 5; t++) acc = __builtin_fmaf(hcr[k + t], tap[t], acc);
+                sv = __builtin_truncf(fminf(acc, 65535.0f));
             }
+            if (EDGE && (r - 2 + k < ylo || r - 2 + k > yhi)) sv = 0.0f;   // uniform
             svr[2 + k] = sv;
-            lor[2 + k] = (sv > th1) ? 0 : 1;
         }
-        // detection rows r-3 .. r (sv rows r-4 .. r+1); the shifts run on the whole wave, ahead
-        // of the per-lane tests.  The eight-neighbour count s8 >= 7 of the reference is "at most one
-        // neighbour <= th1": with cv >= th > th1 the centre is not one of them, so it is the 3 x 3
-        // count of the low flags (column sums, then lanes l-1, l, l+1) being at most one.
+        // detection rows r-3 .. r (sv rows r-4 .. r+1) that have a pixel at the threshold; the shifts
+        // run on the whole wave, ahead of the per-lane tests.  The eight-neighbour count s8 >= 7 of the
+        // reference is "at most one neighbour <= th1": with cv >= th > th1 the centre is not one of them, so
+        // it is the 3 x 3 count of the low flags (column sums, then lanes l-1, l, l+1) being at most one.
+        unsigned long long hit[RS];
+        bool any = false;
 #pragma unroll
         for (int k = 0; k < RS; k++) {
-            const int d = r - 3 + k;
             int ry = ryd + k;
             ry = ry >= H ? ry - H : ry;
-            if (EDGE && (d < ys || d >= ye)) continue;   // uniform
-            const float p01 = svr[k], cv = svr[k + 1], p21 = svr[k + 2];
-            const float p00 = lane_prev(p01), p02 = lane_next(p01);
-            const float p10 = lane_prev(cv), p12 = lane_next(cv);
-            const float p20 = lane_prev(p21), p22 = lane_next(p21);
-            const int lc = lor[k] + lor[k + 1] + lor[k + 2];
-            const int low9 = lane_prev(lc) + lc + lane_next(lc);
-            const bool sin4 = (cv > p01) && (cv >= p12) && (cv >= p21) && (cv > p10);
-            const bool a = cv > p00, bb = cv > p02, cc = cv > p20, dd = cv > p22;
-            const bool sout3 = (a && bb && (cc || dd)) || (cc && dd && (a || bb));
-            const bool mark = det_col && ry >= half && ry < H - half && cv >= th && low9 <= 1 && sin4 && sout3;
-            const bool cand = mark && a && bb && cc && dd;
-            const unsigned long long cm = (__ballot(cand) >> 4) & ((1ULL << SEGW) - 1);
-            const unsigned long long mm = (__ballot(mark) >> 4) & ((1ULL << SEGW) - 1);
-            if (l == 0) {
-                cmask[(size_t)d * nseg] = cm;
-                mmask[(size_t)d * nseg] = mm;
-                if (cm) atomicAdd(&rcount[d], __popcll(cm));
+            const unsigned long long m = __ballot(svr[k + 1] >= thc);
+            hit[k] = ry >= half && ry < H - half ? m : 0ull;
+            any |= hit[k] != 0;
+        }
+        if (!EDGE && !any) {   // uniform
+            if (l < RS) {
+                cmask[(size_t)(r - 3) * nseg + moff] = 0;
+                mmask[(size_t)(r - 3) * nseg + moff] = 0;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < RS; k++) {
+                const int d = r - 3 + k;
+                if (EDGE && (d < ys || d >= ye)) continue;   // uniform
+                unsigned long long cm = 0, mm = 0;
+                const float p01 = svr[k], cv = svr[k + 1], p21 = svr[k + 2];
+                if (hit[k] && __ballot((cv >= thc) & (cv > p01) & (cv >= p21))) {   // uniform
+                    const float p00 = lane_prev(p01), p02 = lane_next(p01);
+                    const float p10 = lane_prev(cv), p12 = lane_next(cv);
+                    const float p20 = lane_prev(p21), p22 = lane_next(p21);
+                    const int lc = (p01 > th1 ? 0 : 1) + (cv > th1 ? 0 : 1) + (p21 > th1 ? 0 : 1);
+                    const int low9 = lane_prev(lc) + lc + lane_next(lc);
+                    const bool sin4 = (cv > p01) & (cv >= p12) & (cv >= p21) & (cv > p10);
+                    const bool a = cv > p00, bb = cv > p02, cc = cv > p20, dd = cv > p22;
+                    const bool sout3 = (a & bb & (cc | dd)) | (cc & dd & (a | bb));
+                    const bool mark = (cv >= thc) & (low9 <= 1) & sin4 & sout3;
+                    cm = (__ballot(mark & a & bb & cc & dd) >> 4) & ((1ULL << SEGW) - 1);
+                    mm = (__ballot(mark) >> 4) & ((1ULL << SEGW) - 1);
+                }
+                if (l == 0) {
+                    cmask[(size_t)d * nseg] = cm;
+                    mmask[(size_t)d * nseg] = mm;
+                    if (cm) atomicAdd(&rcount[d], __popcll(cm));
+                }
             }
         }
         svr[0] = svr[RS];
         svr[1] = svr[RS + 1];
-        lor[0] = lor[RS];
-        lor[1] = lor[RS + 1];
     };
 
     using E = std::true_type;
@@ -479,9 +548,8 @@ __device__ __forceinline__ void walk_body(const uint16_t *__restrict__ frames, c
     }
 }
 
-// The full pass is held to five waves per SIMD (at most 102 VGPRs, no spills): its steps are chains
-// of dependent LDS round trips, and the fifth wave hides a little more of them (1% faster than
-// four; six spill).
+// The full pass is held to five waves per SIMD (at most 96 VGPRs, no spills; six spill): issue slots are
+// 85% taken.
 template <int MODE, bool SMOOTH>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE == 1 ? 5 : 1))) walk_kernel(const uint16_t *__restrict__ frames, ExtractConst c,
                                                   const unsigned long long *__restrict__ var_sums,
@@ -490,13 +558,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE ==
                                                   unsigned long long *__restrict__ mark_mask,
                                                   int *__restrict__ row_count)
 {
-    __shared__ uint16_t raw[WALK_NR][RAWW];
-    __shared__ float hcs[8][64];   // lane-local ring of H-smoothed rows
+    __shared__ __align__(4) uint16_t raw[WALK_NR][ROWW];
     const int xs = (int)blockIdx.x * SEGW;
     if (MODE == 1 && (xs - 4 + 1 < 2 || xs - 4 + 62 > c.W - 3))   // uniform
-        walk_body<MODE, SMOOTH, true>(frames, c, var_sums, tvbuf, cand_mask, mark_mask, row_count, raw, hcs);
+        walk_body<MODE, SMOOTH, true>(frames, c, var_sums, tvbuf, cand_mask, mark_mask, row_count, raw);
     else
-        walk_body<MODE, SMOOTH, false>(frames, c, var_sums, tvbuf, cand_mask, mark_mask, row_count, raw, hcs);
+        walk_body<MODE, SMOOTH, false>(frames, c, var_sums, tvbuf, cand_mask, mark_mask, row_count, raw);
 }
 
 // integer sums of the variance samples of each batch from the region's background-removed values
@@ -927,13 +994,27 @@ static int extract_candidates(qcs_ctx *ctx, const qcs_params &p, const uint16_t 
     c.start_dev = d_start;
     c.nseg = (c.W + SEGW - 1) / SEGW;
     filter_taps_host(R, p.LocType, p.MultiEmitterFitEn, c.taps);
-    // rows per walking wave: long walks amortise the 14-row pipeline fill; shorter ones keep
-    // small calls spread over the chip
+    // Rows per walking wave: long walks amortise the 14-row pipeline fill (32 frames of 2048 x 2048 at 96,
+    // 128, 256 and 512 rows: 413, 410, 426 and 445 us); shorter ones keep small calls spread over the
+    // chip, the shortest while there is not a wave for every SIMD (one frame of 256 x 256 at 8, 16 and 32
+    // rows: 13, 16 and 23 us).
     const int rows_per_batch = c.B * c.H;
+    auto waves = [&](int strips, int rows, int per) { return (long long)strips * ((rows + per - 1) / per) * c.nbatch; };
     c.walk_rows = 128;
-    while (c.walk_rows > 16 &&
-           (long long)c.nseg * ((rows_per_batch + c.walk_rows - 1) / c.walk_rows) * c.nbatch < 8192)
-        c.walk_rows /= 2;
+    while (c.walk_rows > 8 && waves(c.nseg, rows_per_batch, c.walk_rows) < (c.walk_rows > 16 ? 8192 : 1024)) c.walk_rows /= 2;
+    // variance region extent (largest over the batches: the first batch is a full one) and its walks
+    // (8 rows of fill; 32 regions of 512 x 512 at 16, 32, 64 and 128 rows: 35, 32, 39 and 58 us; one of
+    // 246 x 246 at 8, 16 and 32 rows: 9, 13 and 17 us)
+    int Smax;
+    {
+        int sw = c.W / 2 - 5, sh = rows_per_batch / 2 - 5;
+        sw = sw > 256 ? 256 : (sw < 1 ? 1 : sw);
+        sh = sh > 256 ? 256 : (sh < 1 ? 1 : sh);
+        Smax = sw < sh ? sw : sh;
+    }
+    const int var_strips = (2 * Smax + SEGW - 1) / SEGW;
+    c.var_rows = 32;
+    while (c.var_rows > 8 && waves(var_strips, 2 * Smax, c.var_rows) < 4096) c.var_rows /= 2;
 
     const size_t nrows = (size_t)nframes * c.H;
     if (nrows > (size_t)SCAN_TILE * SCAN_TILE) return fail(QCS_ERR_ARG, "too many rows in one extraction call");
@@ -957,17 +1038,9 @@ static int extract_candidates(qcs_ctx *ctx, const qcs_params &p, const uint16_t 
     int *info = ctx->ex_tmp.as<int>();
     int3 *xyb = ctx->ex_xy.as<int3>();
 
-    // variance region extent (largest over the batches: the first batch is a full one)
-    int Smax;
-    {
-        int sw = c.W / 2 - 5, sh = rows_per_batch / 2 - 5;
-        sw = sw > 256 ? 256 : (sw < 1 ? 1 : sw);
-        sh = sh > 256 ? 256 : (sh < 1 ? 1 : sh);
-        Smax = sw < sh ? sw : sh;
-    }
     fill_async(reinterpret_cast<int *>(var_sums), 4 * (size_t)c.nbatch, 0, s);
     fill_async(row_count, nrows, 0, s);
-    hipLaunchKernelGGL((walk_kernel<0, false>), dim3((2 * Smax + SEGW - 1) / SEGW, (2 * Smax + c.walk_rows - 1) / c.walk_rows, c.nbatch),
+    hipLaunchKernelGGL((walk_kernel<0, false>), dim3(var_strips, (2 * Smax + c.var_rows - 1) / c.var_rows, c.nbatch),
                        dim3(64), 0, s, d_frames, c, var_sums, tvbuf, cand, mark, row_count);
     QCS_HIP(hipGetLastError());
     hipLaunchKernelGGL(var_reduce_kernel, dim3(16, c.nbatch), dim3(256), 0, s, c, tvbuf, var_sums);
