@@ -27,6 +27,7 @@
 //   7. cut_kernel         detector classification (multi mode), raw R x R cut, header
 //   8. WLE                PSF width, nearest neighbour (sorted sweep over the list), type
 #include <string.h>
+#include <algorithm>
 #include <type_traits>
 #include "qcs_internal.h"
 
@@ -566,34 +567,52 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MODE ==
         walk_body<MODE, SMOOTH, false>(frames, c, var_sums, tvbuf, cand_mask, mark_mask, row_count, raw);
 }
 
-// integer sums of the variance samples of each batch from the region's background-removed values
+// integer sums of the variance samples of each batch from the region's background-removed values: a
+// work-group takes every VAR_BLOCKS-th row of samples (S <= 256: one a thread), four rows at the most,
+// whose loads are all in flight together (32 regions: 18 -> 11 us)
+constexpr int VAR_BLOCKS = 64;
 __global__ void __launch_bounds__(256) var_reduce_kernel(ExtractConst c, const uint16_t *__restrict__ tvbuf,
                                                          unsigned long long *__restrict__ sums)
 {
+    __shared__ unsigned long long sh[2][4];
     const int b = blockIdx.y;
     const int BH = batch_rows(c, b);
     const int S = var_side(c, BH);
     const uint16_t *t = tvbuf + (size_t)b * VAR_MAX * VAR_MAX;
+    const int i = threadIdx.x;
     unsigned long long s1 = 0, s2 = 0;
-    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < S * S; g += gridDim.x * blockDim.x) {
-        const int i = g % S, j = g / S;   // sample (X, Y) = (cx + i, cy + j), region origin (cx - S, cy - S)
-        int d1 = t[(size_t)(S + j) * VAR_MAX + S + i];
-        const int d2 = t[(size_t)(S + j) * VAR_MAX + i];
-        int d3 = t[(size_t)j * VAR_MAX + S + i];
-        const int d4 = t[(size_t)j * VAR_MAX + i];
-        d1 = d1 < d2 ? d1 : d2;
-        d3 = d3 < d4 ? d3 : d4;
-        d1 = d1 < d3 ? d1 : d3;
-        s1 += (unsigned long long)d1;
-        s2 += (unsigned long long)d1 * (unsigned long long)d1;
+    if (i < S) {
+        // sample (X, Y) = (cx + i, cy + j), region origin (cx - S, cy - S)
+        int v[256 / VAR_BLOCKS];
+#pragma unroll
+        for (int q = 0; q < 256 / VAR_BLOCKS; q++) {
+            const int j = blockIdx.x + q * VAR_BLOCKS;
+            v[q] = 0;
+            if (j < S) {
+                const int d1 = t[(size_t)(S + j) * VAR_MAX + S + i], d2 = t[(size_t)(S + j) * VAR_MAX + i];
+                const int d3 = t[(size_t)j * VAR_MAX + S + i], d4 = t[(size_t)j * VAR_MAX + i];
+                v[q] = min(min(d1, d2), min(d3, d4));
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 256 / VAR_BLOCKS; q++) {
+            s1 += (unsigned long long)v[q];
+            s2 += (unsigned long long)v[q] * (unsigned long long)v[q];
+        }
     }
     for (int off = 32; off > 0; off >>= 1) {
         s1 += __shfl_down(s1, off, 64);
         s2 += __shfl_down(s2, off, 64);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&sums[2 * b + 0], s1);
-        atomicAdd(&sums[2 * b + 1], s2);
+        sh[0][threadIdx.x >> 6] = s1;
+        sh[1][threadIdx.x >> 6] = s2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const unsigned long long *p = sh[threadIdx.x];
+        const unsigned long long s = (p[0] + p[1]) + (p[2] + p[3]);
+        if (s) atomicAdd(&sums[2 * b + threadIdx.x], s);
     }
 }
 
@@ -748,65 +767,77 @@ __global__ void __launch_bounds__(SCAN_BLOCK) scan_apply_kernel(const int *__res
 
 // ---- 4. per-batch bookkeeping ----------------------------------------------------------------
 // info layout: [0] kept total, [1] found total, then per batch b: found, kept, out offset
-__global__ void batch_kernel(ExtractConst c, const int *__restrict__ row_off, const int *__restrict__ tile_sums,
-                             int nrows, int ntiles, int *__restrict__ info)
+// One wave, a batch a lane: a batch's candidates are cut off at its own capacity, and all batches' at the
+// call's, which is the prefix sum of the former cut off.
+__global__ void __launch_bounds__(64) batch_kernel(ExtractConst c, const int *__restrict__ row_off, const int *__restrict__ tile_sums,
+                                                   int nrows, int ntiles, int *__restrict__ info)
 {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    const int total = tile_sums[ntiles];
-    int out = 0, found_all = 0;
-    for (int b = 0; b < c.nbatch; b++) {
-        const int r0 = b * c.B * c.H;
-        const int r1 = r0 + batch_rows(c, b);
-        const int o0 = row_off[r0];
-        const int o1 = (r1 < nrows) ? row_off[r1] : total;
-        const int found = o1 - o0;
-        int kept = found < c.batch_cap ? found : c.batch_cap;
-        const int room = c.cap - out;
-        kept = kept < room ? kept : (room > 0 ? room : 0);
-        info[2 + 3 * b + 0] = found;
-        info[2 + 3 * b + 1] = kept;
-        info[2 + 3 * b + 2] = out;
-        out += kept;
-        found_all += found;
+    const int lane = threadIdx.x, total = tile_sums[ntiles];
+    int out = 0;   // candidates of the chunks before, not cut off
+    for (int b0 = 0; b0 < c.nbatch; b0 += 64) {
+        const int b = b0 + lane;
+        int found = 0, want = 0;
+        if (b < c.nbatch) {
+            const int r0 = b * c.B * c.H, r1 = r0 + batch_rows(c, b);
+            found = (r1 < nrows ? row_off[r1] : total) - row_off[r0];
+            want = min(found, c.batch_cap);
+        }
+        const int incl = wave_inclusive_sum(want), before = out + incl - want;
+        if (b < c.nbatch) {
+            info[2 + 3 * b + 0] = found;
+            info[2 + 3 * b + 1] = max(min(want, c.cap - before), 0);
+            info[2 + 3 * b + 2] = min(before, c.cap);
+        }
+        out += __shfl(incl, 63, 64);
     }
-    info[0] = out;
-    info[1] = found_all;
+    if (lane == 0) {
+        info[0] = min(out, c.cap);
+        info[1] = total;
+    }
 }
 
 // ---- 5. candidate list in raster order -------------------------------------------------------
-// One wave per stacked row: lane s takes segment s's candidate mask (coalesced loads), and a
-// wave prefix sum of the masks' popcounts gives each segment its first slot, so the row's
-// candidates come out in raster order.
-constexpr int EMIT_WAVES = 4;   // rows per work-group
+// One wave per EMIT_U stacked rows, whose loads are in flight together: lane s takes segment s's
+// candidate mask (coalesced loads), and a wave prefix sum of the masks' popcounts gives each segment
+// its first slot, so a row's candidates come out in raster order (65,536 rows with some six candidates each: 19 -> 15 us).
+constexpr int EMIT_WAVES = 4, EMIT_U = 4;
 __global__ void __launch_bounds__(64 * EMIT_WAVES) emit_kernel(ExtractConst c, const unsigned long long *__restrict__ cand_mask,
-                                                               const int *__restrict__ row_off, const int *__restrict__ row_count,
-                                                               int nrows, const int *__restrict__ info, int3 *__restrict__ xyb)
+                                                               const int *__restrict__ row_off, int nrows,
+                                                               const int *__restrict__ info, int3 *__restrict__ xyb)
 {
-    const int row = blockIdx.x * EMIT_WAVES + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (row >= nrows || row_count[row] == 0) return;   // uniform over the wave
-    const int b = row / (c.B * c.H);
-    const int r0 = b * c.B * c.H;
-    const int kept = info[2 + 3 * b + 1], out0 = info[2 + 3 * b + 2];
-    int base = row_off[row] - row_off[r0];
-    const int y = row - r0;   // batch-relative row
-    for (int s0 = 0; s0 < c.nseg; s0 += 64) {
-        const int sgi = s0 + lane;
-        unsigned long long m = (sgi < c.nseg) ? cand_mask[(size_t)row * c.nseg + sgi] : 0ull;
-        const int cnt = __popcll(m);
-        int incl = cnt;
+    const int row0 = (blockIdx.x * EMIT_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * EMIT_U, lane = threadIdx.x & 63;
+    unsigned long long m0[EMIT_U];
+    int off[EMIT_U];
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += v;
+    for (int u = 0; u < EMIT_U; u++) {
+        const int row = row0 + u;
+        const bool in = row < nrows;
+        m0[u] = in && lane < c.nseg ? cand_mask[(size_t)row * c.nseg + lane] : 0ull;
+        off[u] = in ? row_off[row] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < EMIT_U; u++) {
+        const int row = row0 + u;
+        if (row >= nrows || (c.nseg <= 64 && __ballot(m0[u] != 0) == 0)) continue;   // uniform
+        const int b = row / (c.B * c.H);
+        const int r0 = b * c.B * c.H;
+        const int kept = info[2 + 3 * b + 1], out0 = info[2 + 3 * b + 2];
+        int base = off[u] - row_off[r0];
+        const int y = row - r0;   // batch-relative row
+        for (int s0 = 0; s0 < c.nseg; s0 += 64) {
+            const int sgi = s0 + lane;
+            unsigned long long m = s0 == 0 ? m0[u] : ((sgi < c.nseg) ? cand_mask[(size_t)row * c.nseg + sgi] : 0ull);
+            const int cnt = __popcll(m);
+            const int incl = wave_inclusive_sum(cnt);
+            int local = base + incl - cnt;
+            while (m) {
+                const int bit = __ffsll((long long)m) - 1;
+                m &= m - 1;
+                if (local < kept) xyb[out0 + local] = make_int3(sgi * SEGW + bit, y, b);
+                local++;
+            }
+            base += __shfl(incl, 63, 64);
         }
-        int local = base + incl - cnt;
-        while (m) {
-            const int bit = __ffsll((long long)m) - 1;
-            m &= m - 1;
-            if (local < kept) xyb[out0 + local] = make_int3(sgi * SEGW + bit, y, b);
-            local++;
-        }
-        base += __shfl(incl, 63, 64);
     }
 }
 
@@ -825,11 +856,35 @@ __device__ __forceinline__ int mark_count(const unsigned long long *mark, int ns
     return cnt;
 }
 
+// a mark in columns x - half .. x + half of one row's segment masks (two at the most: 2 half + 1 < SEGW),
+// x - 1 .. x + 1 left out with `centre`
+__device__ __forceinline__ bool other_marks(const unsigned long long *__restrict__ mark, int x, int half, bool centre)
+{
+    const int s0 = (x - half) / SEGW, s1 = (x + half) / SEGW;
+    unsigned long long m0 = mark[s0], m1 = mark[s1];   // the same word when one segment holds them all
+    // bits of the window in either segment, from its column 0
+    auto window = [](int lo, int hi) {
+        lo = max(lo, 0);
+        hi = min(hi, SEGW - 1);
+        return lo > hi ? 0ull : (~0ull << lo) & (~0ull >> (63 - hi));
+    };
+    const int c0 = x - s0 * SEGW, c1 = x - s1 * SEGW;
+    unsigned long long w0 = window(c0 - half, c0 + half), w1 = window(c1 - half, c1 + half);
+    if (centre) {
+        w0 &= ~window(c0 - 1, c0 + 1);
+        w1 &= ~window(c1 - 1, c1 + 1);
+    }
+    return ((m0 & w0) | (m1 & w1)) != 0;
+}
+
 // one wave per group of CUT_U consecutive ROI records (grid-stride over the kept count): lanes
 // write consecutive uint16 words of each record, so the stores are contiguous; the CUT_U records'
-// list entries and pixels are loaded before any is stored, so a wave keeps CUT_U independent
-// memory round trips in flight instead of one
-constexpr int CUT_U = 8;
+// pixels are loaded before any is stored, so a wave keeps CUT_U independent memory round trips in
+// flight instead of one.  The marks of all CUT_U windows are one round of loads too, eight lanes a
+// record, and a record's header is one lane's work.  32 frames of 2048 x 2048 with 0.003 molecules per
+// pixel, 7 x 7: 65 -> 60 us, most of it the 64-byte sectors of seven rows a record; CUT_BLOCKS
+// waves fill the chip, and a call of 180 records pays for no more (6.6 -> 4.4 us).
+constexpr int CUT_U = 8, CUT_BLOCKS = 4096;
 
 // R is the cut size; with sel set, record j is candidate sel[j] for j < *sel_n (a set of the
 // mixed-size extraction), else record i is candidate i for i < info[0]
@@ -845,52 +900,49 @@ __global__ void __launch_bounds__(64) cut_kernel(const uint16_t *__restrict__ fr
     const int n = sel ? *sel_n : info[0];
     const int half = R / 2, WR = R * (R + 1), RR = R * R;
     const int l = threadIdx.x;
+    const int start = c.start_dev ? *c.start_dev : c.start_frame;
+    const int BH = c.B * c.H;
     for (int i0 = blockIdx.x * CUT_U; i0 < n; i0 += gridDim.x * CUT_U) {
-        int3 e[CUT_U];
-        int ft[CUT_U];
+        // lane j holds record j's list entry and works out its header
+        int3 e = make_int3(half, half, 0);
+        if (l < CUT_U && i0 + l < n) e = xyb[sel ? sel[i0 + l] : i0 + l];
+        const int valid = min(CUT_U, n - i0);   // uniform
+        int x[CUT_U], y[CUT_U], z[CUT_U];       // uniform
 #pragma unroll
         for (int j = 0; j < CUT_U; j++) {
-            e[j] = (i0 + j < n) ? xyb[sel ? sel[i0 + j] : i0 + j] : make_int3(half, half, 0);
-            ft[j] = QCS_ROITYPE_SINGLE;
+            x[j] = __builtin_amdgcn_readlane(e.x, j);
+            y[j] = __builtin_amdgcn_readlane(e.y, j);
+            z[j] = __builtin_amdgcn_readlane(e.z, j);
         }
+        int ft = QCS_ROITYPE_SINGLE;
         if (c.multi) {
-#pragma unroll
-            for (int j = 0; j < CUT_U; j++) {
-                // lanes 0..R-1 count the marks of one window row each
-                const int x = e[j].x, y = e[j].y;
-                const size_t rbase = (size_t)e[j].z * c.B * c.H;
-                int all = 0, inner = 0;
-                if (l < R && i0 + j < n) {
-                    const size_t row = rbase + y - half + l;
-                    all = mark_count(mark_mask, c.nseg, row, x - half, x + half);
-                    if (l >= half - 1 && l <= half + 1) inner = mark_count(mark_mask, c.nseg, row, x - 1, x + 1);
-                }
-                int d = all - inner;
-                for (int off = 32; off > 0; off >>= 1) d += __shfl_xor(d, off, 64);
-                ft[j] = (d > 0) ? QCS_ROITYPE_MULTI : QCS_ROITYPE_SINGLE;
-            }
+            // eight lanes a record, a window row each: marks outside the centre's 3 x 3
+            const int q = l & 7, ex = __shfl(e.x, l >> 3, 64), ey = __shfl(e.y, l >> 3, 64), ez = __shfl(e.z, l >> 3, 64);
+            bool other = false;
+            for (int r = q; r < R && (l >> 3) < valid; r += 8)
+                other |= other_marks(mark_mask + ((size_t)ez * BH + ey - half + r) * c.nseg, ex, half, r >= half - 1 && r <= half + 1);
+            const unsigned long long m = __ballot(other);
+            if (l < CUT_U && ((m >> (8 * l)) & 0xff)) ft = QCS_ROITYPE_MULTI;
         }
-        for (int k = l; k < WR; k += 64) {
+        for (int k = l; k < RR; k += 64) {
             uint16_t v[CUT_U];
+            const int r = k / R;
+            const size_t off = (size_t)r * c.W + (k - r * R);
 #pragma unroll
-            for (int j = 0; j < CUT_U; j++) {
-                const int x = e[j].x, y = e[j].y, b = e[j].z;
-                if (k < RR) {
-                    const int r = k / R, cc = k - r * R;
-                    const uint16_t *img = frames + (size_t)b * c.B * c.H * c.W;
-                    v[j] = (i0 + j < n) ? img[(size_t)(y - half + r) * c.W + (x - half + cc)] : (uint16_t)0;
-                } else {
-                    const int h = k - RR;
-                    const int fr = (c.start_dev ? *c.start_dev : c.start_frame) + b * c.B + y / c.H;
-                    v[j] = h == 0 ? (uint16_t)x
-                         : h == 1 ? (uint16_t)(y % c.H)
-                         : h == 2 ? (uint16_t)(fr % 65536)
-                         : h == 3 ? (uint16_t)(fr / 65536)
-                         : h == 4 ? (uint16_t)ft[j] : (uint16_t)0;
-                }
-            }
+            for (int j = 0; j < CUT_U; j++)
+                v[j] = j < valid ? (frames + (((size_t)z[j] * BH + y[j] - half) * c.W + x[j] - half))[off] : (uint16_t)0;
 #pragma unroll
             for (int j = 0; j < CUT_U; j++) stage[j * WR + k] = v[j];
+        }
+        if (l < CUT_U) {
+            uint16_t *h = stage + l * WR + RR;
+            const int f = e.y / c.H, fr = start + e.z * c.B + f;
+            h[0] = (uint16_t)e.x;
+            h[1] = (uint16_t)(e.y - f * c.H);
+            h[2] = (uint16_t)(fr % 65536);
+            h[3] = (uint16_t)(fr / 65536);
+            h[4] = (uint16_t)ft;
+            for (int k = 5; k < R; k++) h[k] = 0;
         }
         __syncthreads();
         const int nv = min(CUT_U, n - i0);
@@ -1021,29 +1073,28 @@ static int extract_candidates(qcs_ctx *ctx, const qcs_params &p, const uint16_t 
     if ((size_t)rows_per_batch * c.W >= ((size_t)1 << 31)) return fail(QCS_ERR_ARG, "batched image larger than 2^31 pixels");
     const int ntiles = (int)((nrows + SCAN_TILE - 1) / SCAN_TILE);
     int rc;
-    if ((rc = ctx->ex_var.ensure(sizeof(unsigned long long) * 2 * c.nbatch)) ||
-        (rc = ctx->ex_det.ensure(sizeof(uint16_t) * VAR_MAX * VAR_MAX * (size_t)c.nbatch)) ||
+    const size_t nvs = 4 * (size_t)c.nbatch;   // ints of the variance sums, ahead of the row counts: one fill clears both
+    if ((rc = ctx->ex_det.ensure(sizeof(uint16_t) * VAR_MAX * VAR_MAX * (size_t)c.nbatch)) ||
         (rc = ctx->ex_mark.ensure(sizeof(unsigned long long) * nrows * c.nseg * 2)) ||
-        (rc = ctx->ex_cnt.ensure(sizeof(int) * (nrows * 2 + ntiles + 1))) ||
+        (rc = ctx->ex_cnt.ensure(sizeof(int) * (nvs + nrows * 2 + ntiles + 1))) ||
         (rc = ctx->ex_xy.ensure(sizeof(int3) * (size_t)(cap > 0 ? cap : 1))) ||
         (rc = ctx->ex_tmp.ensure(sizeof(int) * (2 + 3 * (size_t)c.nbatch))))
         return rc;
-    unsigned long long *var_sums = ctx->ex_var.as<unsigned long long>();
+    unsigned long long *var_sums = ctx->ex_cnt.as<unsigned long long>();
     uint16_t *tvbuf = ctx->ex_det.as<uint16_t>();
     unsigned long long *cand = ctx->ex_mark.as<unsigned long long>();
     unsigned long long *mark = cand + nrows * c.nseg;
-    int *row_count = ctx->ex_cnt.as<int>();
+    int *row_count = ctx->ex_cnt.as<int>() + nvs;
     int *row_off = row_count + nrows;
     int *tile_sums = row_off + nrows;
     int *info = ctx->ex_tmp.as<int>();
     int3 *xyb = ctx->ex_xy.as<int3>();
 
-    fill_async(reinterpret_cast<int *>(var_sums), 4 * (size_t)c.nbatch, 0, s);
-    fill_async(row_count, nrows, 0, s);
+    fill_async(ctx->ex_cnt.as<int>(), nvs + nrows, 0, s);
     hipLaunchKernelGGL((walk_kernel<0, false>), dim3(var_strips, (2 * Smax + c.var_rows - 1) / c.var_rows, c.nbatch),
                        dim3(64), 0, s, d_frames, c, var_sums, tvbuf, cand, mark, row_count);
     QCS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(var_reduce_kernel, dim3(16, c.nbatch), dim3(256), 0, s, c, tvbuf, var_sums);
+    hipLaunchKernelGGL(var_reduce_kernel, dim3(VAR_BLOCKS, c.nbatch), dim3(256), 0, s, c, tvbuf, var_sums);
     QCS_HIP(hipGetLastError());
     const dim3 wgrid(c.nseg, (rows_per_batch + c.walk_rows - 1) / c.walk_rows, c.nbatch);
     if (c.smooth)
@@ -1053,8 +1104,8 @@ static int extract_candidates(qcs_ctx *ctx, const qcs_params &p, const uint16_t 
     QCS_HIP(hipGetLastError());
     if ((rc = scan_exclusive(row_count, (int)nrows, row_off, tile_sums, s))) return rc;
     hipLaunchKernelGGL(batch_kernel, dim3(1), dim3(64), 0, s, c, row_off, tile_sums, (int)nrows, ntiles, info);
-    hipLaunchKernelGGL(emit_kernel, dim3((unsigned)((nrows + EMIT_WAVES - 1) / EMIT_WAVES)), dim3(64 * EMIT_WAVES), 0, s, c, cand,
-                       row_off, row_count, (int)nrows, info, xyb);
+    hipLaunchKernelGGL(emit_kernel, dim3((unsigned)((nrows + EMIT_WAVES * EMIT_U - 1) / (EMIT_WAVES * EMIT_U))), dim3(64 * EMIT_WAVES), 0,
+                       s, c, cand, row_off, (int)nrows, info, xyb);
     QCS_HIP(hipGetLastError());
     run.info = info;
     run.xyb = xyb;
@@ -1169,7 +1220,7 @@ int extract_mixed_launch(qcs_ctx *ctx, const uint16_t *d_frames, int nframes, in
     int *lists = offs + 3 * (size_t)ncap;
     int *tsum = lists + 3 * (size_t)ncap;
     if (cap > 0) {
-        const int cut_blocks = cap < 16384 ? cap : 16384;
+        const int cut_blocks = (int)std::min<long long>(((long long)cap + CUT_U - 1) / CUT_U, CUT_BLOCKS);
         hipLaunchKernelGGL(cut_kernel, dim3(cut_blocks), dim3(64), 0, s, d_frames, run.c, 7, run.mark, run.info, run.xyb, nullptr, nullptr,
                            r7);
         QCS_HIP(hipGetLastError());
@@ -1185,7 +1236,7 @@ int extract_mixed_launch(qcs_ctx *ctx, const uint16_t *d_frames, int nframes, in
         hipLaunchKernelGGL(mixed_count_kernel, dim3(1), dim3(1), 0, s, ts, ntiles, sets[k].n, sets[k].d_n);
         QCS_HIP(hipGetLastError());
         if (sets[k].n > 0) {
-            const int blocks = sets[k].n < 16384 ? sets[k].n : 16384;
+            const int blocks = (int)std::min<long long>(((long long)sets[k].n + CUT_U - 1) / CUT_U, CUT_BLOCKS);
             hipLaunchKernelGGL(cut_kernel, dim3(blocks), dim3(64), 0, s, d_frames, run.c, 7 + 2 * k, run.mark, run.info, run.xyb, l,
                                sets[k].d_n, sets[k].d_rois);
             QCS_HIP(hipGetLastError());
@@ -1218,7 +1269,7 @@ extern "C" int qcs_extract_dev(qcs_ctx *ctx, const uint16_t *d_frames, int nfram
     ExtractRun run;
     if ((rc = extract_candidates(ctx, p, d_frames, nframes, start_frame, nullptr, cap, s, run))) return rc;
     if (cap > 0) {
-        const int cut_blocks = cap < 16384 ? cap : 16384;
+        const int cut_blocks = (int)std::min<long long>(((long long)cap + CUT_U - 1) / CUT_U, CUT_BLOCKS);
         hipLaunchKernelGGL(cut_kernel, dim3(cut_blocks), dim3(64), 0, s, d_frames, run.c, run.c.R, run.mark, run.info, run.xyb, nullptr,
                            nullptr, d_rois);
         QCS_HIP(hipGetLastError());

@@ -127,7 +127,7 @@ struct qcs_ctx {
     qcs::Timer timer;
     qcs_fit_stats stats{};
     // extraction scratch
-    qcs::DevBuf ex_bkg, ex_tmp, ex_det, ex_mark, ex_cnt, ex_xy, ex_var, ex_frames;
+    qcs::DevBuf ex_bkg, ex_tmp, ex_det, ex_mark, ex_cnt, ex_xy, ex_frames;
     // fit scratch
     qcs::DevBuf fit_idx1, fit_idx2, fit_idx3, fit_flag, fit_cnt, fit_rows;   // fit_flag: the cascade's carve
     // converged fitting scratch

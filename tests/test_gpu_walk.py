@@ -43,3 +43,39 @@ def test_walk_exact(gpu, W, H, nf, B, loc, multi):
         assert np.array_equal(g_wle.view(np.uint32), wle.view(np.uint32))
         found += n
     assert found > 0 or W < 20
+
+
+@pytest.mark.parametrize("R,multi,B", [(5, 0, 1), (7, 1, 2), (11, 1, 1), (17, 1, 2), (17, 0, 1)])
+def test_list_exact(gpu, R, multi, B):
+    """Windows across strip borders for the marks; nearest neighbours from next door to past the entries that a
+    work-group keeps (a far spot in a wide frame that is crowded elsewhere), alone in a frame, and none."""
+    W, H, nf = 4000, 60, 4
+    rng = np.random.default_rng(R + multi)
+    img = 200.0 + rng.normal(0, 6, (nf, H, W))
+    yy, xx = np.mgrid[-4:5, -4:5]
+    spot = np.exp(-(xx**2 + yy**2) / (2 * 1.3**2))
+
+    def put(f, x, y, a):
+        img[f, y - 4:y + 5, x - 4:x + 5] += a * spot
+
+    for x in range(30, 2600, 11):
+        for y in range(16, 46, 11):
+            put(0, x + int(rng.integers(-1, 2)), y + int(rng.integers(-1, 2)), rng.uniform(2500, 5000))
+    put(0, 3900, 30, 4000.0)
+    put(2, 2000, 30, 4000.0)
+    for x in range(50, 3900, 28):
+        put(3, x, int(rng.integers(18, 42)), 3500.0)
+        put(3, x + int(rng.integers(4, 8)), int(rng.integers(18, 42)), 2500.0)
+    fr = np.clip(np.rint(img), 0, 65535).astype(np.uint16)
+    p = Q.default_params(QE=1.0, ImageWidth=W, ImageHigh=H, BatchedImageNum=B, MultiEmitterFitEn=multi, ROISize=R)
+    rois, wle, n, _ = O.extract(p, fr, start_frame=70000, cap=5000)
+    ctx = Q.Context(p)
+    for cap in (5000, 300):
+        g_rois, g_wle, g_n = ctx.extract(fr, start_frame=70000, cap=cap)
+        if cap == 5000:
+            assert g_n == n and n > 700
+            assert np.array_equal(g_rois, rois)
+            assert np.array_equal(g_wle.view(np.uint32), wle.view(np.uint32))
+        else:
+            r2, w2, n2, _ = O.extract(p, fr, start_frame=70000, cap=cap)
+            assert g_n == n2 and np.array_equal(g_rois, r2) and np.array_equal(g_wle.view(np.uint32), w2.view(np.uint32))
