@@ -41,45 +41,78 @@ __device__ __forceinline__ float div_dh(float x)
     return __builtin_fmaf(__builtin_fmaf(-y, 0.02f, x), 50.0f, y);
 }
 
-// Diagonal Fisher sums of x and y.  NARROW (every model value in [1, 1e20], the argument of each
-// exponential <= 0): qexpf_nonpos, qlogf_normal and div_dh<true> give the same bits as the
-// general forms there.
+// One grid point's terms of the diagonal Fisher sums of x and y.  NARROW (every model value in
+// [1, 1e20], the argument of each exponential <= 0): qexpf_nonpos, qlogf_normal and div_dh<true>
+// give the same bits as the general forms there.
 template <int G, bool NARROW>
-__device__ __forceinline__ void crlb_fisher(float peak, float ix, float iy, float be, float &fx, float &fy)
+__device__ __forceinline__ void crlb_term(int r, int c, float peak, float ix, float iy, float be, float &tx, float &ty)
 {
     const float dh = 0.02f;
     const float xp = 0.0f + dh, xn = (0.0f + dh) - 2.0f * dh;
     auto lg = [](float m) { return NARROW ? qlogf_normal(m) : qlogf(m); };
+    const float m0 = crlb_psf<G, NARROW>(r, c, peak, ix, iy, 0.0f, 0.0f, be);
+    const float l0 = lg(m0);
+    {
+        const float mp = crlb_psf<G, NARROW>(r, c, peak, ix, iy, xp, 0.0f, be);
+        const float mn = crlb_psf<G, NARROW>(r, c, peak, ix, iy, xn, 0.0f, be);
+        const float d2 = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, m0, mp) + mn));
+        const float d2l = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, l0, lg(mp)) + lg(mn)));
+        tx = __builtin_fmaf(-m0, d2l, d2);
+    }
+    {
+        const float mp = crlb_psf<G, NARROW>(r, c, peak, ix, iy, 0.0f, xp, be);
+        const float mn = crlb_psf<G, NARROW>(r, c, peak, ix, iy, 0.0f, xn, be);
+        const float d2 = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, m0, mp) + mn));
+        const float d2l = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, l0, lg(mp)) + lg(mn)));
+        ty = __builtin_fmaf(-m0, d2l, d2);
+    }
+}
+
+// sum += v of lane K of the 16, K = 0 .. 15 in turn (row_newbcast)
+template <int K>
+__device__ __forceinline__ void crlb_add16(float v, float &sum)
+{
+    sum = sum + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xf, 0xf, true));
+    if constexpr (K < 15) crlb_add16<K + 1>(v, sum);
+}
+
+// The sums over the G x G grid in raster order.  L = 1: a lane takes every point.  L = 16: lane l of the 16
+// takes points 16 t + l, and all add the 16 terms of a round in the same order (points past the grid
+// add 0 to a sum that is never -0).
+template <int G, int L, bool NARROW>
+__device__ __forceinline__ void crlb_fisher(float peak, float ix, float iy, float be, float &fx, float &fy)
+{
     fx = 0.0f;
     fy = 0.0f;
-    for (int r = 0; r < G; r++) {
+    float tx, ty;
+    if constexpr (L == 1) {
+        for (int r = 0; r < G; r++) {
 #pragma unroll
-        for (int c = 0; c < G; c++) {
-            const float m0 = crlb_psf<G, NARROW>(r, c, peak, ix, iy, 0.0f, 0.0f, be);
-            const float l0 = lg(m0);
-            {
-                const float mp = crlb_psf<G, NARROW>(r, c, peak, ix, iy, xp, 0.0f, be);
-                const float mn = crlb_psf<G, NARROW>(r, c, peak, ix, iy, xn, 0.0f, be);
-                const float d2 = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, m0, mp) + mn));
-                const float d2l = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, l0, lg(mp)) + lg(mn)));
-                fx = fx + __builtin_fmaf(-m0, d2l, d2);
+            for (int c = 0; c < G; c++) {
+                crlb_term<G, NARROW>(r, c, peak, ix, iy, be, tx, ty);
+                fx = fx + tx;
+                fy = fy + ty;
             }
-            {
-                const float mp = crlb_psf<G, NARROW>(r, c, peak, ix, iy, 0.0f, xp, be);
-                const float mn = crlb_psf<G, NARROW>(r, c, peak, ix, iy, 0.0f, xn, be);
-                const float d2 = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, m0, mp) + mn));
-                const float d2l = div_dh<NARROW>(div_dh<NARROW>(__builtin_fmaf(-2.0f, l0, lg(mp)) + lg(mn)));
-                fy = fy + __builtin_fmaf(-m0, d2l, d2);
-            }
+        }
+    } else {
+        static_assert(L == 16, "a DPP row");
+        for (int p = threadIdx.x & 15; (p & ~15) < G * G; p += 16) {
+            const int q = min(p, G * G - 1), r = q / G;
+            crlb_term<G, NARROW>(r, q - r * G, peak, ix, iy, be, tx, ty);
+            crlb_add16<0>(p < G * G ? tx : 0.0f, fx);
+            crlb_add16<0>(p < G * G ? ty : 0.0f, fy);
         }
     }
 }
 
-template <int G>
+// What bounds a small call is the chain of G^2 points of some 200 instructions, the same for one row as
+// for a lane's worth of rows on every SIMD; with 16 lanes a row it is a sixteenth, and the ordered
+// sums are 15% more instructions (crlb_launch has both sides).
+template <int G, int L>
 __global__ void __launch_bounds__(64) crlb_kernel(float *__restrict__ loc, int n, const int *__restrict__ n_dev, float QE,
                                                   float RN, float PS)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = blockIdx.x * (64 / L) + (int)threadIdx.x / L;
     if (n_dev) n = *n_dev;
     if (i >= n) return;
     float *row = loc + (size_t)i * QCS_REC_FLOATS;
@@ -94,13 +127,14 @@ __global__ void __launch_bounds__(64) crlb_kernel(float *__restrict__ loc, int n
         const float iy = 1.0f / ((2.0f * sy) * sy);
         float fx, fy;
         // model values lie in [be, peak + be] with be > 1
-        if (peak + be < 1e20f) crlb_fisher<G, true>(peak, ix, iy, be, fx, fy);
-        else crlb_fisher<G, false>(peak, ix, iy, be, fx, fy);
+        if (peak + be < 1e20f) crlb_fisher<G, L, true>(peak, ix, iy, be, fx, fy);
+        else crlb_fisher<G, L, false>(peak, ix, iy, be, fx, fy);
         fx = (fx == 0.0f) ? 1.0f : fx;
         fy = (fy == 0.0f) ? 1.0f : fy;
         stdx = sqrtf(1.0f / fx) * PS;
         stdy = sqrtf(1.0f / fy) * PS;
     }
+    if (threadIdx.x % L != 0) return;
     row[9] = stdx;
     row[10] = stdy;
 }
@@ -165,11 +199,16 @@ int fit_launch_me(const qcs_params &p, int model, const uint16_t *d_rois, const 
 int crlb_launch(const qcs_params &p, float *d_loc, int n, const int *d_n, hipStream_t s)
 {
     if (n <= 0) return QCS_OK;
-    const dim3 grid((n + 63) / 64);
-    if (p.LocType == QCS_LOCTYPE_AS3D)
-        hipLaunchKernelGGL(crlb_kernel<15>, grid, dim3(64), 0, s, d_loc, n, d_n, p.QE, p.ReadNoise_e, p.PixelSize);
-    else
-        hipLaunchKernelGGL(crlb_kernel<9>, grid, dim3(64), 0, s, d_loc, n, d_n, p.QE, p.ReadNoise_e, p.PixelSize);
+    const bool el = p.LocType == QCS_LOCTYPE_AS3D;
+    // us per call, 16 lanes / one lane: 9 x 9 11 / 55 at 4,000 rows, 17 / 56 at 20,480, 39 / 55 at 64,000,
+    // 58 / 58 at 100,000, 91 / 59 at 160,000; 15 x 15 24 / 145, 37 / 145, 87 / 140, 127 / 150, 196 / 151
+    const bool split = n <= (el ? 110000 : 90000);
+    const dim3 grid(split ? (n + 3) / 4 : (n + 63) / 64), block(64);
+    const float q = p.QE, rn = p.ReadNoise_e, ps = p.PixelSize;
+    if (el && split) hipLaunchKernelGGL((crlb_kernel<15, 16>), grid, block, 0, s, d_loc, n, d_n, q, rn, ps);
+    else if (el) hipLaunchKernelGGL((crlb_kernel<15, 1>), grid, block, 0, s, d_loc, n, d_n, q, rn, ps);
+    else if (split) hipLaunchKernelGGL((crlb_kernel<9, 16>), grid, block, 0, s, d_loc, n, d_n, q, rn, ps);
+    else hipLaunchKernelGGL((crlb_kernel<9, 1>), grid, block, 0, s, d_loc, n, d_n, q, rn, ps);
     QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
