@@ -9,12 +9,12 @@
 //
 // Sorted compaction: the reference launches one kernel per frame and appends with an atomic
 // counter (within-frame order arbitrary, O(frames x rows) work).  Here the kept rows are stably
-// radix-sorted by frame (sort.hip), so rows of one frame keep their original order.  Rendering splats each localization's 7 x 7 Gaussian with float atomics, as the
-// reference does, but into LDS: localizations are binned by 64 x 64 tile of the SR image (a
-// footprint that straddles a tile edge is listed in each tile it touches), one work-group
-// accumulates a tile with LDS atomics and then adds it to the image with one coalesced
-// read-modify-write.  Scattered atomics into a 1.7 GB image would miss the caches on nearly
-// every update.  The PSF uses the deterministic exponential.
+// radix-sorted by frame (sort.hip), so rows of one frame keep their original order.
+// Rendering splats each localization's 7 x 7 Gaussian with float atomics, as the reference does, but
+// into LDS: localizations are binned by 64 x 64 tile of the SR image (a footprint that straddles a tile
+// edge is listed in each tile it touches), one work-group accumulates a tile with LDS atomics and then
+// adds it to the image with one coalesced read-modify-write.  Scattered atomics into a 1.7 GB image
+// would miss the caches on nearly every update.  The PSF uses the deterministic exponential.
 #include <string.h>
 #include "qcs_internal.h"
 #include "qcs_devmath.h"
