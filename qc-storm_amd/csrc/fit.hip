@@ -282,7 +282,7 @@ size_t cascade_scratch_bytes(int n)
 {
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t ni = (size_t)(n > 0 ? n : 1);
-    return up(64) + 3 * up(sizeof(int) * ni) + up(sizeof(int) * (7 * ni + scan_tile_count(ni) + 1)) +
+    return up(64) + 3 * up(sizeof(int) * ni) + up(sizeof(int) * (6 * ni + scan_tile_count(ni) + 1)) +
            up(sizeof(float) * QCS_REC_FLOATS * 2 * ni);
 }
 
@@ -300,7 +300,7 @@ void cascade_carve(void *base, int n, CascadeBufs &b)
     b.list3 = reinterpret_cast<int *>(p);
     p += up(sizeof(int) * ni);
     b.flag = reinterpret_cast<int *>(p);
-    p += up(sizeof(int) * (7 * ni + scan_tile_count(ni) + 1));
+    p += up(sizeof(int) * (6 * ni + scan_tile_count(ni) + 1));
     b.rows = reinterpret_cast<float *>(p);
 }
 
@@ -310,7 +310,7 @@ int fit_cascade_launch(const qcs_params &p, Timer *tm, const uint16_t *d_rois, c
     const bool as3d = (p.LocType == QCS_LOCTYPE_AS3D);
     int rc;
     int *list1 = b.list1, *list2 = b.list2, *list3 = b.list3;
-    int *f1 = b.flag, *rr = f1 + 2 * n, *fs2 = rr + n, *ff2 = fs2 + n, *fs3 = ff2 + n;
+    int *f1 = b.flag, *rr = f1 + n, *fs2 = rr + n, *ff2 = fs2 + n, *fs3 = ff2 + n;
     int *offs = fs3 + n, *tsum = offs + n;
     int *ff3 = f1;   // f1 is free again once the 1E list is built
     float *sec2 = b.rows, *sec3 = sec2 + (size_t)QCS_REC_FLOATS * n;

@@ -14,7 +14,7 @@
 #include "qcs_internal.h"
 
 namespace {
-// cascade scratch at QCS_NOALLOC_MAX_ROIS ROIs is 13,926,912 bytes (cascade_scratch_bytes)
+// cascade scratch at QCS_NOALLOC_MAX_ROIS ROIs is 13,517,312 bytes (cascade_scratch_bytes)
 constexpr size_t SCRATCH_BYTES = (size_t)14 << 20;
 constexpr int MAX_DEVICES = 64;
 }  // namespace
