@@ -283,15 +283,16 @@ __global__ void __launch_bounds__(64 * SEL_WAVES) cf_select12_kernel(const int *
     }
 }
 
-// stage 2: K = 3 where it beats K = 2, final count into sel[roi], the unused rows of
+// stage 2: K = 3 where it beats K = 2 and the ROI was on list3 (its cap kcap, where given, is 3: only
+// then do t3 and l3 hold a fit of this call), final count into sel[roi], the unused rows of
 // 3 roi .. 3 roi + 2 zeroed, and the ROI appended to the list of its count (klist + (K - 1) cap,
 // counts in kcnt[0..2]): the rows kernels below each evaluate one model, so no wave runs the
 // Fisher matrices of several emitter counts one after the other with lanes masked.
 template <int E, int R>
 __global__ void __launch_bounds__(64 * SEL_WAVES) cf_kpart_kernel(const int *__restrict__ idx, int n, const int *__restrict__ n_dev,
                                                       const float *__restrict__ t3, const double *__restrict__ l2,
-                                                      const double *__restrict__ l3, CSelConst c, int *__restrict__ sel,
-                                                      float *__restrict__ rows, int *__restrict__ kcnt, int *__restrict__ klist,
+                                                      const double *__restrict__ l3, const int *__restrict__ kcap, CSelConst c,
+                                                      int *__restrict__ sel, float *__restrict__ rows, int *__restrict__ kcnt, int *__restrict__ klist,
                                                       int cap)
 {
     __shared__ BlockAppend<SEL_WAVES, 3> ba;
@@ -302,7 +303,7 @@ __global__ void __launch_bounds__(64 * SEL_WAVES) cf_kpart_kernel(const int *__r
     if (j < n) {
         roi = idx ? idx[j] : j;
         K = sel[roi];
-        if (K == 2 && c.kmax >= 3 && t3 && cf_valid<3 + E, R>(t3 + (size_t)roi * CM<3 + E>::P, c.n_min) &&
+        if (K == 2 && c.kmax >= 3 && t3 && (!kcap || kcap[roi] >= 3) && cf_valid<3 + E, R>(t3 + (size_t)roi * CM<3 + E>::P, c.n_min) &&
             l3[roi] - l2[roi] > (double)c.llr_half)
             K = 3;
         sel[roi] = K;
@@ -353,11 +354,12 @@ int select12_launch(const qcs_params &p, int kmax, const int *idx, int n, const 
     return QCS_OK;
 }
 
-// final counts and rows of the n listed ROIs (all n when idx is null; *d_n caps n when given);
+// final counts and rows of the n listed ROIs (all n when idx is null; *d_n caps n when given); kcap as in
+// select12_launch;
 // kcnt: 3 device ints, klist: 3 n ints of scratch
 int rows_launch(const qcs_params &p, int kmax, const uint16_t *rois, const int *idx, int n, const int *d_n, const float *t1,
-                const float *t2, const float *t3, const double *l2, const double *l3, int *sel, float *rows, int *kcnt,
-                int *klist, hipStream_t s)
+                const float *t2, const float *t3, const double *l2, const double *l3, const int *kcap, int *sel, float *rows,
+                int *kcnt, int *klist, hipStream_t s)
 {
     if (n <= 0) return QCS_OK;
     const CSelConst c = csel_const(p, kmax);
@@ -367,7 +369,7 @@ int rows_launch(const qcs_params &p, int kmax, const uint16_t *rois, const int *
     const float *tk[3] = {t1, t2, t3};
     if (p.LocType == QCS_LOCTYPE_AS3D) {
         CF_DISPATCH_R(p.ROISize, hipLaunchKernelGGL((cf_kpart_kernel<CF_ELLIPTIC, RT>), sgrid, sblock, 0, s, idx, n, d_n,
-                                                     kmax >= 3 ? t3 : nullptr, l2, l3, c, sel, rows, kcnt, klist, n))
+                                                     kmax >= 3 ? t3 : nullptr, l2, l3, kcap, c, sel, rows, kcnt, klist, n))
         QCS_HIP(hipGetLastError());
         CF_DISPATCH_R(p.ROISize, {
             hipLaunchKernelGGL((cf_rows_kernel<1 + CF_ELLIPTIC, RT>), grid, block, 0, s, rois, klist, kcnt, n, tk[0], c, rows);
@@ -380,7 +382,7 @@ int rows_launch(const qcs_params &p, int kmax, const uint16_t *rois, const int *
         })
     } else {
         CF_DISPATCH_R(p.ROISize, hipLaunchKernelGGL((cf_kpart_kernel<0, RT>), sgrid, sblock, 0, s, idx, n, d_n,
-                                                     kmax >= 3 ? t3 : nullptr, l2, l3, c, sel, rows, kcnt, klist, n))
+                                                     kmax >= 3 ? t3 : nullptr, l2, l3, kcap, c, sel, rows, kcnt, klist, n))
         QCS_HIP(hipGetLastError());
         CF_DISPATCH_R(p.ROISize, {
             hipLaunchKernelGGL((cf_rows_kernel<1, RT>), grid, block, 0, s, rois, klist, kcnt, n, tk[0], c, rows);
@@ -411,7 +413,7 @@ int plain_path(qcs_ctx *ctx, int kmax, const uint16_t *rois, const int *idx, int
     fill_async(cnt3, 1, 0, s);
     if ((rc = select12_launch(ctx->p, kmax, idx, n, d_n, t1, t2, l1, l2, nullptr, sel, cnt3, list3, s))) return rc;
     if (kmax >= 3 && (rc = cfit_launch(ctx, 3, rois, list3, n, cnt3, CF_INIT_ADD, t2, n2, t3, n3, info3, l3, s))) return rc;
-    return rows_launch(ctx->p, kmax, rois, idx, n, d_n, t1, t2, t3, l2, l3, sel, rows, kcnt, klist, s);
+    return rows_launch(ctx->p, kmax, rois, idx, n, d_n, t1, t2, t3, l2, l3, nullptr, sel, rows, kcnt, klist, s);
 }
 
 // ---- learned warm start -----------------------------------------------------------------------
@@ -716,7 +718,8 @@ int warm_launch(qcs_ctx *ctx, qcs_net *net, const uint16_t *d_rois, int n, float
     // selection as on the plain path
     if ((rc = select12_launch(p, 3, nullptr, n, nullptr, m.t1, m.t2, m.l1, m.l2, m.cs, sel, cnt + WC_L3, m.list3, s))) return rc;
     if ((rc = cfit_launch(ctx, 3, d_rois, m.list3, n, cnt + WC_L3, CF_INIT_ADD, m.t2, 8, m.t3, 11, m.info3, m.l3, s))) return rc;
-    if ((rc = rows_launch(p, 3, d_rois, nullptr, n, nullptr, m.t1, m.t2, m.t3, m.l2, m.l3, sel, d_loc, m.kcnt, m.klist, s)))
+    if ((rc = rows_launch(p, 3, d_rois, nullptr, n, nullptr, m.t1, m.t2, m.t3, m.l2, m.l3, m.cs, sel, d_loc, m.kcnt, m.klist,
+                          s)))
         return rc;
     if ((rc = timer_end(ctx->timer, TM_CFIT, s, ev, n))) return rc;
     if (h_stats) return stats_copy(ctx, m, n, sel, h_stats, s);
@@ -827,7 +830,7 @@ extern "C" int qcs_fit_mle_mixed_dev(qcs_ctx *ctx, const qcs_roi_set *sets, int 
         const size_t o = off[i];
         int *sel = sets[i].d_sel ? sets[i].d_sel : m.sel + o;
         if ((rc = rows_launch(p, kmax, sets[i].d_rois, nullptr, sets[i].n, sets[i].d_n, m.t1 + o * n1, m.t2 + o * n2,
-                              m.t3 + o * n3, m.l2 + o, m.l3 + o, sel, sets[i].d_loc, m.kcnt + 4 * i,
+                              m.t3 + o * n3, m.l2 + o, m.l3 + o, nullptr, sel, sets[i].d_loc, m.kcnt + 4 * i,
                               m.klist + 3 * o, s)))
             return rc;
     }

@@ -146,6 +146,34 @@ def test_warm_path_queue_matches_one_pass(gpu):
     assert res[1][2]["fallbacks"] == res[0][2]["fallbacks"]
 
 
+@pytest.mark.parametrize("queue", [0, 1])
+def test_warm_path_reads_no_fit_of_an_earlier_call(gpu, queue):
+    """ROIs that the network caps at two emitters have no three-emitter fit: what an earlier plain call on
+    the same context left in its place (here valid fits of bright three-emitter ROIs) must not count."""
+    n = 3000
+    rois, _ = _sim(7, n, 6200)
+    d_rois = torch.from_numpy(rois.view(np.int16)).cuda()
+    sp = Q.default_sim(width=7, height=7, n_per_unit_max=3, min_sep=2.0, max_sep=4.0, photons_min=4000.0, photons_max=9000.0)
+    d_other = torch.from_numpy(Q.sim_rois_host(sp, 6201, n)[0].view(np.int16)).cuda()
+    net = Q.Net(seed=5)   # untrained: predicts two emitters for nearly every ROI
+    ctx = Q.Context(Q.default_params(QE=1.0, ROISize=7, PixelSize=100.0))
+    ctx.set_tuning(queue=queue, warm_pmin=0.0)   # every prediction caps its ROI
+    loc = torch.zeros((3 * n, 12), dtype=torch.float32, device="cuda")
+    sel = torch.zeros(n, dtype=torch.int32, device="cuda")
+    res = []
+    for plain in (d_other, d_other.flip(0).contiguous()):   # the scratch has its size after the first of them
+        ctx.fit_plain_stats_dev(plain, n, 3, loc, sel)
+        st = ctx.fit_warm_dev(net, d_rois, n, loc, sel)
+        torch.cuda.synchronize()
+        print("queue", queue, "stats", st)
+        assert st["capped"] == n and st["pred_k3"] == 0 and st["pred_k2"] > n // 2
+        assert st["final_k3"] == 0
+        res.append((loc.cpu().numpy(), sel.cpu().numpy()))
+    np.testing.assert_array_equal(res[1][1], res[0][1])
+    np.testing.assert_array_equal(res[1][0].view(np.uint32), res[0][0].view(np.uint32))
+    assert res[0][1].max() == 2 and not res[0][0].reshape(n, 3, 12)[:, 2].any()
+
+
 def test_tuning_rejects_bad_queue_settings(gpu):
     ctx = Q.Context(Q.default_params(QE=1.0, ROISize=7))
     with pytest.raises(RuntimeError):
