@@ -165,7 +165,8 @@ __device__ __forceinline__ float lane_next(float v) { return __int_as_float(lane
 
 // acc[k] += x[k] of lane l - 1 (PREV) or l + 1, times w, for four rows: the shift is part of the
 // instruction (the compiler makes it a move of its own before a multiply-add).  A DPP operand needs two
-// wait states after the instruction that wrote it, once for the four.
+// wait states after the instruction that wrote it, once for the four.  acc[0] is written before x[1] is
+// read, so no sum may share a register with an input of the same value ("+&v").
 template <bool PREV>
 __device__ __forceinline__ void fma_shifted(float (&acc)[4], const float (&x)[4], float w)
 {
@@ -175,14 +176,14 @@ __device__ __forceinline__ void fma_shifted(float (&acc)[4], const float (&x)[4]
             "v_fmac_f32_dpp %1, %5, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
             "v_fmac_f32_dpp %2, %6, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
             "v_fmac_f32_dpp %3, %7, %8 wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
-            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w));
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w));
     else
         asm("s_nop 1\n\t"
             "v_fmac_f32_dpp %0, %4, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
             "v_fmac_f32_dpp %1, %5, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
             "v_fmac_f32_dpp %2, %6, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
             "v_fmac_f32_dpp %3, %7, %8 wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:1"
-            : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w));
+            : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]) : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w));
 }
 
 // two 16-bit lanes of a 32-bit register
