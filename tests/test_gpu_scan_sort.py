@@ -79,3 +79,13 @@ def test_stats_far_apart_frames(gpu):
     loc = _stat_rows(700, 9, 5, 100, 64, True)
     loc[:, 11] = np.sort(np.random.default_rng(1).choice([-70000.0, -3.0, 0.0, 1.0, 123456.0], 700)).astype(np.float32)
     _check(p, loc)
+
+
+# the neighbour pass takes 32,768 molecules a round: less than one, a little more than one, several
+@pytest.mark.parametrize("n,lt", [(32000, 0), (34500, 0), (34500, 1), (120011, 0)])
+def test_stats_rounds_of_the_neighbour_pass(gpu, n, lt):
+    p = Q.default_params(ImageWidth=4000, ImageHigh=3000, LocType=lt)
+    loc = _stat_rows(n, n + lt, 3, 4000, 3000, True)   # three frames: none is left out
+    loc[:, 1:3] = np.clip(loc[:, 1:3], 5.5, [3994.0, 2994.0])
+    got = _check(p, loc)
+    assert got["density_total"] == n and got["density_n1"] > 0
