@@ -17,7 +17,7 @@
 //
 // A pass reads its items from a source and writes them to a destination.  The row sort's first pass
 // reads the rows themselves, where rows that are not kept count nowhere, and its last pass writes
-// rows: up to 256 frames are one pass of three launches with no flags, no list and no key arrays,
+// rows (in calls of up to SORT_COPY_ROWS): up to 256 frames are one pass of three launches with no flags, no list and no key arrays,
 // and the number of kept rows stays on the device until the end.
 #include <limits.h>
 #include "qcs_internal.h"
@@ -129,6 +129,7 @@ __global__ void __launch_bounds__(SB) radix_scatter_kernel(Src src, Dst dst, int
         const int i = t0 + k * SB + tid;
         K key = 0;
         const bool valid = src.key(i, n, key);
+        const int val = valid ? src.val(i) : 0;   // in flight while the ranks are worked out
         const int d = (int)((key >> shift) & (K)(RADIX - 1));
         unsigned long long m = __ballot(valid);
 #pragma unroll
@@ -142,7 +143,7 @@ __global__ void __launch_bounds__(SB) radix_scatter_kernel(Src src, Dst dst, int
         if (valid) {
             int pos = base[d] + rank;
             for (int w = 0; w < wv; w++) pos += wcnt[w][d];
-            dst.put(pos, key, src.val(i));
+            dst.put(pos, key, val);
         }
         __syncthreads();
         int add = 0;
@@ -150,6 +151,15 @@ __global__ void __launch_bounds__(SB) radix_scatter_kernel(Src src, Dst dst, int
         for (int w = 0; w < SB / 64; w++) add += wcnt[w][tid];
         base[tid] += add;
     }
+}
+
+// rows idx[0 .. *m_dev) of loc, 16 bytes a lane
+__global__ void __launch_bounds__(SB) copy_rows_kernel(const float4 *__restrict__ loc, const int *__restrict__ idx, int n,
+                                                       const int *__restrict__ m_dev, float4 *__restrict__ out)
+{
+    const size_t t = (size_t)blockIdx.x * SB + threadIdx.x, j = t / 3;
+    if (j >= (size_t)min(*m_dev, n)) return;
+    out[t] = loc[(size_t)idx[j] * 3 + (t - j * 3)];
 }
 
 // inclusive max-scan: per-tile scan, scan of the tile maxima, then the carry-in
@@ -270,6 +280,14 @@ size_t sort_rows_tmp_ints(int n, int first, int end)
     return radix_sort_tmp_ints(n) + (((unsigned)end - (unsigned)first) > 255u ? (size_t)n * 4 : 0);
 }
 
+// Of several passes the last writes the rows itself up to SORT_COPY_ROWS; beyond, where the rows are far from
+// the caches, it leaves the order and a launch of its own copies the rows, all in flight at once (us per call,
+// rows in the last pass / copied; frames in order and shuffled, 5,000 frames: 1,000,000 rows 82 / 91 and
+// 111 / 112; 2,200,000 145 / 134 and 255 / 191; 8,000,000 521 / 427 and 881 / 651).  A single pass reads
+// its rows in order and writes them: 96 / 98 and 99 / 125 at 2,200,000 rows of 10 frames, 394 / 341 and
+// 415 / 452 at 8,000,000.
+constexpr int SORT_COPY_ROWS = 1500000;
+
 int sort_rows_by_frame(const float *d_loc, int n, int first, int end, float *d_out, int *d_m, int *tmp, hipStream_t s)
 {
     const unsigned span = ((unsigned)end - (unsigned)first);
@@ -282,11 +300,16 @@ int sort_rows_by_frame(const float *d_loc, int n, int first, int end, float *d_o
     if ((rc = radix_pass<unsigned>(rows, PairDst<unsigned>{k0, v0}, n, 0, tmp, d_m, s))) return rc;
     for (int shift = 8; shift < 32 && (span >> shift) != 0; shift += 8) {
         const PairSrc<unsigned> src{k0, v0, n, d_m};
-        if (shift + 8 >= 32 || (span >> (shift + 8)) == 0) return radix_pass<unsigned>(src, out, n, shift, tmp, nullptr, s);
+        const bool last = shift + 8 >= 32 || (span >> (shift + 8)) == 0;
+        if (last && n <= SORT_COPY_ROWS) return radix_pass<unsigned>(src, out, n, shift, tmp, nullptr, s);
         if ((rc = radix_pass<unsigned>(src, PairDst<unsigned>{k1, v1}, n, shift, tmp, nullptr, s))) return rc;
         unsigned *tk = k0; k0 = k1; k1 = tk;
         int *tv = v0; v0 = v1; v1 = tv;
     }
+    static_assert(QCS_REC_FLOATS == 12, "a row is three 16-byte words");
+    hipLaunchKernelGGL(copy_rows_kernel, dim3((unsigned)(((size_t)n * 3 + SB - 1) / SB)), dim3(SB), 0, s,
+                       reinterpret_cast<const float4 *>(d_loc), v0, n, d_m, reinterpret_cast<float4 *>(d_out));
+    QCS_HIP(hipGetLastError());
     return QCS_OK;
 }
 

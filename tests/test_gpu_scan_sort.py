@@ -89,3 +89,22 @@ def test_stats_rounds_of_the_neighbour_pass(gpu, n, lt):
     loc[:, 1:3] = np.clip(loc[:, 1:3], 5.5, [3994.0, 2994.0])
     got = _check(p, loc)
     assert got["density_total"] == n and got["density_n1"] > 0
+
+
+# past 1,500,000 rows of more than 256 frames the last pass leaves the order and the rows are copied by it
+@pytest.mark.parametrize("n", [1500000, 1500001])
+@pytest.mark.parametrize("nf", [256, 257, 70000])
+def test_rows_of_large_calls(gpu, n, nf):
+    g = torch.Generator(device="cuda").manual_seed(nf)
+    d = torch.rand((n, 12), generator=g, device="cuda")
+    d[:, 0] = torch.randint(0, 5, (n,), generator=g, device="cuda").float()
+    fr = torch.randint(0, nf + 2, (n,), generator=g, device="cuda")   # one before the first and one past the last
+    d[:, 11] = fr.float()
+    keep = torch.nonzero((d[:, 0] > 1) & (fr >= 1) & (fr <= nf)).flatten()
+    ref = d[keep[torch.sort(fr[keep], stable=True).indices]]
+    out = torch.full_like(d, -7.0)
+    ctx = Q.Context(Q.default_params(ImageWidth=64, ImageHigh=64))
+    m = ctx.compact_sorted_dev(d, n, 1, nf, out)
+    assert m == len(keep)
+    assert torch.equal(out[:m], ref)
+    assert bool((out[m:] == -7.0).all())
