@@ -15,6 +15,7 @@ def pytest_configure(config):
 
 def _gpu_available():
     try:
+        import torch  # noqa: F401  before the library: torch finds no device once another HIP runtime is loaded
         import qcstorm
         return qcstorm.lib().qcs_device_count() > 0
     except Exception:
