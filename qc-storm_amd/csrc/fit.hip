@@ -153,9 +153,33 @@ __global__ void __launch_bounds__(64) crlb_kernel(float *__restrict__ loc, int n
 //         hold the other sizes back: 2991 against 4082 with 2 lanes at 320,000)
 //   13, 15  16 at every size (13: 1150 against 1364 and 1799 with 8 and 4 at 80,000)
 //   17x17 16 to 20,000 (1082 / 1346, 1842 / 1840 at 40,000), then 8
-static int lanes_1e(int model, int R, int n)
+//
+// With the hardware exp and log (fast) an evaluation is half as long, the lines lie lower, and while a launch
+// is less than one wave per SIMD (65,536 lanes) the group can be as wide as that allows (wide / narrow):
+//   5x5   8 to 8,192 (65 / 73 at 5,000), 4 to 16,384 (76 / 89 at 10,000), 2 to 32,768 (103 / 126 at 30,000),
+//         then 1 (147 against 171 at 60,000, 398 against 488 at 240,000)
+//   7x7   8 to 8,192 (72 / 81 at 5,000), 4 to 36,000 (145 / 184 at 30,000, 193 / 191 at 40,000), then 1
+//         (205 against 251 at 60,000, 759 against 1002 at 320,000) but for the start of its second round
+//         (80,000: 311 / 344)
+//   9x9   16 to 6,000 (102 / 114 at 5,000, 140 / 115 at 10,000), 4 to 16,384 (115 / 161 at 10,000,
+//         202 / 168 at 20,000), 2 to 36,000 (181 / 277 at 30,000, 306 / 284 at 40,000) and from 65,536 to
+//         100,000 (452 / 498 at 80,000), else 1 (1114 against 1345 at 320,000); elliptical 2 to 200,000
+//         (960 / 1072 at 160,000, 1446 / 1372 at 240,000)
+//   13x13 16 to 26,000 (285 / 314 at 20,000, 424 / 333 at 30,000), then 2 (559 against 624 and 755 with 4 and
+//         16 at 60,000, 1233 against 1383 and 1709 at 160,000); elliptical 4 (486 against 605 with 2 at
+//         30,000, 1956 against 2006 at 160,000)
+static int lanes_1e(int model, int R, int n, bool fast)
 {
     const bool el = model == MODEL_AS3D;
+    if (fast) {
+        switch (R) {
+        case 5: return n <= 8192 ? 8 : n <= 16384 ? 4 : n <= 32768 ? 2 : 1;
+        case 7: return n <= 8192 ? 8 : n <= 36000 || (n > 65536 && n <= 100000) ? 4 : 1;
+        case 9: return n <= 6000 ? 16 : n <= 16384 ? 4 : (el ? n <= 200000 : n <= 36000 || (n > 65536 && n <= 100000)) ? 2 : 1;
+        case 13: return n <= 26000 ? 16 : el ? 4 : 2;
+        default: break;
+        }
+    }
     switch (R) {
     case 5: return n <= 24000 ? 8 : n <= 64000 ? 4 : n <= 240000 ? 2 : 1;
     case 7: return n <= 24000 ? 8 : n <= (el ? 200000 : 400000) ? 4 : 1;
@@ -184,7 +208,8 @@ int fit_launch_1e(const qcs_params &p, const uint16_t *d_rois, const float *d_wl
     if (n <= 0) return QCS_OK;
     const int R = p.ROISize, model = (p.LocType == QCS_LOCTYPE_AS3D) ? MODEL_AS3D : MODEL_GS2D;
     const SplitArgs a{d_rois, d_wle, d_idx, n, d_n, d_loc, nullptr, d_flag, nullptr};
-    return fit_split_1e(model, R, lanes_1e(model, R, n), p.FitMath == QCS_MATH_FAST, a, make_fit_const(p), s);
+    const bool fast = p.FitMath == QCS_MATH_FAST;
+    return fit_split_1e(model, R, lanes_1e(model, R, n, fast), fast, a, make_fit_const(p), s);
 }
 
 // multi-emitter stage over list[j], j < *n_dev (grid sized for n_max)

@@ -364,14 +364,16 @@ __device__ __forceinline__ void split_fit(const float (&q)[SplitShape<MODEL, R, 
     }
 }
 
-// work-group: its four waves share the log table (32 KB for the one-emitter models).  G = 1 is held to
-// two waves per SIMD: the 7x7 2D kernel then takes 225 VGPRs without spills.
+// work-group: its four waves share the log table (32 KB for the one-emitter models).  G = 1, and the
+// fast 13x13 pair of lanes (91 pixels a lane), are held to two waves per SIMD: the 7x7 2D kernel then
+// takes 225 VGPRs without spills, and the 13x13 one spills 58 but runs 60,000 fits in one round (638 -> 559 us).
 constexpr int FS_BLOCK = 256;
+template <int R, int G> constexpr bool kTwoWaves = G == 1 || ((R + G - 1) / G) * R > 80;
 
 // Items i < n (or *n_dev) of list idx (or the ROIs themselves).  One-emitter models write the ROI's
 // row and flag a[roi]; multi-emitter models write as finish_me does (second rows, a = fs, b = ff).
 template <int MODEL, int R, int G, bool FAST>
-__global__ void __launch_bounds__(FS_BLOCK) __attribute__((amdgpu_waves_per_eu(G == 1 ? 2 : 1, G == 1 ? 2 : 10))) fit_split_kernel(const uint16_t *__restrict__ rois, const float *__restrict__ wle,
+__global__ void __launch_bounds__(FS_BLOCK) __attribute__((amdgpu_waves_per_eu(kTwoWaves<R, G> ? 2 : 1, kTwoWaves<R, G> ? 2 : 10))) fit_split_kernel(const uint16_t *__restrict__ rois, const float *__restrict__ wle,
                                                              const int *__restrict__ idx, int n, const int *__restrict__ n_dev,
                                                              float *__restrict__ loc, float *__restrict__ second, int *__restrict__ fa,
                                                              int *__restrict__ fb, FitConst fc)

@@ -22,6 +22,14 @@ static int by_size(int R, int G, const SplitArgs &a, const FitConst &fc, hipStre
     if (R == 15 && G == 16) return launch_split<MODEL, 15, 16, FAST>(a, fc, s);
     if (R == 17 && G == 8) return launch_split<MODEL, 17, 8, FAST>(a, fc, s);
     if (R == 17 && G == 16) return launch_split<MODEL, 17, 16, FAST>(a, fc, s);
+    if constexpr (FAST) {
+        if (R == 9 && G == 1) return launch_split<MODEL, 9, 1, FAST>(a, fc, s);
+        if constexpr (MODEL == MODEL_GS2D) {
+            if (R == 13 && G == 2) return launch_split<MODEL, 13, 2, FAST>(a, fc, s);
+        } else {
+            if (R == 13 && G == 4) return launch_split<MODEL, 13, 4, FAST>(a, fc, s);
+        }
+    }
     return fail(QCS_ERR_ARG, "ROISize %d not supported by the fitter (odd, 5..17)", R);
 }
 

@@ -91,3 +91,24 @@ def test_fast_math_groups_agree(gpu, loc):
         if ref is None:
             ref = got.view(torch.int32).clone()
         assert torch.equal(got.view(torch.int32), ref[idx])
+
+
+# both sides of the lines that calls with the hardware exp and log have of their own
+FAST = [(0, 5, (8192, 8193, 16385, 32769)), (1, 5, (32769,)), (0, 7, (8193, 36001, 65537, 100001)), (1, 7, (36001, 65537)),
+        (0, 9, (6000, 6001, 16385, 36001, 65537, 100001)), (1, 9, (6001, 16385, 200001)), (0, 13, (26000, 26001, 70003)),
+        (1, 13, (26000, 26001))]
+
+
+@pytest.mark.parametrize("loc,R,lines", FAST)
+def test_fast_math_lines_agree(gpu, loc, R, lines):
+    import torch
+    m = 151
+    rois, wle = _sample(R, loc, m, 1)
+    params = Q.default_params(QE=1.0, ROISize=R, LocType=loc, FitMath=Q.MATH_FAST, p1_XGY=-111.11, p1_XLY=-111.11)
+    ref, _, _ = _tiled(params, rois, wle, m, m)
+    ref = ref.view(torch.int32)
+    assert (ref[:, 0] != 0).sum().item() > m // 8   # the 5x5 window refuses most elliptical shapes (40 stay)
+    for n in lines:
+        got, rows, idx = _tiled(params, rois, wle, n, n)
+        assert rows == n
+        assert torch.equal(got.view(torch.int32), ref[idx]), n
