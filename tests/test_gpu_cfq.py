@@ -1,4 +1,5 @@
-"""The persistent work-queue fitter (cfq.hip) against the one-pass fitter (cfit_kernel).
+"""The persistent work-queue fitter (cfq.hip, cfs.hip) against the one-pass fitter (cfit_kernel).  The sizes here
+are below the one-lane queue's line; test_gpu_cfs.py has the ones above it.
 
 Both run the same arithmetic per BFGS step, so parameters, iteration counts, flags and FP64
 log-likelihoods must be bit-identical whatever order the queue hands the ROIs out in; the
@@ -43,7 +44,7 @@ def test_queue_matches_one_pass_bitwise(gpu, R, n):
     ctx = Q.Context(Q.default_params(QE=1.0, ROISize=R))
     ctx.set_tuning(queue=0)
     ref = _chain(ctx, d_rois, n)
-    for wpc in (0, 1):   # all resident waves / one wave per CU (many refills per lane)
+    for wpc in (0, 1):   # all resident waves / one wave per CU; calls this small are the split kernel's (cfs.hip)
         ctx.set_tuning(queue=1, waves_per_cu=wpc)
         got = _chain(ctx, d_rois, n)
         for K, ((t0, i0, l0), (t1, i1, l1)) in enumerate(zip(ref, got), start=1):

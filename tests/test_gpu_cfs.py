@@ -71,3 +71,57 @@ def test_split_fits_pin_stop_and_flat_stop(gpu):
     assert (out[0][1][:, 1] & Q.CFIT_PINNED).any()
     for t, i in out[1:]:
         assert torch.equal(t, out[0][0]) and torch.equal(i, out[0][1])
+
+
+# One wave per CU has 16,384 lanes on 256 CUs: a lane of the one-lane kernel runs three fits and more, in chunks from
+# the queue, before the wave leaves its last ones; a group of the split kernel (elliptical K = 3) takes nine.
+@pytest.mark.parametrize("loc,R,n", [(0, 7, 50001), (0, 7, 49000), (0, 9, 50001), (0, 11, 50001), (1, 7, 40001), (1, 9, 50001), (1, 11, 40001)])
+def test_refilled_lanes_match_bitwise(gpu, loc, R, n):
+    import torch
+    m = 499
+    sp = Q.default_sim(width=R, height=R, astig=loc, n_per_unit_max=3, min_sep=1.0, max_sep=4.0, photons_min=300.0, photons_max=6000.0)
+    rois, _ = Q.sim_rois_host(sp, 5400 + 10 * R + loc, m)
+    d = torch.from_numpy(rois.view(np.int16)).cuda()
+    p = Q.default_params(QE=1.0, ROISize=R, LocType=loc, p1_XGY=-111.11, p1_XLY=-111.11)
+    ctx, one = Q.Context(p), Q.Context(p)
+    ctx.set_tuning(waves_per_cu=1)
+    one.set_tuning(queue=0)
+    idx = torch.arange(n, device="cuda") % m
+    r = d[idx].contiguous()
+    prev = None
+    for K in (1, 2, 3):
+        mode = Q.CFIT_INIT_HEUR if K == 1 else Q.CFIT_INIT_ADD
+        th, info, ll = _fit(one, K, d, m, mode, prev)
+        t, i, l = _fit(ctx, K, r, n, mode, prev[idx].contiguous() if prev is not None else None)
+        assert torch.equal(t.view(torch.int32), th.view(torch.int32)[idx]), K
+        assert torch.equal(i[:, :2], info[idx, :2]), K
+        assert torch.equal(l.view(torch.int64), ll.view(torch.int64)[idx]), K
+        assert bool((i[:, 2] <= info[idx, 2]).all()), K
+        prev = th
+
+
+@pytest.mark.parametrize("wpc", [0, 1])
+def test_mixed_sizes_past_the_line_match_one_pass(gpu, wpc):
+    """Three sizes in one launch of the one-lane kernel, each with its own queue and left fits."""
+    import torch
+    m = 300
+    ctx = Q.Context(Q.default_params(QE=1.0, ROISize=7, PixelSize=100.0))
+    ctx.set_tuning(waves_per_cu=wpc)
+    sets, refs = [], []
+    for R, n in ((7, 30001), (9, 20003), (11, 9007)):
+        sp = Q.default_sim(width=R, height=R, n_per_unit_max=3, min_sep=1.0, max_sep=4.0, photons_min=500.0, photons_max=5000.0)
+        d = torch.from_numpy(Q.sim_rois_host(sp, 5500 + R, m)[0].view(np.int16)).cuda()
+        one = Q.Context(Q.default_params(QE=1.0, ROISize=R, PixelSize=100.0))
+        one.set_tuning(queue=0)
+        rl = torch.zeros((3 * m, 12), dtype=torch.float32, device="cuda")
+        rs = torch.zeros(m, dtype=torch.int32, device="cuda")
+        one.fit_mle_dev(d, m, 3, rl, rs)
+        idx = torch.arange(n, device="cuda") % m
+        sets.append((R, d[idx].contiguous(), n, torch.full((3 * n, 12), -7.0, device="cuda"), torch.full((n,), -7, dtype=torch.int32, device="cuda")))
+        refs.append((rl.reshape(m, 36), rs, idx))
+    ctx.fit_mle_mixed_dev(sets, 3)
+    torch.cuda.synchronize()
+    for (R, _, n, loc, sel), (rl, rs, idx) in zip(sets, refs):
+        assert torch.equal(sel, rs[idx]), R
+        assert torch.equal(loc.reshape(n, 36).view(torch.int32), rl[idx].view(torch.int32)), R
+        assert (rs == 3).any() and (rs == 1).any()
