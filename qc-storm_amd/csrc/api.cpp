@@ -238,8 +238,8 @@ int qcs_ctx_set_params(qcs_ctx *c, const qcs_params *p)
 int qcs_ctx_destroy(qcs_ctx *c)
 {
     if (!c) return QCS_OK;
-    qcs::DevBuf *bufs[] = {&c->ex_bkg, &c->ex_tmp, &c->ex_det, &c->ex_mark, &c->ex_cnt, &c->ex_xy,
-                           &c->ex_frames, &c->fit_idx1, &c->fit_idx2, &c->fit_idx3, &c->fit_flag, &c->fit_cnt,
+    qcs::DevBuf *bufs[] = {&c->ex_tmp, &c->ex_det, &c->ex_mark, &c->ex_cnt, &c->ex_xy,
+                           &c->ex_frames, &c->fit_flag, &c->fit_cnt,
                            &c->fit_rows, &c->h_rois_dev, &c->h_wle_dev, &c->h_loc_dev, &c->cf_theta, &c->cf_ll,
                            &c->cf_list, &c->cf_rows, &c->cf_queue, &c->rn_buf, &c->st_buf,
                            &c->dr_img, &c->dr_cc, &c->dr_shift, &c->dr_frames, &c->dp_hist,

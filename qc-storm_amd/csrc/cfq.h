@@ -4,15 +4,16 @@
 
 namespace qcs {
 
+enum { CX_ROI = 0, CX_ST = 1, CX_T = 2, CX_ITERS = 3, CX_EVALS = 4, CX_SLOPE = 5, CX_ALPHA = 6, CX_DMAX = 7, CX_DU = 8 };
+
 // record of one work item: theta, loss, gradient, "identity start" flag, packed D0, padding; a
 // fit left by a one-lane wave adds the state of its line search and its counters at OX
 template <int KK> struct CQ {
     static constexpr int P = CP<KK>::P, NS = CP<KK>::NS;
     static constexpr int OL = P, OG = P + 1, OF = 2 * P + 1, OD = 2 * P + 2;
     static constexpr int W = (2 * P + 2 + NS + 3) & ~3;   // floats, a multiple of 4
-    static constexpr int OX = W, XW = (W + 9 + P + 3) & ~3;
+    static constexpr int OX = W, XW = (W + CX_DU + P + 3) & ~3;
 };
-enum { CX_ROI = 0, CX_ST = 1, CX_T = 2, CX_ITERS = 3, CX_EVALS = 4, CX_PIN = 5, CX_SLOPE = 6, CX_ALPHA = 7, CX_DMAX = 8, CX_DU = 9 };
 
 enum { CQ_IDLE = 0, CQ_DIR = 1, CQ_LS = 2 };
 

@@ -24,6 +24,7 @@
 // of the one-pass kernel, so both give bit-identical parameters, iteration counts and flags (the
 // evaluation counts differ by the saved gradient evaluations).
 #include <string.h>
+#include <algorithm>
 #include <type_traits>
 #include "cfq.h"
 
@@ -121,7 +122,7 @@ __device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CqLeft
         else return QLds{qs};
     }();
     const int n = S.n_dev ? min(*S.n_dev, S.n) : S.n;   // a device count never exceeds the capacity
-    int st = CQ_IDLE, roi = 0, iters = 0, flags = 0, evals = 0, t = 0, pin_run = 0;
+    int st = CQ_IDLE, roi = 0, iters = 0, flags = 0, evals = 0, t = 0;
     bool first = false, dry = n <= 0;
     float th[P], g[P], du[P], L = 0.0f, slope = 0.0f, alpha = 1.0f, dmax = 0.0f;
 #pragma unroll
@@ -197,7 +198,6 @@ __device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CqLeft
         iters = 0;
         flags = 0;
         evals = 1;
-        pin_run = 0;
         st = CQ_DIR;
     };
     // quasi-Newton direction from a fresh gradient; converged fits end here
@@ -246,7 +246,6 @@ __device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CqLeft
                     h[CX_T] = t;
                     h[CX_ITERS] = iters;
                     h[CX_EVALS] = evals;
-                    h[CX_PIN] = pin_run;
                 }
                 break;
             }
@@ -269,13 +268,8 @@ __device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CqLeft
             }
             const float Lold = L;
             L = Lt;
-            if constexpr (CM<KK>::AS && CM<KK>::K == 3)
-                if (c.pin_stop) pin_run = cf_at_bound<KK, R>(th) ? pin_run + 1 : 0;
             if (Lold - L < c.ftol) {   // the likelihood has stopped moving
                 flags |= CF_CONVERGED | CF_FLAT;
-                finish();
-            } else if (pin_run >= CF_PIN_RUN) {
-                flags |= CF_PINNED;
                 finish();
             } else if (iters >= c.max_iter) {
                 flags |= CF_MAXITER;
@@ -301,6 +295,8 @@ __device__ __forceinline__ void cfq_run(const CfqSet &S, int *head, const CqLeft
     }
 }
 
+// The elliptical three-emitter model (KK = 13) has no one-lane kernel: the split one takes all of its
+// launches (cq_route), and its opt-in stop at a bound (pin_stop) is there.
 template <int KK, int RMAX>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(CqLayout<KK, RMAX>::WAVES))) cfq_kernel(CfqArgs a)
 {
@@ -351,6 +347,17 @@ static void cq_rec_w(int KK, int &w, int &xw)
     }
 }
 
+// models with a one-lane kernel
+#define CQ_DISPATCH_KK(KK_, ...)                                                          \
+    switch (KK_) {                                                                         \
+    case 1: { constexpr int KT = 1; __VA_ARGS__; } break;                                  \
+    case 2: { constexpr int KT = 2; __VA_ARGS__; } break;                                  \
+    case 3: { constexpr int KT = 3; __VA_ARGS__; } break;                                  \
+    case 11: { constexpr int KT = 11; __VA_ARGS__; } break;                                \
+    case 12: { constexpr int KT = 12; __VA_ARGS__; } break;                                \
+    default: return fail(QCS_ERR_ARG, "model %d has no one-lane fitter", KK_);              \
+    }
+
 // resident work-groups per CU of kernel f
 static int cq_occupancy(const void *f)
 {
@@ -368,7 +375,7 @@ static int cq_waves_per_cu(int KK, int RMAX)
     int &v = cache[as][K - 1][ri];
     if (v == 0) {
         const void *f = nullptr;
-        CF_DISPATCH_KK(KK, CF_DISPATCH_R(RMAX, f = reinterpret_cast<const void *>(&cfq_kernel<KT, RT>)))
+        CQ_DISPATCH_KK(KK, CF_DISPATCH_R(RMAX, f = reinterpret_cast<const void *>(&cfq_kernel<KT, RT>)))
         v = cq_occupancy(f);
     }
     return v;
@@ -422,12 +429,14 @@ int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_
     if (items == 0) return QCS_OK;
     int cus = 0;
     QCS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-    int wpc = cq_waves_per_cu(KK, rmax);
-    if (ctx->tune.waves_per_cu > 0 && ctx->tune.waves_per_cu < wpc) wpc = ctx->tune.waves_per_cu;
-    long long waves = (items + 63) / 64;
-    if (waves > (long long)cus * wpc) waves = (long long)cus * wpc;
     int most;
     const bool split = cq_route(KK, items, most);
+    long long waves = 0;   // of the one-lane launch
+    if (!split) {
+        int wpc = cq_waves_per_cu(KK, rmax);
+        if (ctx->tune.waves_per_cu > 0 && ctx->tune.waves_per_cu < wpc) wpc = ctx->tune.waves_per_cu;
+        waves = std::min((items + 63) / 64, (long long)cus * wpc);
+    }
     const size_t lcap = split ? 0 : (size_t)waves * most;   // fits the waves may leave, per set
     int rc;
     if ((rc = ctx->cf_queue.ensure(256 + (total + lcap * XW * nsets) * sizeof(float)))) return rc;
@@ -461,7 +470,7 @@ int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_
         if ((rc = cfs_launch(a, KK, rmax, items, cus, ctx->tune.waves_per_cu, s))) return rc;
     } else {
         const dim3 pgrid((unsigned)waves), block(64);
-        CF_DISPATCH_KK(KK, CF_DISPATCH_R(rmax, hipLaunchKernelGGL((cfq_kernel<KT, RT>), pgrid, block, 0, s, a)))
+        CQ_DISPATCH_KK(KK, CF_DISPATCH_R(rmax, hipLaunchKernelGGL((cfq_kernel<KT, RT>), pgrid, block, 0, s, a)))
         QCS_HIP(hipGetLastError());
         a.heads = heads + 4;
         if ((rc = cfs_launch(a, KK, rmax, (long long)lcap, cus, ctx->tune.waves_per_cu, s))) return rc;

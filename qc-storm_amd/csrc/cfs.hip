@@ -136,7 +136,7 @@ __device__ __forceinline__ void cfs_run(const CfqSet &S, int *head, const CqLeft
                     t = h[CX_T];
                     iters = h[CX_ITERS];
                     evals = h[CX_EVALS];
-                    pin_run = h[CX_PIN];
+                    pin_run = 0;   // only the models without it have left fits
                     slope = rec[Q::OX + CX_SLOPE];
                     alpha = rec[Q::OX + CX_ALPHA];
                     dmax = rec[Q::OX + CX_DMAX];

@@ -127,9 +127,9 @@ struct qcs_ctx {
     qcs::Timer timer;
     qcs_fit_stats stats{};
     // extraction scratch
-    qcs::DevBuf ex_bkg, ex_tmp, ex_det, ex_mark, ex_cnt, ex_xy, ex_frames;
+    qcs::DevBuf ex_tmp, ex_det, ex_mark, ex_cnt, ex_xy, ex_frames;
     // fit scratch
-    qcs::DevBuf fit_idx1, fit_idx2, fit_idx3, fit_flag, fit_cnt, fit_rows;   // fit_flag: the cascade's carve
+    qcs::DevBuf fit_flag, fit_cnt, fit_rows;   // fit_flag: the cascade's carve
     // converged fitting scratch
     qcs::DevBuf cf_theta, cf_ll, cf_list, cf_rows, cf_queue;
     // mixed-size extraction (7 x 7 cuts, WLE, size flags, set lists) and the frames path's sets
