@@ -96,10 +96,10 @@ struct DSplit {   // D[i] in registers for i < NREG, else at p[(i - NREG) * 64]
     __device__ __forceinline__ float &operator[](int i) { return (NREG > 0 && i < NREG) ? r[i] : p[(i - NREG) * 64]; }
 };
 
-// ln x for normal x: v_log_f32 times ln 2 in two parts, the arithmetic of __logf without its scaling of
-// subnormal and selection of infinite arguments (five instructions instead of twelve, a sixth of a
-// pixel's).  The losses take it of mu / q with mu >= 1e-6 and q below 2^17 / QE, which is normal; an
-// infinite mu makes the loss NaN either way.
+// ln x for normal x: v_log_f32 times ln 2 as a sum of two floats, the arithmetic (and the bits) of HIP's
+// __logf without its scaling of subnormal and selection of infinite arguments (five instructions instead of
+// twelve, a sixth of a pixel's).  The losses take it of mu / q with mu >= 1e-6 and q below 2^17 / QE, which
+// is normal; an infinite mu makes the loss NaN either way.
 __device__ __forceinline__ float cf_logf(float x)
 {
     const float r = __builtin_amdgcn_logf(x);

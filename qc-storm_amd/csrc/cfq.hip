@@ -391,6 +391,9 @@ static int cq_waves_per_cu(int KK, int RMAX)
 //           K = 2  8,192: 1238 / 1708 / 10466  16,461: 3180 / 2071 / 10046  262,144: 10734 / 7626 / 17499
 //           K = 3  16,461: 4401 / 5510 / 22605  262,144: 23268 / 32635 / 51638 (a quarter of its fits run to
 //                  the iteration cap, at 160 evaluations a fit): split at every size
+// `items` is the sets' capacity.  Where the counts are on the device (the three-emitter stage of every path,
+// all of the frames path) fewer fits run than that, so a launch may take the one-lane kernel below its
+// line; the lines hold for launches whose count is their work.
 // Leaving early pays while the one-lane waves are few (16 of 64 lanes in 2D, 32 elliptical); beyond
 // 49,152 fits, 8 (2D K = 1, 64,000: 250 against 291 at 16 and 345 at 4), elliptical K = 2 still 32.
 static bool cq_route(int KK, long long items, int &most)

@@ -24,10 +24,10 @@
 // start that way.
 //
 // What bounds it: a lone fit, the latency of a round (2.5 us elliptical K = 3: 81 chained FMAs over LDS, the
-// 16-parameter products); many, VALU issue, about 1,400 instructions per round of four fits, of which
-// the pixel terms use 9 of 16 lanes at 9x9.  Measured against one fit per lane, three launches and
-// selection: elliptical 9x9, 500 ROIs 21.1 -> 1.6 ms, 16,461 ROIs 34 -> 7.0 ms; 2D 7x7, 2,000 ROIs
-// 2.6 -> 0.56 ms.
+// 16-parameter products); many, VALU issue (0.76 of the cycles on 2^18 elliptical ROIs at K = 3), 312
+// instructions per loss evaluation or 1,250 per round of four fits, of which the pixel terms use 9 of 16 lanes
+// at 9x9.  Measured against one fit per lane to the end, three launches and selection: elliptical 9x9,
+// 500 ROIs 21.1 -> 1.6 ms, 16,461 ROIs 35.3 -> 6.1 ms; 2D 7x7, 2,000 ROIs 2.6 -> 0.56 ms.
 #include <string.h>
 #include "cfq.h"
 

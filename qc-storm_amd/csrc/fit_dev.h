@@ -1,6 +1,6 @@
 // fit_dev.h -- models of the reference-schedule fitters: parameter layouts, start vectors, weights,
-// acceptance rules and rows, shared by the one-ROI-per-lane kernel (fit.hip) and the kernels that
-// split an ROI over a group of lanes (fit_split.hip).
+// acceptance rules and rows, used by the kernels of fit_split.h (instantiated in fit_split_1e.hip and
+// fit_split_me.hip) and their host side (fit.hip).
 //
 // Reference kernels (DLL = MLEbfgs/bfgs_MLE_dll x64/bfgsMLE_dll/bfgsMLE_dll):
 //   bfgsMLELoc_Gauss2D      DLL/bfgsMLE_Loc_LD/bfgsMLE_GS2D_core.h:56-310
@@ -14,8 +14,9 @@
 
 namespace qcs {
 
-// Arguments of the split-ROI fits (fit_split.h): items i < n (or *n_dev) of list idx (or the ROIs
-// themselves); fa / fb as the one-lane kernels' flags.
+// Arguments of the fits (fit_split.h): items i < n (or *n_dev) of list idx (or the ROIs themselves).  fa, by
+// ROI: one-emitter fits that go to the two-emitter stage (finish_1e); fa and fb, by item: accepted second
+// and rejected first emitters of the multi-emitter stages (finish_me), whose second rows go to second.
 struct SplitArgs {
     const uint16_t *rois;
     const float *wle;

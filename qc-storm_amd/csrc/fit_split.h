@@ -28,12 +28,12 @@
 // _any form of the log, whose range and special-value handling gives the value the CPU oracle
 // computes.
 //
-// What bounds it: many ROIs, VALU issue (7x7 2D at G = 1: about 143,000 VALU instructions per wave,
-// 10.7 per pixel evaluation); few, the latency of the chain.  Measured, us per call with CRLB,
-// against one ROI per lane with a uniform loop over the evaluations:
-//   7x7 2D     20,480 ROIs 458 -> 180 (G = 8), 1,000,003 ROIs 4050 -> 3610 (G = 1)
-//   9x9 3D     5,377 ROIs 1448 -> 230 (G = 16);  11x11 2D 100,001 ROIs 2870 -> 1080 (G = 4)
-//   cascade    20,480 ROIs of dense frames, 7x7: 4800 -> 1060 (G = 8)
+// What bounds it: many ROIs, VALU issue (7x7 2D at G = 1: 163,800 VALU instructions per fit, 19 per pixel
+// of an evaluation with everything; 210,200 at G = 4); few, the latency of the chain.  Measured, us per call
+// with CRLB, against one ROI per lane with a uniform loop over the evaluations:
+//   7x7 2D     20,480 ROIs 498 -> 173 (G = 8), 1,000,003 ROIs 4030 -> 3670 (G = 1)
+//   9x9 3D     5,377 ROIs 1445 -> 191 (G = 16);  11x11 2D 100,001 ROIs 3090 -> 1090 (G = 4)
+//   cascade    20,480 ROIs of dense frames, 7x7: 4850 -> 950 (G = 8)
 #pragma once
 #include <type_traits>
 #include "fit_dev.h"

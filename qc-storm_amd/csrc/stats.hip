@@ -19,7 +19,8 @@
 // it costs: the frame range stays on the device and everything is read back once, eight launches
 // and one wait.  Sorting the molecules by (frame, cell) and searching the sorted keys took 19
 // launches and five waits, and each search is a chain of fifteen dependent loads (20,480 rows:
-// neighbours 28.8 -> 10 us, row pass 28.6 -> 6 us; with compaction and rendering 417 -> 215 us).
+// neighbours 28.8 -> 10 us, row pass 28.6 -> 6 us; with compaction and rendering 417 -> 215 us; 2,200,000 rows
+// in 200 frames 1,890 -> 660 us, 8,000,000 in 100,000 frames 4,390 -> 2,670 us).
 #include <limits.h>
 #include <stddef.h>
 #include <algorithm>
@@ -145,6 +146,9 @@ __global__ void __launch_bounds__(RT) stat_rows_kernel(const float *__restrict__
 // distance test passes are then at most one cell apart in x and in y even after the rounding of the
 // quotients.  A molecule's bucket is a hash of its frame and cell; the cells around one molecule may
 // share a bucket, so an entry carries its frame and cell and counts for its own cell only.
+// The hash: the cell times Knuth's multiplicative constant (2^32 / golden ratio), plus the frame times
+// xxHash32's second prime, then a shift and the multiplier 0x2c1b3c6d of the 32-bit mixers in common use; its
+// upper bits are the bucket.
 struct Grid {
     int W, H, ncx, lb;   // 2^lb buckets
     float cell, r2;
