@@ -108,3 +108,19 @@ def test_rows_of_large_calls(gpu, n, nf):
     assert m == len(keep)
     assert torch.equal(out[:m], ref)
     assert bool((out[m:] == -7.0).all())
+
+
+# cells of fewer and of more molecules than a lane walks by itself (24), and both in one call
+@pytest.mark.parametrize("lt", [0, 1])
+@pytest.mark.parametrize("n,dense", [(400, False), (800, False), (900, True), (5000, False), (20000, True)])
+def test_stats_dense_cells(gpu, n, dense, lt):
+    W = 96
+    p = Q.default_params(ImageWidth=W, ImageHigh=W, LocType=lt)
+    rng = np.random.default_rng(n + lt)
+    loc = _stat_rows(n, n + lt, 2, W, W, False)
+    if dense:   # half of them within one cell's width
+        loc[: n // 2, 1:3] = rng.uniform(41.0, 49.0, (n // 2, 2))
+        loc[:, 1:] = loc[rng.permutation(n), 1:]
+        loc = loc[np.argsort(loc[:, 11], kind="stable")]
+    got = _check(p, loc)
+    assert got["density_total"] > n // 2
