@@ -25,6 +25,7 @@ __device__ __forceinline__ void cf_wave_fence()
 }
 
 // split launch over the sets of a (cfs.hip): fresh items, or where a.left[i].rec is set the left fits
+int cfs_waves_per_cu(int KK, int RMAX);   // its resident waves per CU
 int cfs_launch(const CfqArgs &a, int KK, int rmax, long long items, int cus, int max_waves_per_cu, hipStream_t s);
 
 }  // namespace qcs

@@ -393,15 +393,19 @@ static int cq_waves_per_cu(int KK, int RMAX)
 //                  the iteration cap, at 160 evaluations a fit): split at every size
 // `items` is the sets' capacity.  Where the counts are on the device (the three-emitter stage of every path,
 // all of the frames path) fewer fits run than that, so a launch may take the one-lane kernel below its
-// line; the lines hold for launches whose count is their work.
+// line; the lines hold for launches whose count is their work.  A limit on the waves per CU below half of
+// what the split kernel keeps lowers the lines in proportion: it takes resident fits from that kernel, while
+// one lane per fit has many to spare (2D 7x7, 20,000 ROIs through K = 1..3 at one wave per CU 3007 -> 2046 us
+// with 2656 one-lane alone, at two 1945 -> 1593).
 // Leaving early pays while the one-lane waves are few (16 of 64 lanes in 2D, 32 elliptical); beyond
 // 49,152 fits, 8 (2D K = 1, 64,000: 250 against 291 at 16 and 345 at 4), elliptical K = 2 still 32.
-static bool cq_route(int KK, long long items, int &most)
+static bool cq_route(int KK, int rmax, long long items, int max_waves_per_cu, int &most)
 {
     const bool el = KK > CF_ELLIPTIC;
     const int K = el ? KK - CF_ELLIPTIC : KK;
     static const int line[3] = {12000, 28000, 40000};
     most = el ? (items <= 49152 || K == 2 ? 32 : 8) : (items <= 49152 ? 16 : 8);
+    if (max_waves_per_cu > 0) items = items * std::max(cfs_waves_per_cu(KK, rmax), 2 * max_waves_per_cu) / (2 * max_waves_per_cu);
     return el ? (K == 3 || items <= 12000) : items <= line[K - 1];
 }
 
@@ -433,7 +437,7 @@ int cfq_launch(qcs_ctx *ctx, int K, const CfqSet *sets_in, int nsets, hipStream_
     int cus = 0;
     QCS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
     int most;
-    const bool split = cq_route(KK, items, most);
+    const bool split = cq_route(KK, rmax, items, ctx->tune.waves_per_cu, most);
     long long waves = 0;   // of the one-lane launch
     if (!split) {
         int wpc = cq_waves_per_cu(KK, rmax);

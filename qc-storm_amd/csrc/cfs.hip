@@ -543,7 +543,7 @@ __global__ void __launch_bounds__(CS_BLOCK) cfs_kernel(CfqArgs a, int ways)
 }
 
 // resident single-wave work-groups per CU (cached)
-static int cs_waves_per_cu(int KK, int RMAX)
+int cfs_waves_per_cu(int KK, int RMAX)
 {
     static int cache[2][3][3] = {{{0}}};
     const int ri = RMAX == 7 ? 0 : (RMAX == 9 ? 1 : 2);
@@ -569,7 +569,7 @@ static int cs_waves_per_cu(int KK, int RMAX)
 
 int cfs_launch(const CfqArgs &a, int KK, int rmax, long long items, int cus, int max_waves_per_cu, hipStream_t s)
 {
-    int wpc = cs_waves_per_cu(KK, rmax);
+    int wpc = cfs_waves_per_cu(KK, rmax);
     if (max_waves_per_cu > 0 && max_waves_per_cu < wpc) wpc = max_waves_per_cu;
     const long long most = (long long)cus * wpc;
     // one fit per wave, its four groups sharing it, while every fit gets a wave at once

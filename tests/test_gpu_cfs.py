@@ -75,7 +75,7 @@ def test_split_fits_pin_stop_and_flat_stop(gpu):
 
 # One wave per CU has 16,384 lanes on 256 CUs: a lane of the one-lane kernel runs three fits and more, in chunks from
 # the queue, before the wave leaves its last ones; a group of the split kernel (elliptical K = 3) takes nine.
-@pytest.mark.parametrize("loc,R,n", [(0, 7, 50001), (0, 7, 49000), (0, 9, 50001), (0, 11, 50001), (1, 7, 40001), (1, 9, 50001), (1, 11, 40001)])
+@pytest.mark.parametrize("loc,R,n", [(0, 7, 50001), (0, 7, 49000), (0, 7, 15001), (0, 9, 50001), (0, 11, 50001), (1, 7, 40001), (1, 9, 50001), (1, 11, 40001)])
 def test_refilled_lanes_match_bitwise(gpu, loc, R, n):
     import torch
     m = 499
